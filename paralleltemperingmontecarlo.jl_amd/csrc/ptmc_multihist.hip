@@ -1,298 +1,424 @@
-// Multihistogram heat capacity (multihistogram_NVT, src/multihist_NVT.jl:11-221)
-// in FP64 on the device, one workgroup per PT run.
+// Multihistogram heat capacities (multihistogram_NVT, src/multihist_NVT.jl:11-221,
+// and multihistogram_NPT, src/multihist_NPT.jl:17-340) in FP64 on the device.
 //
 // The reference iterates free energies f_i = log sum_m q(beta_i, m) with
-//   q(b, m) = H_m / D_m * exp(-b E_m - off_m),
-//   off_m   = max(-1e6, max_i(-beta_i E_m - f_i)) + log(1000),
-//   D_m     = sum_i n_i exp(-beta_i E_m - f_i - off_m),  H_m = sum_i h_i(m).
-// off_m and D_m do not depend on b, so each iteration computes them once per
-// bin (same operations, same order as every call in the reference) and then
-// the R sums over bins.  Heat capacities follow on a 10x denser temperature
-// grid: Cv = (<E^2> - <E>^2) / (k T^2).
+//   q(b, m) = H_m / D_m * exp(-b h_m - off_m),
+//   off_m   = max(-1e6, max_i(-beta_i h_m - f_i)) + log(1000),
+//   D_m     = sum_i n_i exp(-beta_i h_m - f_i - off_m),  H_m = sum_i h_i(m),
+// over the energy bins (h = E), or the (energy, volume) bins with h = E + pV.
+// off_m cancels from q, so it may be taken from any earlier free energies f0:
+// with K_im = exp(-beta_i h_m - f0_i - off_m(f0)) an iteration is
+//   D_m = sum_i n_i K_im exp(-(f_i - f0_i)),  f_i = f0_i + log sum_m H_m K_im / D_m,
+// two products with a matrix that stays, and no exponential per (i, m).  K is
+// rebuilt (f0 = f) once some |f_i - f0_i| passes MH_REBASE, long before a
+// term that matters could leave the range of a double.  Heat capacities
+// follow on the output grid: C = (<h^2> - <h>^2) / (k T^2).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
 #include <vector>
 
 #include "../../include/ptmc.h"
+#include "ptmc_device.hpp"
 
 namespace {
 
 constexpr int MH_THREADS = 256;
+constexpr int MH_BINS = 128;                   // bins of a block, whose sums are formed together
+constexpr size_t MH_SLICE_LDS = 96 * 1024;     // largest slice of a run's bins kept in LDS
+constexpr double MH_REBASE = 16.0;
+constexpr unsigned MH_SPIN = 1u << 26;         // polls of a grid barrier before it gives up (seconds)
 
 struct MHArgs {
-    int n_temps, n_bin, n_res, max_iter;
+    int n_temps, n_bin, n_bins, n_res, max_iter;  // n_bins: n_bin (NVT) or n_bin^2 (NPT) bins of a run
+    int npt, n_wg, n_blk, wg_blk;  // workgroups of a run, its blocks of MH_BINS bins, blocks of a workgroup
     double conv;
     const double *beta;      // runs x R
-    const double *hist;      // runs x R x (n_bin + 2)
-    const double *en_min;    // runs
-    const double *en_max;    // runs
-    const double *beta_res;  // runs x n_res
-    const double *t_res;     // runs x n_res
-    double k_boltzmann;
-    double *cv;              // runs x n_res
-    double *free_energy;     // runs x R
-    int *iterations;         // runs
-};
-
-__global__ void __launch_bounds__(MH_THREADS) multihist_kernel(MHArgs a)
-{
-    extern __shared__ __align__(16) unsigned char lds[];
-    const int R = a.n_temps, nb = a.n_bin, run = blockIdx.x, tid = threadIdx.x;
-    double *fe = reinterpret_cast<double *>(lds);  // R
-    double *nfe = fe + R;                          // R
-    double *ncyc = nfe + R;                        // R
-    double *beta = ncyc + R;                       // R
-    double *off = beta + R;                        // nb
-    double *ratio = off + nb;                      // nb
-    double *hsum = ratio + nb;                     // nb
-    int *flag = reinterpret_cast<int *>(hsum + nb);
-
-    const double *H = a.hist + (size_t)run * R * (nb + 2);
-    const double emin = a.en_min[run];
-    const double de = (a.en_max[run] - emin) / (double)nb;
-    for (int i = tid; i < R; i += MH_THREADS) {
-        double s = 0.0;
-        for (int m = 1; m <= nb; ++m) s = s + H[(size_t)i * (nb + 2) + m];
-        ncyc[i] = s;
-        fe[i] = 0.0;
-        beta[i] = a.beta[(size_t)run * R + i];
-    }
-    __syncthreads();
-    for (int m = tid; m < nb; m += MH_THREADS) {
-        double s = 0.0;
-        for (int i = 0; i < R; ++i) s = s + H[(size_t)i * (nb + 2) + m + 1];
-        hsum[m] = s;
-    }
-    __syncthreads();
-
-    auto bin_terms = [&]() {
-        for (int m = tid; m < nb; m += MH_THREADS) {
-            const double et = emin + ((double)(m + 1) - 0.5) * de;
-            double o = -1.0e6;
-            for (int i = 0; i < R; ++i) o = fmax(o, -beta[i] * et - fe[i]);
-            o = o + log(1000.0);
-            double d = 0.0;
-            for (int i = 0; i < R; ++i) d = d + ncyc[i] * exp(-beta[i] * et - fe[i] - o);
-            off[m] = o;
-            ratio[m] = hsum[m] / d;
-        }
-    };
-
-    int it = 0;
-    for (it = 1; it <= a.max_iter; ++it) {
-        bin_terms();
-        __syncthreads();
-        for (int i = tid; i < R; i += MH_THREADS) {
-            double s = 0.0;
-            for (int m = 0; m < nb; ++m) {
-                const double et = emin + ((double)(m + 1) - 0.5) * de;
-                s = s + ratio[m] * exp(-beta[i] * et - off[m]);
-            }
-            nfe[i] = log(s);
-        }
-        __syncthreads();
-        if (tid == 0) {
-            double delta = 0.0;
-            for (int i = 0; i < R; ++i) {
-                const double d = fabs(nfe[i] - fe[i]);
-                delta = delta + d * d;
-                fe[i] = nfe[i];
-            }
-            *flag = delta < a.conv;
-        }
-        __syncthreads();
-        if (*flag) break;
-    }
-    if (it > a.max_iter) it = a.max_iter;
-    bin_terms();
-    __syncthreads();
-    for (int j = tid; j < a.n_res; j += MH_THREADS) {
-        const double bt = a.beta_res[(size_t)run * a.n_res + j];
-        double nc = 0.0;
-        for (int m = 0; m < nb; ++m) {
-            const double et = emin + ((double)(m + 1) - 0.5) * de;
-            nc = nc + ratio[m] * exp(-bt * et - off[m]);
-        }
-        double e1 = 0.0, e2 = 0.0;
-        for (int m = 0; m < nb; ++m) {
-            const double et = emin + ((double)(m + 1) - 0.5) * de;
-            const double q = ratio[m] * exp(-bt * et - off[m]);
-            e1 = e1 + q / nc * et;
-            e2 = e2 + q / nc * (et * et);
-        }
-        const double t = a.t_res[(size_t)run * a.n_res + j];
-        a.cv[(size_t)run * a.n_res + j] = (e2 - e1 * e1) / (a.k_boltzmann * (t * t));
-    }
-    for (int i = tid; i < R; i += MH_THREADS) a.free_energy[(size_t)run * R + i] = fe[i];
-    if (tid == 0) a.iterations[run] = it;
-}
-
-// ---- multihistogram_NPT (src/multihist_NPT.jl:17-340): the same fixed-point
-// iteration over the (energy, volume) bins of the sampled 2D histograms, with
-// the enthalpy h = E + pV in place of E, and heat capacities from the
-// enthalpy fluctuation, Cp = (<h^2> - <h>^2) / (k T^2).  n_bin^2 bins do not
-// fit LDS: the per-bin terms live in a global scratch block and each thread
-// always owns the same bins, so no barrier separates writing and reading
-// them.  Sums over bins are per-thread partials combined by a fixed-order
-// block reduction.
-constexpr int MHN_THREADS = 256;
-
-struct MHNArgs {
-    int n_temps, n_bin, n_res, max_iter;
-    double conv;
-    const double *beta;      // runs x R
-    const double *hist;      // runs x R x (n_bin + 2)^2, rows energy, columns volume
+    const double *hist;      // runs x R x (n_bin + 2), or x (n_bin + 2)^2: rows energy, columns volume
     const double *en_min, *en_max, *v_min, *v_max, *pressure;  // runs
     const double *beta_res;  // runs x n_res
     const double *t_res;     // runs x n_res
     double k_boltzmann;
-    double *cp;              // runs x n_res
-    double *moments;         // runs x n_res x 3: <E>, <V>, <h>
-    double *free_energy;     // runs x R
-    int *iterations;         // runs
-    double *scratch;         // runs x 3 x n_bin^2: histogram sums, offsets, ratios
+    double *c;               // runs x n_res heat capacities
+    double *moments;         // runs x n_res x 3: <E>, <V>, <h>, or null
+    double *free_energy;     // runs x R, or null
+    int *iterations;         // runs, or null
+    double *ncyc;            // runs x R histogram totals, or null: each workgroup forms its run's
+    double *off, *ratio;     // runs x n_bins: offsets and H_m / D_m of the last free energies
+    double *part;            // runs x 2 x n_blk x R block sums (n_wg > 1)
+    unsigned *count;         // runs arrivals at the barrier, zeroed (n_wg > 1)
+    int *error;              // set when a barrier gave up, zeroed (n_wg > 1)
 };
 
-// Sum over the block in a fixed order (xor butterfly in each wave, then the
-// wave totals in wave order); every thread returns the total.
-__device__ double block_sum(double v, double *red)
+// energy and volume of bin b, from the run's range
+struct MHBins {
+    int nb, npt;
+    double emin, de, vmin, dv, p;
+    __device__ MHBins(const MHArgs &a, int run) : nb(a.n_bin), npt(a.npt)
+    {
+        emin = a.en_min[run];
+        de = (a.en_max[run] - emin) / (double)nb;
+        vmin = dv = p = 0.0;
+        if (npt) {
+            vmin = a.v_min[run];
+            dv = (a.v_max[run] - vmin) / (double)nb;
+            p = a.pressure[run];
+        }
+    }
+    __device__ double energy(int b) const { return emin + ((double)((npt ? b / nb : b) + 1) - 0.5) * de; }
+    __device__ double volume(int b) const { return npt ? vmin + ((double)(b % nb + 1) - 0.5) * dv : 0.0; }
+    __device__ double h(int b) const { return npt ? energy(b) + p * volume(b) : energy(b); }
+    __device__ size_t stride() const { return npt ? (size_t)(nb + 2) * (nb + 2) : (size_t)nb + 2; }
+    __device__ size_t cell(int b) const
+    {
+        return npt ? (size_t)(b / nb + 1) * (nb + 2) + (b % nb + 1) : (size_t)b + 1;
+    }
+};
+
+// sum over each row of 16 lanes and over the wave, in every lane
+__device__ __forceinline__ double mh_row_sum(double v) { return ptmc::group_sum<16>(v); }
+__device__ __forceinline__ double mh_wave_sum(double v)
 {
-    for (int o = 32; o > 0; o >>= 1) v = v + __shfl_xor(v, o, 64);
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) red[w] = v;
-    __syncthreads();
-    double t = 0.0;
-    for (int k = 0; k < MHN_THREADS / 64; ++k) t = t + red[k];
-    __syncthreads();
-    return t;
+    v = mh_row_sum(v);
+    v = v + __shfl_xor(v, 16, 64);
+    return v + __shfl_xor(v, 32, 64);
 }
 
-__global__ void __launch_bounds__(MHN_THREADS) multihist_npt_kernel(MHNArgs a)
+// total of one histogram over the workgroup's threads (red: a double per
+// wave), complete in thread 0
+__device__ double mh_total(const double *H, const MHBins &bins, int n_bins, double *red)
 {
-    extern __shared__ __align__(16) unsigned char lds[];
-    const int R = a.n_temps, nb = a.n_bin, run = blockIdx.x, tid = threadIdx.x;
-    const int B = nb * nb, W = nb + 2;
-    double *fe = reinterpret_cast<double *>(lds);  // R
-    double *nfe = fe + R;                          // R
-    double *ncyc = nfe + R;                        // R
-    double *beta = ncyc + R;                       // R
-    double *red = beta + R;                        // MHN_THREADS / 64
-    int *flag = reinterpret_cast<int *>(red + MHN_THREADS / 64);
+    double s = 0.0;
+    for (int b = threadIdx.x; b < n_bins; b += MH_THREADS) s = s + H[bins.cell(b)];
+    s = mh_wave_sum(s);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    for (int w = 1; w < MH_THREADS / 64; ++w) s = s + red[w];
+    return s;
+}
 
-    const double *H = a.hist + (size_t)run * R * W * W;
-    double *hs = a.scratch + (size_t)run * 3 * B;
-    double *off = hs + B;
-    double *ratio = off + B;
-    const double emin = a.en_min[run], vmin = a.v_min[run], p = a.pressure[run];
-    const double de = (a.en_max[run] - emin) / (double)nb;
-    const double dv = (a.v_max[run] - vmin) / (double)nb;
-    auto energy = [&](int b) { return emin + ((double)(b / nb + 1) - 0.5) * de; };
-    auto volume = [&](int b) { return vmin + ((double)(b % nb + 1) - 0.5) * dv; };
-    auto cell = [&](int i, int b) { return H[(size_t)i * W * W + (size_t)(b / nb + 1) * W + (b % nb + 1)]; };
+// histogram totals n_i: one workgroup per (run, temperature)
+__global__ void __launch_bounds__(MH_THREADS) mh_total_kernel(MHArgs a)
+{
+    __shared__ double red[MH_THREADS / 64];
+    const MHBins bins(a, blockIdx.x / a.n_temps);
+    const double s = mh_total(a.hist + (size_t)blockIdx.x * bins.stride(), bins, a.n_bins, red);
+    if (threadIdx.x == 0) a.ncyc[blockIdx.x] = s;
+}
 
-    for (int i = tid; i < R; i += MHN_THREADS) {
-        fe[i] = 0.0;
-        beta[i] = a.beta[(size_t)run * R + i];
-    }
-    for (int b = tid; b < B; b += MHN_THREADS) {
-        double s = 0.0;
-        for (int i = 0; i < R; ++i) s = s + cell(i, b);
-        hs[b] = s;
-    }
-    for (int i = 0; i < R; ++i) {
-        double s = 0.0;
-        for (int b = tid; b < B; b += MHN_THREADS) s = s + cell(i, b);
-        s = block_sum(s, red);
-        if (tid == 0) ncyc[i] = s;
+// All workgroups of a run have arrived `epoch` times.  The launch is
+// cooperative (every workgroup is resident), and a wait that lasts for
+// seconds gives up with the error flag, so every wave ends.
+__device__ bool mh_barrier(const MHArgs &a, int run, unsigned epoch, int *s_ok)
+{
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        __hip_atomic_fetch_add(&a.count[run], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned want = epoch * (unsigned)a.n_wg;
+        int ok = 0;
+        for (unsigned n = 0; n < MH_SPIN; ++n) {
+            if (__hip_atomic_load(&a.count[run], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= want) {
+                ok = 1;
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        if (!ok) *a.error = 1;
+        *s_ok = ok;
     }
     __syncthreads();
+    return *s_ok != 0;
+}
 
-    auto bin_terms = [&]() {
-        for (int b = tid; b < B; b += MHN_THREADS) {
-            const double h = energy(b) + p * volume(b);
+// LDS of mh_iterate_kernel in doubles: the temperatures' terms, and with KEEP
+// a slice of `bins` bins (matrix, histogram sums, offsets, ratios)
+__host__ __device__ inline size_t mh_lds(int R, bool keep, bool totals)
+{
+    return (size_t)3 * R + (keep || R <= MH_THREADS ? MH_THREADS : 0) + (totals ? R : 0);
+}
+__host__ __device__ inline size_t mh_slice(int R, size_t bins) { return bins * ((size_t)R + 3); }
+
+// The fixed point of every run.  KEEP: a workgroup keeps its bins' slice of K
+// and their terms in LDS; an iteration reads K twice, lanes over bins both
+// times (no bank conflicts), and ends in one sum per temperature.  Otherwise
+// (slices beyond LDS, and the entry point without workspace) an entry of K is
+// formed where it is read, with the same bits.  One workgroup per run where
+// the bins are few (NVT: 100-200) or there is no workspace; else the run's
+// bins are cut over n_wg workgroups, which exchange their sums once per
+// iteration (written and read past the per-XCD L2 by agent-scope accesses,
+// two buffers in turn so that one barrier suffices) and each form the same
+// free energies.  Sums are formed per block of MH_BINS bins and the blocks
+// added in one order, so that results do not depend on the cut.
+//
+// Bound by the latency of an iteration's chain (two reductions, one exp and
+// log per temperature, the barrier), not by arithmetic: 4.5 us an iteration
+// for 16 runs of 32 x 100 bins (917 -> 184 us a call's kernel against one
+// exponential per temperature and bin twice an iteration), 8 us for one run
+// of 48 x 10^4 bins on 79 workgroups (98 -> 1.02 ms; 17 us an iteration with
+// shuffles instead of row permutations and the exchange's loads one by one).
+template <bool KEEP>
+__global__ void __launch_bounds__(MH_THREADS) mh_iterate_kernel(MHArgs a)
+{
+    extern __shared__ __align__(16) unsigned char lds[];
+    __shared__ int s_ok, s_stop, s_rebase;
+    __shared__ double red[MH_THREADS / 64];
+    const int R = a.n_temps, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int run = blockIdx.x / a.n_wg, wg = blockIdx.x % a.n_wg;
+    const int b0 = wg * a.wg_blk * MH_BINS, nc = min(a.wg_blk * MH_BINS, a.n_bins - b0);
+    const int nblk = (nc + MH_BINS - 1) / MH_BINS;
+    // blocks are added in q interleaved sequences, then the sequences
+    const int q = R < MH_THREADS ? MH_THREADS / R : 1;
+    double *fe = reinterpret_cast<double *>(lds);  // R free energies
+    double *f0 = fe + R;                           // R those of K
+    double *wgt = f0 + R;                          // R: n_i exp(-(f_i - f0_i)), until the bins' ratios are formed
+    double *nfe = wgt;                             // R sums, then new free energies, after that
+    double *dpart = wgt + R;                       // halves of the bins' sums; the q sequences (R <= MH_THREADS)
+    double *end = fe + mh_lds(R, KEEP, false);
+    double *ncyc = a.ncyc ? a.ncyc + (size_t)run * R : end;  // end: the entry point without workspace, never KEEP
+    const size_t g0 = (size_t)run * a.n_bins + b0;
+    double *hs = end;                              // KEEP: nc histogram sums
+    double *off = KEEP ? hs + nc : a.off + g0;
+    double *ratio = KEEP ? off + nc : a.ratio + g0;  // H_m / D_m
+    double *K = ratio + nc;                        // KEEP: R x nc
+    const MHBins bins(a, run);
+    const double *beta = a.beta + (size_t)run * R;
+    const double *H = a.hist + (size_t)run * R * bins.stride();
+
+    for (int i = tid; i < R; i += MH_THREADS) fe[i] = 0.0;
+    if (!a.ncyc) {
+        for (int i = 0; i < R; ++i) {
+            const double s = mh_total(H + (size_t)i * bins.stride(), bins, a.n_bins, red);
+            if (tid == 0) ncyc[i] = s;
+            __syncthreads();
+        }
+    }
+    auto hist_sum = [&](int m) {
+        const double *h = H + bins.cell(b0 + m);
+        double s = 0.0;
+        for (int i = 0; i < R; ++i) s = s + h[(size_t)i * bins.stride()];
+        return s;
+    };
+    if constexpr (KEEP)
+        for (int m = tid; m < nc; m += MH_THREADS) hs[m] = hist_sum(m);
+    if (tid == 0) s_rebase = 1;
+    __syncthreads();
+
+    auto term = [&](int i, double h, double o) { return exp(-beta[i] * h - f0[i] - o); };
+    // offsets of the current free energies, K from them
+    auto rebase = [&]() {
+        for (int i = tid; i < R; i += MH_THREADS) f0[i] = fe[i];
+        for (int m = tid; m < nc; m += MH_THREADS) {
+            const double h = bins.h(b0 + m);
             double o = -1.0e6;
             for (int i = 0; i < R; ++i) o = fmax(o, -beta[i] * h - fe[i]);
-            o = o + log(1000.0);
-            double d = 0.0;
-            for (int i = 0; i < R; ++i) d = d + ncyc[i] * exp(-beta[i] * h - fe[i] - o);
-            off[b] = o;
-            ratio[b] = hs[b] / d;
+            off[m] = o + log(1000.0);
         }
+        __syncthreads();
+        if constexpr (KEEP)
+            for (int e = tid; e < R * nc; e += MH_THREADS) {
+                const int i = e / nc, m = e % nc;
+                K[e] = term(i, bins.h(b0 + m), off[m]);
+            }
+    };
+    // H_m / D_m: D_m from four interleaved sums over the temperatures, by one
+    // thread per bin, or by two where that leaves none idle
+    auto ratios = [&]() {
+        for (int i = tid; i < R; i += MH_THREADS) wgt[i] = ncyc[i] * exp(f0[i] - fe[i]);
+        __syncthreads();
+        if constexpr (KEEP) {
+            auto pair = [&](int m, int p) {
+                double d = 0.0, d1 = 0.0;
+                int i = p;
+#pragma unroll 4
+                for (; i + 2 < R; i += 4) {
+                    d = __builtin_fma(wgt[i], K[(size_t)i * nc + m], d);
+                    d1 = __builtin_fma(wgt[i + 2], K[(size_t)(i + 2) * nc + m], d1);
+                }
+                if (i < R) d = __builtin_fma(wgt[i], K[(size_t)i * nc + m], d);
+                return d + d1;
+            };
+            if (nc <= MH_THREADS / 2) {
+                const int m = tid % nc, p = tid / nc;
+                if (p < 2) dpart[tid] = pair(m, p);
+                __syncthreads();
+                if (tid < nc) ratio[tid] = hs[tid] / (dpart[tid] + dpart[nc + tid]);
+            } else {
+                for (int m = tid; m < nc; m += MH_THREADS) ratio[m] = hs[m] / (pair(m, 0) + pair(m, 1));
+            }
+        } else {
+            for (int m = tid; m < nc; m += MH_THREADS) {
+                const double h = bins.h(b0 + m), o = off[m];
+                double d[4] = {0.0, 0.0, 0.0, 0.0};
+                for (int i = 0; i < R; i += 4)
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        if (i + k < R) d[k] = __builtin_fma(wgt[i + k], term(i + k, h, o), d[k]);
+                ratio[m] = hist_sum(m) / ((d[0] + d[2]) + (d[1] + d[3]));
+            }
+        }
+        __syncthreads();
     };
 
     int it = 0;
     for (it = 1; it <= a.max_iter; ++it) {
-        bin_terms();
-        for (int i = 0; i < R; ++i) {
-            double s = 0.0;
-            for (int b = tid; b < B; b += MHN_THREADS) {
-                const double h = energy(b) + p * volume(b);
-                s = s + ratio[b] * exp(-beta[i] * h - off[b]);
+        if (s_rebase) rebase();
+        __syncthreads();
+        ratios();
+        double *part = a.n_wg > 1 ? a.part + ((size_t)run * 2 + (it & 1)) * a.n_blk * R : nullptr;
+        // block sums, a row of 16 lanes per temperature (all steps of the row
+        // sum are lane permutations of the VALU); without a cut they go
+        // straight into the sequences, each temperature's by one row in order
+        for (int i0 = 0; i0 < R; i0 += MH_THREADS / 16) {
+            const int i = i0 + tid / 16, row = tid & 15;
+            for (int g = 0; g < nblk; ++g) {
+                double s = 0.0;
+#pragma unroll
+                for (int u = 0; u < MH_BINS; u += 16) {
+                    const int m = g * MH_BINS + u + row;
+                    if (i < R && m < nc) {
+                        double k;
+                        if constexpr (KEEP) k = K[(size_t)i * nc + m];
+                        else k = term(i, bins.h(b0 + m), off[m]);
+                        s = __builtin_fma(ratio[m], k, s);
+                    }
+                }
+                s = mh_row_sum(s);
+                if (row == 0 && i < R) {
+                    if (a.n_wg > 1) {
+                        __hip_atomic_store(&part[(size_t)(wg * a.wg_blk + g) * R + i], s, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+                    } else {
+                        double *acc = q > 1 ? &dpart[(g % q) * R + i] : &nfe[i];
+                        *acc = g < q ? 0.0 + s : *acc + s;
+                    }
+                }
             }
-            s = block_sum(s, red);
-            if (tid == 0) nfe[i] = log(s);
+            if (a.n_wg == 1 && row == 0 && i < R)
+                for (int k = nblk; k < q; ++k) dpart[k * R + i] = 0.0;
+        }
+        if (a.n_wg > 1) {
+            if (!mh_barrier(a, run, (unsigned)it, &s_ok)) break;
+            for (int e = tid; e < q * R; e += MH_THREADS) {
+                const int i = e % R;
+                double s = 0.0;
+                // 16 loads in flight: each takes about a microsecond
+                for (int g = e / R; g < a.n_blk; g += 16 * q) {
+                    double v[16];
+#pragma unroll
+                    for (int u = 0; u < 16; ++u)
+                        if (g + u * q < a.n_blk)
+                            v[u] = __hip_atomic_load(&part[(size_t)(g + u * q) * R + i], __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+                    for (int u = 0; u < 16; ++u)
+                        if (g + u * q < a.n_blk) s = s + v[u];
+                }
+                if (q > 1) dpart[e] = s;
+                else nfe[e] = s;
+            }
         }
         __syncthreads();
-        if (tid == 0) {
-            double delta = 0.0;
-            for (int i = 0; i < R; ++i) {
-                const double d = fabs(nfe[i] - fe[i]);
+        for (int i = tid; i < R; i += MH_THREADS) {
+            double s = nfe[i];
+            if (q > 1) {
+                s = dpart[i];
+                for (int k = 1; k < q; ++k) s = s + dpart[k * R + i];
+            }
+            nfe[i] = f0[i] + log(s);
+        }
+        __syncthreads();
+        if (wave == 0) {
+            double delta = 0.0, far = 0.0;
+            bool nan = false;
+            for (int i = lane; i < R; i += 64) {
+                const double d = fabs(nfe[i] - fe[i]), r = fabs(nfe[i] - f0[i]);
                 delta = delta + d * d;
+                far = fmax(far, r);
+                nan = nan || !(r == r);
                 fe[i] = nfe[i];
             }
-            *flag = delta < a.conv;
-        }
-        __syncthreads();
-        if (*flag) break;
-    }
-    if (it > a.max_iter) it = a.max_iter;
-    bin_terms();
-    for (int j = 0; j < a.n_res; ++j) {
-        const double bt = a.beta_res[(size_t)run * a.n_res + j];
-        double s = 0.0;
-        for (int b = tid; b < B; b += MHN_THREADS) {
-            const double h = energy(b) + p * volume(b);
-            s = s + ratio[b] * exp(-bt * h - off[b]);
-        }
-        const double nc = block_sum(s, red);
-        double e1 = 0.0, v1 = 0.0, h1 = 0.0, h2 = 0.0;
-        for (int b = tid; b < B; b += MHN_THREADS) {
-            const double et = energy(b), vol = volume(b);
-            const double h = et + p * vol;
-            const double w = ratio[b] * exp(-bt * h - off[b]) / nc;
-            e1 = e1 + w * et;
-            v1 = v1 + w * vol;
-            h1 = h1 + w * h;
-            h2 = h2 + w * (h * h);
-        }
-        e1 = block_sum(e1, red);
-        v1 = block_sum(v1, red);
-        h1 = block_sum(h1, red);
-        h2 = block_sum(h2, red);
-        if (tid == 0) {
-            const double t = a.t_res[(size_t)run * a.n_res + j];
-            a.cp[(size_t)run * a.n_res + j] = (h2 - h1 * h1) / (a.k_boltzmann * (t * t));
-            if (a.moments) {
-                double *mo = a.moments + ((size_t)run * a.n_res + j) * 3;
-                mo[0] = e1;
-                mo[1] = v1;
-                mo[2] = h1;
+            delta = mh_wave_sum(delta);
+            const bool move = __ballot(nan || far > MH_REBASE) != 0ull;
+            if (lane == 0) {
+                s_stop = delta < a.conv;
+                s_rebase = move;
             }
         }
+        __syncthreads();
+        if (s_stop) break;
     }
-    if (a.free_energy)
-        for (int i = tid; i < R; i += MHN_THREADS) a.free_energy[(size_t)run * R + i] = fe[i];
-    if (tid == 0 && a.iterations) a.iterations[run] = it;
+    if (it > a.max_iter) it = a.max_iter;
+    // offsets and ratios of the last free energies, for the output grid
+    __syncthreads();
+    rebase();
+    __syncthreads();
+    ratios();
+    if constexpr (KEEP) {
+        for (int m = tid; m < nc; m += MH_THREADS) {
+            a.off[g0 + m] = off[m];
+            a.ratio[g0 + m] = ratio[m];
+        }
+    }
+    if (wg == 0) {
+        if (a.free_energy)
+            for (int i = tid; i < R; i += MH_THREADS) a.free_energy[(size_t)run * R + i] = fe[i];
+        if (tid == 0 && a.iterations) a.iterations[run] = it;
+    }
+}
+
+// Reweighting: one workgroup of T threads per (run, output temperature), one
+// pass over the bins.  h is taken from the middle of its range, so that the
+// variance loses fewer digits than <h^2> - <h>^2 of the raw values.
+template <int T>
+__global__ void __launch_bounds__(T) mh_result_kernel(MHArgs a)
+{
+    __shared__ double red[5][T / 64];
+    const int run = blockIdx.x / a.n_res, tid = threadIdx.x;
+    const MHBins bins(a, run);
+    const double *off = a.off + (size_t)run * a.n_bins, *ratio = a.ratio + (size_t)run * a.n_bins;
+    const double bt = a.beta_res[blockIdx.x];
+    const double mid = bins.h(a.npt ? (a.n_bin / 2) * a.n_bin + a.n_bin / 2 : a.n_bin / 2);
+    double s[5] = {0.0, 0.0, 0.0, 0.0, 0.0};  // 1, E, V, h, h^2
+    for (int b = tid; b < a.n_bins; b += T) {
+        const double h = bins.h(b);
+        const double q = ratio[b] * exp(-bt * h - off[b]);
+        const double hc = h - mid;
+        s[0] = s[0] + q;
+        if (a.npt) {
+            s[1] = __builtin_fma(q, bins.energy(b), s[1]);
+            s[2] = __builtin_fma(q, bins.volume(b), s[2]);
+        }
+        s[3] = __builtin_fma(q, hc, s[3]);
+        s[4] = __builtin_fma(q, hc * hc, s[4]);
+    }
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+        s[k] = mh_wave_sum(s[k]);
+        if ((tid & 63) == 0) red[k][tid >> 6] = s[k];
+    }
+    __syncthreads();
+    if (tid != 0) return;
+    for (int w = 1; w < T / 64; ++w)
+        for (int k = 0; k < 5; ++k) s[k] = s[k] + red[k][w];
+    const double h1 = s[3] / s[0], h2 = s[4] / s[0], t = a.t_res[blockIdx.x];
+    a.c[blockIdx.x] = (h2 - h1 * h1) / (a.k_boltzmann * (t * t));
+    if (a.moments) {
+        double *mo = a.moments + (size_t)blockIdx.x * 3;
+        mo[0] = s[1] / s[0];
+        mo[1] = s[2] / s[0];
+        mo[2] = h1 + mid;
+    }
 }
 
 // Device-resident scratch of the allocation-free entry point: the per-bin
-// terms of every run of one call (3 n_bin^2 doubles per run), one copy per
-// GPU for the life of the process.  Every element a call reads it has
-// written first (histogram sums, then offsets and ratios per iteration), so
-// nothing needs clearing between calls; calls that overlap on one GPU share
+// terms of every run of one call (3 n_bin^2 doubles per run are asked for, the
+// offsets and ratios use two thirds), one copy per GPU for the life of the
+// process.  Every element a call reads it has written first, so nothing needs
+// clearing between calls; calls that overlap on one GPU share
 // it and race.
 static __device__ __align__(256) double npt_scratch[PTMC_NOALLOC_NPT_SCRATCH_DOUBLES];
 
@@ -301,14 +427,188 @@ constexpr int MAX_DEVICES = 64;
 std::mutex npt_scratch_mutex;
 double *npt_scratch_ptr[MAX_DEVICES] = {};
 
-template <typename T>
-struct DBuf {
-    T *p = nullptr;
-    ~DBuf()
+// One device allocation of a call, cut into 256-byte aligned pieces.
+struct Arena {
+    char *p = nullptr;
+    size_t used = 0;
+    ~Arena()
     {
         if (p) (void)hipFree(p);
     }
+    size_t take(size_t bytes)
+    {
+        const size_t at = used;
+        used += (bytes + 255) & ~(size_t)255;
+        return at;
+    }
 };
+
+struct MHCall {
+    int n_runs, n_temps, n_bin, n_res, max_iter, npt;
+    const double *beta, *hist, *en_min, *en_max, *v_min, *v_max, *pressure, *beta_res, *t_res;
+    double k_boltzmann, conv;
+    double *c, *moments, *free_energy;
+    int *iterations;
+};
+
+#define MHCHK(x)                                     \
+    do {                                             \
+        if ((x) != hipSuccess) return PTMC_E_DEVICE; \
+    } while (0)
+
+// the output grid; a wave per temperature where a run has a few hundred bins
+hipError_t mh_results(const MHArgs &a, unsigned n, hipStream_t s)
+{
+    if (a.n_bins <= 512) hipLaunchKernelGGL(mh_result_kernel<64>, dim3(n), dim3(64), 0, s, a);
+    else hipLaunchKernelGGL(mh_result_kernel<256>, dim3(n), dim3(256), 0, s, a);
+    return hipGetLastError();
+}
+
+int mh_run(const MHCall &q, int device, size_t max_lds)
+{
+    const size_t R = q.n_temps, B = q.npt ? (size_t)q.n_bin * q.n_bin : (size_t)q.n_bin;
+    const size_t cells = q.npt ? (size_t)(q.n_bin + 2) * (q.n_bin + 2) : (size_t)q.n_bin + 2;
+    const size_t nR = (size_t)q.n_runs * R, nX = (size_t)q.n_runs * q.n_res;
+    int cus = 0;
+    MHCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+    // Workgroups of a run.  Up to 512 bins (NVT histograms) one, if its slice
+    // fits LDS: an iteration (4.5 us) is not worth a barrier between workgroups
+    // (about 3 us).  Else the bins are cut so that every slice fits LDS, and
+    // over more workgroups while the runs leave compute units idle (48 x 10^4
+    // NPT bins: 79 workgroups of one block each).
+    MHArgs a{};
+    a.n_blk = (int)((B + MH_BINS - 1) / MH_BINS);
+    auto cut = [&](int n) {
+        a.wg_blk = (a.n_blk + n - 1) / n;
+        a.n_wg = (a.n_blk + a.wg_blk - 1) / a.wg_blk;
+    };
+    auto slice = [&]() { return 8 * mh_slice(q.n_temps, std::min(B, (size_t)a.wg_blk * MH_BINS)); };
+    cut(1);
+    const size_t base = 8 * mh_lds(q.n_temps, true, false);
+    const size_t room = std::min(MH_SLICE_LDS, max_lds > base ? max_lds - base : 0);
+    if (B > 512 || slice() > room) {
+        cut(std::max(1, std::min(a.n_blk, cus / q.n_runs)));
+        while (slice() > room && a.wg_blk > 1 && a.n_wg < cus) cut(std::min(cus, 2 * a.n_wg));
+    }
+    const bool keep = slice() <= room;
+    const size_t lds = keep ? base + slice() : 8 * mh_lds(q.n_temps, false, false);
+    const void *fn = keep ? reinterpret_cast<const void *>(&mh_iterate_kernel<true>)
+                          : reinterpret_cast<const void *>(&mh_iterate_kernel<false>);
+    MHCHK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    // runs of one launch: all, or as many as are resident together when a run has several workgroups
+    const int batch = a.n_wg == 1 ? q.n_runs : std::max(1, std::min(q.n_runs, cus / a.n_wg));
+
+    Arena m;
+    const size_t o_small = m.take((2 * nX + nR + 5 * (size_t)q.n_runs) * 8);
+    const size_t o_hist = m.take(nR * cells * 8);
+    const size_t o_out = m.take(((q.moments ? 4 : 1) * nX + nR) * 8 + (size_t)q.n_runs * sizeof(int));
+    const size_t o_ncyc = m.take(nR * 8), o_off = m.take((size_t)q.n_runs * B * 8);
+    const size_t o_ratio = m.take((size_t)q.n_runs * B * 8);
+    const size_t o_part = m.take(a.n_wg > 1 ? 2 * nR * a.n_blk * 8 : 8);
+    const size_t o_count = m.take(((size_t)q.n_runs + 1) * sizeof(unsigned));
+    MHCHK(hipMalloc((void **)&m.p, m.used));
+
+    // the small inputs in one copy
+    std::vector<double> in(2 * nX + nR + 5 * (size_t)q.n_runs, 0.0);
+    double *w = in.data();
+    auto put = [&](const double *from, size_t n) {
+        if (from) std::memcpy(w, from, n * 8);
+        w += n;
+    };
+    put(q.beta, nR);
+    put(q.beta_res, nX);
+    put(q.t_res, nX);
+    for (const double *p : {q.en_min, q.en_max, q.v_min, q.v_max, q.pressure}) put(p, q.n_runs);
+    MHCHK(hipMemcpyAsync(m.p + o_small, in.data(), in.size() * 8, hipMemcpyHostToDevice, 0));
+    MHCHK(hipMemcpyAsync(m.p + o_hist, q.hist, nR * cells * 8, hipMemcpyHostToDevice, 0));
+    MHCHK(hipMemsetAsync(m.p + o_count, 0, ((size_t)q.n_runs + 1) * sizeof(unsigned), 0));
+
+    a.n_temps = q.n_temps;
+    a.n_bin = q.n_bin;
+    a.n_bins = (int)B;
+    a.n_res = q.n_res;
+    a.max_iter = q.max_iter;
+    a.npt = q.npt;
+    a.conv = q.conv;
+    a.k_boltzmann = q.k_boltzmann;
+    double *d = reinterpret_cast<double *>(m.p + o_small);
+    a.beta = d;
+    a.beta_res = d + nR;
+    a.t_res = d + nR + nX;
+    a.en_min = d + nR + 2 * nX;
+    a.en_max = a.en_min + q.n_runs;
+    a.v_min = a.en_max + q.n_runs;
+    a.v_max = a.v_min + q.n_runs;
+    a.pressure = a.v_max + q.n_runs;
+    a.hist = reinterpret_cast<double *>(m.p + o_hist);
+    a.c = reinterpret_cast<double *>(m.p + o_out);
+    a.moments = q.moments ? a.c + nX : nullptr;
+    a.free_energy = a.c + (q.moments ? 4 : 1) * nX;
+    a.iterations = reinterpret_cast<int *>(a.free_energy + nR);
+    a.ncyc = reinterpret_cast<double *>(m.p + o_ncyc);
+    a.off = reinterpret_cast<double *>(m.p + o_off);
+    a.ratio = reinterpret_cast<double *>(m.p + o_ratio);
+    a.part = reinterpret_cast<double *>(m.p + o_part);
+    a.count = reinterpret_cast<unsigned *>(m.p + o_count);
+    a.error = reinterpret_cast<int *>(a.count + q.n_runs);
+
+    hipLaunchKernelGGL(mh_total_kernel, dim3((unsigned)nR), dim3(MH_THREADS), 0, 0, a);
+    MHCHK(hipGetLastError());
+    for (int r0 = 0; r0 < q.n_runs; r0 += batch) {
+        const int nr = std::min(batch, q.n_runs - r0);
+        MHArgs b = a;  // the batch's runs
+        b.beta += (size_t)r0 * R;
+        b.hist += (size_t)r0 * R * cells;
+        b.en_min += r0;
+        b.en_max += r0;
+        b.v_min += r0;
+        b.v_max += r0;
+        b.pressure += r0;
+        b.free_energy += (size_t)r0 * R;
+        b.iterations += r0;
+        b.ncyc += (size_t)r0 * R;
+        b.off += (size_t)r0 * B;
+        b.ratio += (size_t)r0 * B;
+        b.part += 2 * (size_t)r0 * a.n_blk * R;
+        b.count += r0;
+        void *args[] = {&b};
+        if (a.n_wg > 1)
+            MHCHK(hipLaunchCooperativeKernel(fn, dim3(nr * a.n_wg), dim3(MH_THREADS), args, (unsigned)lds, 0));
+        else
+            MHCHK(hipLaunchKernel(fn, dim3(nr), dim3(MH_THREADS), args, lds, 0));
+    }
+    MHCHK(mh_results(a, (unsigned)nX, 0));
+
+    // all results in one copy
+    std::vector<char> out(((q.moments ? 4 : 1) * nX + nR) * 8 + (size_t)q.n_runs * sizeof(int));
+    int error = 0;
+    MHCHK(hipMemcpyAsync(out.data(), m.p + o_out, out.size(), hipMemcpyDeviceToHost, 0));
+    if (a.n_wg > 1) MHCHK(hipMemcpyAsync(&error, a.error, sizeof(int), hipMemcpyDeviceToHost, 0));
+    MHCHK(hipDeviceSynchronize());
+    if (error) return PTMC_E_DEVICE;
+    const char *r = out.data();
+    auto get = [&](void *to, size_t bytes) {
+        if (to) std::memcpy(to, r, bytes);
+        r += bytes;
+    };
+    get(q.c, nX * 8);
+    if (q.moments) get(q.moments, 3 * nX * 8);
+    get(q.free_energy, nR * 8);
+    get(q.iterations, (size_t)q.n_runs * sizeof(int));
+    return PTMC_OK;
+}
+
+// device and LDS checks of a call; lds: what the description needs at least
+int mh_device(int device, size_t lds, size_t &max_lds)
+{
+    int ndev = 0, v = 0;
+    if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= 0) return PTMC_E_NO_DEVICE;
+    if (device < 0 || device >= ndev || hipSetDevice(device) != hipSuccess) return PTMC_E_ARG;
+    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, device) != hipSuccess)
+        return PTMC_E_DEVICE;
+    max_lds = (size_t)v;
+    return lds > max_lds ? PTMC_E_UNSUPPORTED : PTMC_OK;
+}
 
 }  // namespace
 
@@ -321,60 +621,12 @@ extern "C" int ptmc_multihistogram_nvt(int32_t n_runs, int32_t n_temps, int32_t 
     if (n_runs <= 0 || n_temps <= 0 || n_bin <= 0 || n_result <= 0 || max_iter <= 0 || !beta || !hist ||
         !en_min || !en_max || !beta_result || !t_result || !cv)
         return PTMC_E_ARG;
-    int ndev = 0;
-    if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= 0) return PTMC_E_NO_DEVICE;
-    if (device < 0 || device >= ndev || hipSetDevice(device) != hipSuccess) return PTMC_E_ARG;
-    const size_t lds = sizeof(double) * (4 * (size_t)n_temps + 3 * (size_t)n_bin) + sizeof(int);
-    int max_lds = 0;
-    if (hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device) != hipSuccess)
-        return PTMC_E_DEVICE;
-    if (lds > (size_t)max_lds) return PTMC_E_UNSUPPORTED;
-    const size_t nR = (size_t)n_runs * n_temps, nH = nR * (n_bin + 2), nX = (size_t)n_runs * n_result;
-    DBuf<double> d_beta, d_hist, d_emin, d_emax, d_bres, d_tres, d_cv, d_fe;
-    DBuf<int> d_it;
-#define MHCHK(x)                                  \
-    do {                                          \
-        if ((x) != hipSuccess) return PTMC_E_DEVICE; \
-    } while (0)
-    MHCHK(hipMalloc((void **)&d_beta.p, nR * 8));
-    MHCHK(hipMalloc((void **)&d_hist.p, nH * 8));
-    MHCHK(hipMalloc((void **)&d_emin.p, n_runs * 8));
-    MHCHK(hipMalloc((void **)&d_emax.p, n_runs * 8));
-    MHCHK(hipMalloc((void **)&d_bres.p, nX * 8));
-    MHCHK(hipMalloc((void **)&d_tres.p, nX * 8));
-    MHCHK(hipMalloc((void **)&d_cv.p, nX * 8));
-    MHCHK(hipMalloc((void **)&d_fe.p, nR * 8));
-    MHCHK(hipMalloc((void **)&d_it.p, n_runs * sizeof(int)));
-    MHCHK(hipMemcpy(d_beta.p, beta, nR * 8, hipMemcpyHostToDevice));
-    MHCHK(hipMemcpy(d_hist.p, hist, nH * 8, hipMemcpyHostToDevice));
-    MHCHK(hipMemcpy(d_emin.p, en_min, n_runs * 8, hipMemcpyHostToDevice));
-    MHCHK(hipMemcpy(d_emax.p, en_max, n_runs * 8, hipMemcpyHostToDevice));
-    MHCHK(hipMemcpy(d_bres.p, beta_result, nX * 8, hipMemcpyHostToDevice));
-    MHCHK(hipMemcpy(d_tres.p, t_result, nX * 8, hipMemcpyHostToDevice));
-    MHArgs a{};
-    a.n_temps = n_temps;
-    a.n_bin = n_bin;
-    a.n_res = n_result;
-    a.max_iter = max_iter;
-    a.conv = conv_threshold;
-    a.beta = d_beta.p;
-    a.hist = d_hist.p;
-    a.en_min = d_emin.p;
-    a.en_max = d_emax.p;
-    a.beta_res = d_bres.p;
-    a.t_res = d_tres.p;
-    a.k_boltzmann = k_boltzmann;
-    a.cv = d_cv.p;
-    a.free_energy = d_fe.p;
-    a.iterations = d_it.p;
-    hipLaunchKernelGGL(multihist_kernel, dim3(n_runs), dim3(MH_THREADS), lds, 0, a);
-    MHCHK(hipGetLastError());
-    MHCHK(hipDeviceSynchronize());
-    MHCHK(hipMemcpy(cv, d_cv.p, nX * 8, hipMemcpyDeviceToHost));
-    if (free_energy) MHCHK(hipMemcpy(free_energy, d_fe.p, nR * 8, hipMemcpyDeviceToHost));
-    if (iterations) MHCHK(hipMemcpy(iterations, d_it.p, n_runs * sizeof(int), hipMemcpyDeviceToHost));
-#undef MHCHK
-    return PTMC_OK;
+    size_t max_lds = 0;
+    const int rc = mh_device(device, sizeof(double) * (4 * (size_t)n_temps + 3 * (size_t)n_bin) + sizeof(int), max_lds);
+    if (rc) return rc;
+    const MHCall q{n_runs, n_temps, n_bin, n_result, max_iter, 0, beta, hist, en_min, en_max, nullptr, nullptr,
+                   nullptr, beta_result, t_result, k_boltzmann, conv_threshold, cv, nullptr, free_energy, iterations};
+    return mh_run(q, device, max_lds);
 }
 
 extern "C" int ptmc_multihistogram_npt(int32_t n_runs, int32_t n_temps, int32_t n_bin, const double *beta,
@@ -388,70 +640,15 @@ extern "C" int ptmc_multihistogram_npt(int32_t n_runs, int32_t n_temps, int32_t 
         !en_min || !en_max || !v_min || !v_max || !pressure || !beta_result || !t_result || !cp)
         return PTMC_E_ARG;
     if ((int64_t)n_bin * n_bin > (int64_t)1 << 26) return PTMC_E_UNSUPPORTED;
-    int ndev = 0;
-    if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= 0) return PTMC_E_NO_DEVICE;
-    if (device < 0 || device >= ndev || hipSetDevice(device) != hipSuccess) return PTMC_E_ARG;
-    const size_t lds = sizeof(double) * (4 * (size_t)n_temps + MHN_THREADS / 64) + sizeof(int);
-    int max_lds = 0;
-    if (hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device) != hipSuccess)
-        return PTMC_E_DEVICE;
-    if (lds > (size_t)max_lds) return PTMC_E_UNSUPPORTED;
-    const size_t W = (size_t)n_bin + 2, B = (size_t)n_bin * n_bin;
-    const size_t nR = (size_t)n_runs * n_temps, nH = nR * W * W, nX = (size_t)n_runs * n_result;
-    DBuf<double> d_beta, d_hist, d_bounds, d_bres, d_tres, d_cp, d_mom, d_fe, d_scr;
-    DBuf<int> d_it;
-#define MHCHK(x)                                     \
-    do {                                             \
-        if ((x) != hipSuccess) return PTMC_E_DEVICE; \
-    } while (0)
-    MHCHK(hipMalloc((void **)&d_beta.p, nR * 8));
-    MHCHK(hipMalloc((void **)&d_hist.p, nH * 8));
-    MHCHK(hipMalloc((void **)&d_bounds.p, 5 * (size_t)n_runs * 8));
-    MHCHK(hipMalloc((void **)&d_bres.p, nX * 8));
-    MHCHK(hipMalloc((void **)&d_tres.p, nX * 8));
-    MHCHK(hipMalloc((void **)&d_cp.p, nX * 8));
-    MHCHK(hipMalloc((void **)&d_mom.p, 3 * nX * 8));
-    MHCHK(hipMalloc((void **)&d_fe.p, nR * 8));
-    MHCHK(hipMalloc((void **)&d_scr.p, 3 * B * (size_t)n_runs * 8));
-    MHCHK(hipMalloc((void **)&d_it.p, n_runs * sizeof(int)));
-    MHCHK(hipMemcpy(d_beta.p, beta, nR * 8, hipMemcpyHostToDevice));
-    MHCHK(hipMemcpy(d_hist.p, hist, nH * 8, hipMemcpyHostToDevice));
-    const double *bounds[5] = {en_min, en_max, v_min, v_max, pressure};
-    for (int k = 0; k < 5; ++k)
-        MHCHK(hipMemcpy(d_bounds.p + (size_t)k * n_runs, bounds[k], n_runs * 8, hipMemcpyHostToDevice));
-    MHCHK(hipMemcpy(d_bres.p, beta_result, nX * 8, hipMemcpyHostToDevice));
-    MHCHK(hipMemcpy(d_tres.p, t_result, nX * 8, hipMemcpyHostToDevice));
-    MHNArgs a{};
-    a.n_temps = n_temps;
-    a.n_bin = n_bin;
-    a.n_res = n_result;
-    a.max_iter = max_iter;
-    a.conv = conv_threshold;
-    a.beta = d_beta.p;
-    a.hist = d_hist.p;
-    a.en_min = d_bounds.p;
-    a.en_max = d_bounds.p + n_runs;
-    a.v_min = d_bounds.p + 2 * (size_t)n_runs;
-    a.v_max = d_bounds.p + 3 * (size_t)n_runs;
-    a.pressure = d_bounds.p + 4 * (size_t)n_runs;
-    a.beta_res = d_bres.p;
-    a.t_res = d_tres.p;
-    a.k_boltzmann = k_boltzmann;
-    a.cp = d_cp.p;
-    a.moments = d_mom.p;
-    a.free_energy = d_fe.p;
-    a.iterations = d_it.p;
-    a.scratch = d_scr.p;
-    hipLaunchKernelGGL(multihist_npt_kernel, dim3(n_runs), dim3(MHN_THREADS), lds, 0, a);
-    MHCHK(hipGetLastError());
-    MHCHK(hipDeviceSynchronize());
-    MHCHK(hipMemcpy(cp, d_cp.p, nX * 8, hipMemcpyDeviceToHost));
-    if (moments) MHCHK(hipMemcpy(moments, d_mom.p, 3 * nX * 8, hipMemcpyDeviceToHost));
-    if (free_energy) MHCHK(hipMemcpy(free_energy, d_fe.p, nR * 8, hipMemcpyDeviceToHost));
-    if (iterations) MHCHK(hipMemcpy(iterations, d_it.p, n_runs * sizeof(int), hipMemcpyDeviceToHost));
-#undef MHCHK
-    return PTMC_OK;
+    size_t max_lds = 0;
+    const int rc = mh_device(device, sizeof(double) * (4 * (size_t)n_temps + 4) + sizeof(int), max_lds);
+    if (rc) return rc;
+    const MHCall q{n_runs, n_temps, n_bin, n_result, max_iter, 1, beta, hist, en_min, en_max, v_min, v_max, pressure,
+                   beta_result, t_result, k_boltzmann, conv_threshold, cp, moments, free_energy, iterations};
+    return mh_run(q, device, max_lds);
 }
+
+#undef MHCHK
 
 extern "C" int ptmc_multihistogram_npt_noalloc(int32_t n_runs, int32_t n_temps, int32_t n_bin, const double *beta,
                                                const double *hist, const double *en_min, const double *en_max,
@@ -469,11 +666,14 @@ extern "C" int ptmc_multihistogram_npt_noalloc(int32_t n_runs, int32_t n_temps, 
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= 0) return PTMC_E_NO_DEVICE;
     if (device < 0 || device >= ndev || device >= MAX_DEVICES || hipSetDevice(device) != hipSuccess)
         return PTMC_E_ARG;
-    const size_t lds = sizeof(double) * (4 * (size_t)n_temps + MHN_THREADS / 64) + sizeof(int);
     int max_lds = 0;
     if (hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device) != hipSuccess)
         return PTMC_E_DEVICE;
-    if (lds > (size_t)max_lds) return PTMC_E_UNSUPPORTED;
+    if (sizeof(double) * (4 * (size_t)n_temps + 4) + sizeof(int) > (size_t)max_lds) return PTMC_E_UNSUPPORTED;
+    const size_t lds = 8 * mh_lds(n_temps, false, true);
+    if (hipFuncSetAttribute(reinterpret_cast<const void *>(&mh_iterate_kernel<false>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+        return PTMC_E_DEVICE;
     double *scr = nullptr;
     {
         std::lock_guard<std::mutex> lock(npt_scratch_mutex);
@@ -484,9 +684,13 @@ extern "C" int ptmc_multihistogram_npt_noalloc(int32_t n_runs, int32_t n_temps, 
         }
         scr = npt_scratch_ptr[device];
     }
-    MHNArgs a{};
+    MHArgs a{};
     a.n_temps = n_temps;
     a.n_bin = n_bin;
+    a.n_bins = n_bin * n_bin;
+    a.npt = 1;
+    a.n_blk = a.wg_blk = (a.n_bins + MH_BINS - 1) / MH_BINS;
+    a.n_wg = 1;
     a.n_res = n_result;
     a.max_iter = max_iter;
     a.conv = conv_threshold;
@@ -500,13 +704,15 @@ extern "C" int ptmc_multihistogram_npt_noalloc(int32_t n_runs, int32_t n_temps, 
     a.beta_res = beta_result;
     a.t_res = t_result;
     a.k_boltzmann = k_boltzmann;
-    a.cp = cp;
+    a.c = cp;
     a.moments = moments;
     a.free_energy = free_energy;
     a.iterations = iterations;
-    a.scratch = scr;
-    hipLaunchKernelGGL(multihist_npt_kernel, dim3(n_runs), dim3(MHN_THREADS), lds, static_cast<hipStream_t>(stream),
-                       a);
+    a.off = scr;
+    a.ratio = scr + (size_t)n_runs * a.n_bins;
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    hipLaunchKernelGGL(mh_iterate_kernel<false>, dim3(n_runs), dim3(MH_THREADS), lds, s, a);
     if (hipGetLastError() != hipSuccess) return PTMC_E_DEVICE;
+    if (mh_results(a, (unsigned)n_runs * (unsigned)n_result, s) != hipSuccess) return PTMC_E_DEVICE;
     return PTMC_OK;
 }
