@@ -163,6 +163,55 @@ __device__ __forceinline__ T group_sum(T v)
     return v;
 }
 
+// Value of the lane whose index differs in bit 4 (ROW = 16) or bit 5 (ROW =
+// 32), from gfx950's row swaps: v_permlane16_swap(a, b) exchanges the odd
+// 16-lane rows of a with the even rows of b, v_permlane32_swap(a, b) the upper
+// half of a with the lower half of b.  With a = b = v, the returned a holds
+// the even (lower) rows twice and b the odd (upper) rows twice, so a lane of
+// an even row finds its partner in b and a lane of an odd row in a.
+template <int ROW>
+__device__ __forceinline__ uint32_t row_xor_u32(uint32_t v)
+{
+    const bool odd = (threadIdx.x & ROW) != 0;
+    if constexpr (ROW == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        return odd ? r[0] : r[1];
+    } else {
+        static_assert(ROW == 32, "row swap of 16 or 32 lanes");
+        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        return odd ? r[0] : r[1];
+    }
+}
+template <int ROW>
+__device__ __forceinline__ float row_xor(float v) { return __uint_as_float(row_xor_u32<ROW>(__float_as_uint(v))); }
+
+// v + (v of the lane across the row boundary), from one row swap of v with
+// a copy of itself: after v_permlane16_swap(a = v, b = v) (or the 32-lane
+// swap) a lane of an even row holds its own value in a and its partner's in
+// b, a lane of an odd row the reverse, so a + b is the pair sum on every lane
+// (the same bits as v + partner: the two operands are the same, in either
+// order).
+template <int ROW>
+__device__ __forceinline__ float row_pair_sum(float v)
+{
+    const uint32_t u = __float_as_uint(v);
+    if constexpr (ROW == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    } else {
+        static_assert(ROW == 32, "row swap of 16 or 32 lanes");
+        const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+}
+template <int ROW>
+__device__ __forceinline__ double row_xor(double v)
+{
+    const uint64_t b = (uint64_t)__double_as_longlong(v);
+    const uint32_t lo = row_xor_u32<ROW>((uint32_t)b), hi = row_xor_u32<ROW>((uint32_t)(b >> 32));
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
 // Value of lane `src` (absolute lane index within the wave) of a 32-bit word.
 __device__ __forceinline__ uint32_t lane_get(uint32_t v, int src) { return (uint32_t)__shfl((int)v, src, 64); }
 

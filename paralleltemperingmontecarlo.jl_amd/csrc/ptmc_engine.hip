@@ -27,10 +27,10 @@ SweepFn nnp_sweep_da_fn();
 bool pair_slot_fns(int pk, int kc, bool da, SweepFn *sweep, SweepFn *init);
 size_t pair_slot_lds_bytes(bool da);
 SweepFn nnp_init_fn(int np);
-SweepFn nnp2_sweep_fn();
-SweepFn nnp2_init_fn();
-SweepFn nnp2_sweep_fn_f32();
-SweepFn nnp2_init_fn_f32();
+SweepFn nnp2_sweep_fn(bool pow);
+SweepFn nnp2_init_fn(bool pow);
+SweepFn nnp2_sweep_fn_f32(bool pow);
+SweepFn nnp2_init_fn_f32(bool pow);
 void (*nnp_cycle_fn())(SweepArgs, int);
 hipError_t sur_launch_desc(const float *x, const int32_t *n_atoms, float *bd, float r_cut, int n, hipStream_t st);
 hipError_t sur_launch_collect(const SweepArgs &a, int n_slots, float *bd, double *be, int32_t *bn, long long base,
@@ -181,13 +181,13 @@ struct ptmc_engine {
     bool nnvt = false;
     struct {
         std::vector<double> rad, ang, p1, p2;
-        std::vector<int32_t> grp, gfn;
+        std::vector<int32_t> grp, gfn, gprog;
         int n1 = 0, n2 = 0, n_swaps = 0, n_rad = 0, n_ang = 0, ng = 0, h1 = 0, h2 = 0, n_groups = 0;
         int act[4] = {0, 0, 0, 0};
         double r_cut = 0.0;
     } nnp2;
-    DevBuf<double> d_n2_rad, d_n2_ang, d_n2_p1, d_n2_p2, d_n2_feat, d_n2_eatom;
-    DevBuf<int32_t> d_n2_grp, d_n2_gfn;
+    DevBuf<double> d_n2_rad, d_n2_ang, d_n2_p1, d_n2_p2, d_n2_feat, d_n2_eatom, d_n2_pair;
+    DevBuf<int32_t> d_n2_grp, d_n2_gfn, d_n2_gprog;
     Nnp2Tables nnp2_dev{};
     size_t nnp2_lds = 0;
 
@@ -859,12 +859,26 @@ int prepare_nnp2(ptmc_engine *h)
     HIPCHK(h, hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
     const int N = n.n1 + n.n2;
     const bool f32 = h->cfg.precision == 1;
-    h->nnp2_lds = nnp2_lds_bytes(N, n.ng, n.n_rad + n.n_ang, n.h1, n.h2, f32 ? 4 : 8);
+    // groups of a pass: as many as the workgroup has pairs of waves, fewer
+    // where LDS would not hold their rows
+    int pass = std::max(1, std::min(NNP2_GP, n.n_groups));
+    auto lds = [&]() { return nnp2_lds_bytes(N, n.ng, n.n_ang, pass, n.h1, n.h2, f32 ? 4 : 8); };
+    while (pass > 1 && (long long)lds() > max_lds) --pass;
+    h->nnp2_lds = lds();
+    // weights into what LDS is left
+    const size_t esz = f32 ? 4 : 8, w23 = 2 * esz * ((size_t)n.h1 * n.h2 + 2 * n.h2 + 1), w1 = esz * ((size_t)n.ng + 1) * n.h1;
+    int stage = 0;
+    for (size_t add : {w23, w1, w1}) {
+        if (h->nnp2_lds + add > (size_t)max_lds) break;
+        h->nnp2_lds += add;
+        ++stage;
+    }
     if ((long long)h->nnp2_lds > max_lds)
         return fail(h, PTMC_E_UNSUPPORTED, "%d atoms with %d feature rows need %zu B of LDS (%d available)", N, n.ng,
                     h->nnp2_lds, max_lds);
-    const void *fs = (const void *)(f32 ? nnp2_sweep_fn_f32() : nnp2_sweep_fn());
-    const void *fi = (const void *)(f32 ? nnp2_init_fn_f32() : nnp2_init_fn());
+    const bool pw = std::find(n.gprog.begin(), n.gprog.end(), NNP2_POW) != n.gprog.end();
+    const void *fs = (const void *)(f32 ? nnp2_sweep_fn_f32(pw) : nnp2_sweep_fn(pw));
+    const void *fi = (const void *)(f32 ? nnp2_init_fn_f32(pw) : nnp2_init_fn(pw));
     HIPCHK(h, hipFuncSetAttribute(fs, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->nnp2_lds));
     HIPCHK(h, hipFuncSetAttribute(fi, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->nnp2_lds));
     int slot = 0;
@@ -894,10 +908,12 @@ int prepare_nnp2(ptmc_engine *h)
     int rc;
     if ((rc = upload(h, h->d_n2_rad, n.rad)) || (rc = upload(h, h->d_n2_ang, n.ang)) ||
         (rc = upload(h, h->d_n2_p1, n.p1)) || (rc = upload(h, h->d_n2_p2, n.p2)) ||
-        (rc = upload(h, h->d_n2_grp, n.grp)) || (rc = upload(h, h->d_n2_gfn, n.gfn)))
+        (rc = upload(h, h->d_n2_grp, n.grp)) || (rc = upload(h, h->d_n2_gfn, n.gfn)) ||
+        (rc = upload(h, h->d_n2_gprog, n.gprog)))
         return rc;
     if ((rc = dalloc(h, h->d_n2_feat, (size_t)slot * NNP_NP * n.ng))) return rc;
     if ((rc = dalloc(h, h->d_n2_eatom, (size_t)slot * NNP_NP))) return rc;
+    if ((rc = dalloc(h, h->d_n2_pair, (size_t)slot * n.n_groups * N * 64 / (f32 ? 2 : 1)))) return rc;
     Nnp2Tables &t = h->nnp2_dev;
     t.n1 = n.n1;
     t.n_swaps = n.n_swaps;
@@ -913,12 +929,16 @@ int prepare_nnp2(ptmc_engine *h)
     t.rad = h->d_n2_rad.p;
     t.ang = h->d_n2_ang.p;
     t.n_groups = n.n_groups;
+    t.pass = pass;
+    t.stage = stage;
     t.grp = h->d_n2_grp.p;
     t.gfn = h->d_n2_gfn.p;
+    t.gprog = h->d_n2_gprog.p;
     t.p1 = h->d_n2_p1.p;
     t.p2 = h->d_n2_p2.p;
     t.feat = h->d_n2_feat.p;
     t.eatom = h->d_n2_eatom.p;
+    t.pair = h->d_n2_pair.p;
     return PTMC_OK;
 }
 
@@ -1182,8 +1202,10 @@ int ptmc_destroy(ptmc_handle h)
     h->d_n2_p2.free_();
     h->d_n2_feat.free_();
     h->d_n2_eatom.free_();
+    h->d_n2_pair.free_();
     h->d_n2_grp.free_();
     h->d_n2_gfn.free_();
+    h->d_n2_gprog.free_();
     h->d_sur_w.free_();
     h->d_sur_m.free_();
     h->d_sur_v.free_();
@@ -1351,32 +1373,53 @@ int ptmc_set_potential_nnp2(ptmc_handle h, int32_t n1, int32_t n2, int32_t n_swa
     if (n.ang.empty()) n.ang.assign(15, 0.0);
     n.p1.assign(params1, params1 + n_params);
     n.p2.assign(params2, params2 + n_params);
-    // angular functions grouped by equal eta (first appearance order, stable
-    // inside a group), at most NNP2_GMAX per group
+    // angular functions grouped by equal eta (first appearance order), sorted
+    // by (lambda, zeta) so that powers follow from each other, at most
+    // NNP2_GMAX per group
     n.grp.clear();
     n.gfn.clear();
+    n.gprog.clear();
     {
         std::vector<char> done(n_ang, 0);
         for (int q = 0; q < n_ang; ++q) {
             if (done[q]) continue;
             const double eta = ang[(size_t)q * 15];
-            int cnt = 0;
+            std::vector<int32_t> same;
             for (int r = q; r < n_ang; ++r) {
                 if (done[r] || ang[(size_t)r * 15] != eta) continue;
-                if (cnt == NNP2_GMAX) {
-                    n.grp.push_back((int32_t)n.gfn.size() - cnt);
-                    n.grp.push_back(cnt);
-                    cnt = 0;
-                }
-                n.gfn.push_back(r);
+                same.push_back(r);
                 done[r] = 1;
-                ++cnt;
             }
-            n.grp.push_back((int32_t)n.gfn.size() - cnt);
-            n.grp.push_back(cnt);
+            auto key = [&](int32_t r) { return std::make_pair(ang[(size_t)r * 15 + 1], ang[(size_t)r * 15 + 2]); };
+            std::stable_sort(same.begin(), same.end(), [&](int32_t u, int32_t v) { return key(u) < key(v); });
+            for (size_t k = 0; k < same.size(); k += NNP2_GMAX) {
+                const size_t cnt = std::min(same.size() - k, (size_t)NNP2_GMAX);
+                n.grp.push_back((int32_t)n.gfn.size());
+                n.grp.push_back((int32_t)cnt);
+                n.gfn.insert(n.gfn.end(), same.begin() + k, same.begin() + k + cnt);
+                // powers: squarings of 1 + lambda cos, or of the function
+                // before where its zeta times a power of two is this one's
+                for (size_t l = 0; l < cnt; ++l) {
+                    auto doublings = [](double base, double zeta) {
+                        for (int d = 0; d < 8; ++d, base += base)
+                            if (base == zeta) return d;
+                        return -1;
+                    };
+                    const auto k1 = key(same[k + l]);
+                    int prog = NNP2_POW;
+                    const int fresh = doublings(1.0, k1.second);
+                    if (fresh >= 0) prog = NNP2_FRESH + fresh;
+                    if (l > 0 && n.gprog.back() != NNP2_POW && key(same[k + l - 1]).first == k1.first) {
+                        const int next = doublings(key(same[k + l - 1]).second, k1.second);
+                        if (next >= 0) prog = NNP2_CHAIN + next;
+                    }
+                    n.gprog.push_back(prog);
+                }
+            }
         }
         n.n_groups = (int)n.grp.size() / 2;
         if (n.gfn.empty()) n.gfn.assign(1, 0);
+        if (n.gprog.empty()) n.gprog.assign(1, 0);
         if (n.grp.empty()) n.grp.assign(2, 0);
     }
     PotParams p{};

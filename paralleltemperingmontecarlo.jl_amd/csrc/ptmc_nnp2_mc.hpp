@@ -7,31 +7,37 @@
 // :270-282), moves src/MCMoves.jl:115-145, :363-385, commit
 // src/swap_config.jl:223-277.
 //
-// One workgroup owns one configuration for a cycle of N + n_swaps moves, as
-// the single-species kernels do.  Its positions, squared distances and
-// cutoffs (R2, FC) and the trial feature matrix D live in LDS; the current
-// feature matrix G and per-atom energies stay in the slot's HBM buffers.
-// A move is an atom displacement or, with probability n_swaps / (N +
-// n_swaps), an exchange of one atom of each species (slot semantics: the
-// atoms keep their species and trade positions).  For the moved set M (one
-// atom, or the two swapped ones) the trial features are
-//   * columns of M: rebuilt in full from the trial positions, the partner
-//     pairs of an angular sum split into NNP2_NCH chunks whose partial sums
-//     are reduced in a fixed order;
-//   * columns within the cutoff of an old or new position of M: G plus the
-//     change of every radial pair and angular triangle holding an atom of M
-//     (new minus old, per-species scale);
-//   * other columns: unchanged, not built.
-// Only changed columns are built; the networks run on them alone (an
-// unchanged column gives the same atomic energy bit for bit), the
-// Metropolis test uses the FP64 energy change, and an accepted move writes
-// the changed columns back.  The reference builds the same trial matrix as
-// G plus deltas accumulated per pair / triangle (DeltaMatrix.jl:23-624);
-// every sum here is gathered by one thread in a fixed order, so a run does
-// not depend on the schedule and agrees with the reference's arithmetic to
-// rounding.  Angular functions of equal eta form groups that share each
-// triangle's cosine and exponential; (column, group) and (moved column,
-// group, chunk) tasks come from an LDS queue, heaviest first.
+// One workgroup owns one configuration for a cycle of N + n_swaps moves.  A
+// move is an atom displacement or, with probability n_swaps / (N + n_swaps),
+// an exchange of one atom of each species (slot semantics: the atoms keep
+// their species and trade positions).  The trial feature matrix D is the
+// current one, G, with
+//   * columns of unmoved atoms: plus the change of every radial pair and
+//     angular triangle holding a moved atom (new minus old, per-species scale);
+//   * columns of moved atoms: rebuilt from the trial positions.
+// The reference builds the same trial matrix as G plus deltas accumulated per
+// pair / triangle (DeltaMatrix.jl:23-624); every sum here is formed in a fixed
+// order, so a run does not depend on the schedule.
+//
+// The exponential and cutoffs of a triangle factor over its sides:
+//   exp(-eta (r_cj^2 + r_ck^2 + r_jk^2)) f_cj f_ck f_jk = P_cj P_ck P_jk,
+//   P_ab = exp(-eta r_ab^2) f_ab,
+// so that a triangle costs a cosine, two products and its functions' powers,
+// and exponentials are taken per pair only.  Angular functions of equal eta
+// form a group with one matrix P (device memory, the slot's own, rows of 64
+// lanes; read from L2, loads one partner ahead), two waves per group, each
+// over every other partner k with a lane per target atom j: k's record is the
+// same for all lanes, j's terms stay in registers, and the triangle's angle at
+// the moved atom is summed along the way (both orders of a pair).  Powers of
+// functions sorted by (lambda, zeta) come from one squaring chain.
+//
+// Bound by the instructions of the triangle visits (about 45 and 10 per
+// function each, only partners inside the cut-off, half of a move's time) and
+// the latency of the move's phases (rows, pair factors, three layers, commit).
+// Cu50Zn5 (5 + 26 functions, 7 groups, one workgroup of 16 waves per CU), a
+// launch of 57 moves: 11.1 ms with an exponential, a division and two square
+// roots per triangle and group, 1.9 ms so; 25 ladders of 10 1.35 -> 6.5e6
+// moves/s, 50 ladders in binary32 2.85 -> 8.5e6.
 // (no include guard: included once per element type)
 #include "ptmc_nnp_layout.hpp"
 #include "ptmc_sweep.hpp"
@@ -40,36 +46,114 @@ namespace ptmc {
 
 namespace {
 
-struct N2Lds {
-    N2R *X, *XT, *R2, *FC, *RN, *FN, *D, *eat, *eatn, *W, *S;
-    int *mi, *chg;
+constexpr int N2_NW = NNP2_NT / 64;
+
+// one move's draws: the atom move, and the species picks of a swap
+struct N2Draw {
+    MoveDraw<N2R> d;
+    int p, q;
 };
 
-__device__ inline N2Lds n2_lds(unsigned char *raw, int N, int ng, int nfn, int h1, int h2)
+// The potential's tables as the kernels read them: from the kernel argument
+// through a pointer that n2_fresh renews at every phase of a move, so that
+// the compiler loads a field where it is used instead of keeping all of them
+// (and spilling them) over the whole launch.
+typedef const __attribute__((address_space(4))) SweepArgs N2Args;
+typedef const __attribute__((address_space(4))) Nnp2Tables N2Tab;
+
+__device__ __forceinline__ N2Args &n2_args()
 {
+    N2Args *p = (N2Args *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *p;
+}
+__device__ __forceinline__ N2Tab &n2_fresh() { return n2_args().nnp2; }
+
+struct N2Group;
+
+// LDS, most of it at offsets known to the compiler
+struct N2Lds {
+    N2R *rec;                     // [2][64][8]: trial position, unit vector from the moved atom's trial position
+    N2Draw *dr;                   // draws of 64 moves
+    struct N2Group *G;            // [pass] group records
+    N2R *X;                       // [3][64] positions
+    N2R *r2n, *fn, *r2o, *fo, *rin;  // [2][64] of the moved atoms: trial and old r^2 and cutoff, trial 1/r
+    N2R *eat, *eatn;              // [64] per-atom energies, current and trial
+    N2R *RI;                      // [N][N] inverse distances (0 on the diagonal)
+    N2R *D;                       // [ng][N] trial features
+    N2R *H1, *H2;                 // [h1][N], [h2][N]
+    N2R *B;                       // [pass][NNP2_GMAX][2][N] changes of part 1 (over H1, H2)
+    N2R *PP;                      // [2][pass][64][2]: trial and old P of the moved atoms
+    N2R *S;                       // [2][n_ang][3][2] angular sums at the moved atoms
+    N2R *W;                       // staged weights
+};
+
+__device__ __forceinline__ N2Lds n2_lds(N2Tab &T, int N)
+{
+    extern __shared__ __align__(16) unsigned char lds_raw[];
     N2Lds l;
-    N2R *p = reinterpret_cast<N2R *>(raw);
-    l.X = p;
-    l.XT = l.X + 3 * N;
-    l.R2 = l.XT + 3 * N;
-    l.FC = l.R2 + N * N;
-    l.RN = l.FC + N * N;
-    l.FN = l.RN + 2 * N;
-    l.D = l.FN + 2 * N;
-    l.eat = l.D + (size_t)N * ng;
-    l.eatn = l.eat + N;
-    l.W = l.eatn + N;
-    l.S = l.W + 2 * nnp2_params(ng, h1, h2);
-    l.mi = reinterpret_cast<int *>(l.S + nnp2_scratch_doubles(N, nfn, h1, h2));
-    l.chg = l.mi + N;
+    l.rec = reinterpret_cast<N2R *>(lds_raw);
+    l.dr = reinterpret_cast<N2Draw *>(l.rec + 2 * 64 * 8);
+    l.G = reinterpret_cast<N2Group *>(reinterpret_cast<unsigned char *>(l.dr) + NNP2_DRAWS * NNP2_DRAW_BYTES);
+    l.X = reinterpret_cast<N2R *>(reinterpret_cast<unsigned char *>(l.G) + NNP2_GP * NNP2_GROUP_BYTES);
+    l.r2n = l.X + 3 * 64;
+    l.fn = l.r2n + 2 * 64;
+    l.r2o = l.fn + 2 * 64;
+    l.fo = l.r2o + 2 * 64;
+    l.rin = l.fo + 2 * 64;
+    l.eat = l.rin + 2 * 64;
+    l.eatn = l.eat + 64;
+    l.RI = l.eatn + 64;
+    l.PP = l.RI + N * N;
+    l.D = l.PP + 2 * T.pass * 64 * 2;
+    l.H1 = l.B = l.D + N * T.ng;
+    l.H2 = l.H1 + N * T.h1;
+    l.S = l.H1 + N * max(T.h1 + T.h2, 2 * NNP2_GMAX * T.pass);
+    l.W = l.S + 12 * T.n_ang;
     return l;
 }
+static_assert(sizeof(N2Draw) <= NNP2_DRAW_BYTES, "draw record");
 
-// type-2 cutoff (MachineLearningPotential/Cutoff.jl:79-90)
+// type-2 cutoff 0.5 (cos(pi r / rc) + 1) (MachineLearningPotential/Cutoff.jl:79-90)
+// as cos^2(pi t / 2), t = r / rc, the cosine by its Taylor series in t^2 (FP64
+// through t^24, remainder below 1e-18 on [0, 1]; binary32 through t^14)
 __device__ __forceinline__ N2R n2_cut(N2R r, N2R rc)
 {
-    return r < rc ? N2R(0.5) * (cos(N2R(3.14159265358979323846) * (r / rc)) + N2R(1.0)) : N2R(0.0);
+    constexpr int K = sizeof(N2R) == 8 ? 12 : 7;
+    const N2R t = r / rc, u = t * t;
+    N2R c = (N2R)cutoff_cos_coef(K);
+#pragma unroll
+    for (int k = K - 1; k >= 0; --k) c = fma_<N2R>(c, u, (N2R)cutoff_cos_coef(k));
+    return r < rc ? c * c : N2R(0.0);
 }
+
+// tanh x = t / (t + 2), t = e^(2x) - 1 = 2^k q + (2^k - 1) with q = e^r - 1 by
+// its Taylor series, 2x = k ln 2 + r (Cody-Waite): within 2 ulp, small x
+// included; a fifth of the library's instructions.
+__device__ __forceinline__ double n2_tanh(double x)
+{
+    const double y = fmin(fabs(x), 20.0) * 2.0;
+    const double kd = rint(y * 1.4426950408889634);
+    const double r = fma(-kd, 1.90821492927058770002e-10, fma(-kd, 6.93147180369123816490e-01, y));
+    double q = 1.0 / 6227020800.0;
+    q = fma(q, r, 1.0 / 479001600.0);
+    q = fma(q, r, 1.0 / 39916800.0);
+    q = fma(q, r, 1.0 / 3628800.0);
+    q = fma(q, r, 1.0 / 362880.0);
+    q = fma(q, r, 1.0 / 40320.0);
+    q = fma(q, r, 1.0 / 5040.0);
+    q = fma(q, r, 1.0 / 720.0);
+    q = fma(q, r, 1.0 / 120.0);
+    q = fma(q, r, 1.0 / 24.0);
+    q = fma(q, r, 1.0 / 6.0);
+    q = fma(q, r, 0.5);
+    q = fma(q * r, r, r);
+    const double p = __longlong_as_double((long long)(1023 + (int)kd) << 52);
+    const double t = fma(p, q, p - 1.0);
+    const double v = t / (t + 2.0);
+    return x != x ? x : copysign(v, x);
+}
+__device__ __forceinline__ float n2_tanh(float x) { return tanhf(x); }
 
 __device__ __forceinline__ N2R n2_d2(const N2R *a, const N2R *b)
 {
@@ -83,7 +167,8 @@ __device__ __forceinline__ N2R n2_rad(N2R r2, N2R f, N2R eta)
     return (f != N2R(0.0) && f != N2R(1.0)) ? f * exp(-eta * r2) : N2R(0.0);
 }
 
-// (1 + lambda cos)^zeta: integer zeta by squaring, else pow
+// b^zeta: integer zeta by squaring, else pow (rounding can leave b = 1 +
+// lambda cos a little below zero)
 __device__ __forceinline__ N2R n2_pow(N2R b, N2R zeta)
 {
     if (zeta >= N2R(0.0) && zeta <= N2R(64.0) && zeta == rint(zeta)) {
@@ -96,590 +181,811 @@ __device__ __forceinline__ N2R n2_pow(N2R b, N2R zeta)
         }
         return r;
     }
-    return pow(b, zeta);
+    return pow(zeta == rint(zeta) || b > N2R(0.0) ? b : N2R(0.0), zeta);
 }
 
-// squared distance / cutoff between atoms a and b in the trial configuration
-__device__ __forceinline__ N2R n2_rt(const N2Lds &L, int N, int a, int b)
+// sum over the wave, in every lane
+__device__ __forceinline__ N2R n2_wave_sum(N2R v)
 {
-    const int ma = L.mi[a], mb = L.mi[b];
-    return ma >= 0 ? L.RN[ma * N + b] : (mb >= 0 ? L.RN[mb * N + a] : L.R2[a * N + b]);
-}
-__device__ __forceinline__ N2R n2_ft(const N2Lds &L, int N, int a, int b)
-{
-    const int ma = L.mi[a], mb = L.mi[b];
-    return ma >= 0 ? L.FN[ma * N + b] : (mb >= 0 ? L.FN[mb * N + a] : L.FC[a * N + b]);
+    v = group_sum<16>(v);
+    v = v + row_xor<16>(v);
+    return v + row_xor<32>(v);
 }
 
-// R2 / FC of the configuration X
-__device__ void n2_tables(const N2Lds &L, int N, N2R rc)
+__device__ __forceinline__ N2R n2_uniform(N2R v)
 {
-    for (int e = threadIdx.x; e < N * N; e += NNP2_NT) {
-        const int p = e / N, q = e % N;
-        const N2R r2 = p == q ? N2R(0.0) : n2_d2(&L.X[3 * p], &L.X[3 * q]);
-        L.R2[e] = r2;
-        L.FC[e] = n2_cut(sqrt(r2), rc);
+    if constexpr (sizeof(N2R) == 8) {
+        const uint64_t b = (uint64_t)__double_as_longlong((double)v);
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b);
+        const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
+        return (N2R)__longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+    } else {
+        return (N2R)__uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint((float)v)));
     }
 }
 
-// An angular group: the functions of one eta (at most NNP2_GMAX), which
-// share every triangle's geometry and exponential.
-struct N2Grp {
-    int cnt;
-    int q[NNP2_GMAX];
-    N2R lam[NNP2_GMAX], zeta[NNP2_GMAX];
-    N2R eta;
+// The functions of an angular group, sorted by (lambda, zeta), uniform over
+// the wave; prog[l] says how function l takes its power of b = 1 + lambda cos:
+// NNP2_FRESH + n: n squarings of a new b; NNP2_CHAIN + n: n squarings of
+// function l - 1's power; NNP2_POW: n2_pow (kernels compiled with POW; its
+// registers would spill the visits of the others).
+struct N2Group {
+    N2R eta, lam[NNP2_GMAX];
+    int cnt, q[NNP2_GMAX], prog[NNP2_GMAX];
 };
+static_assert(sizeof(N2Group) <= NNP2_GROUP_BYTES, "group record");
 
-__device__ __forceinline__ void n2_load_group(const Nnp2Tables &T, int g, N2Grp &G)
+// records of groups g0, g0 + 1, ... of a pass into LDS
+__device__ __forceinline__ void n2_stage_groups(N2Tab &T, N2Group *to, int g0)
 {
-    const int first = T.grp[2 * g], cnt = T.grp[2 * g + 1];
-    G.cnt = cnt;
+    for (int u = threadIdx.x; u < T.pass * NNP2_GMAX; u += NNP2_NT) {
+        const int gl = u / NNP2_GMAX, l = u % NNP2_GMAX;
+        if (g0 + gl >= T.n_groups) continue;
+        const int first = T.grp[2 * (g0 + gl)], cnt = T.grp[2 * (g0 + gl) + 1], f = first + (l < cnt ? l : 0), q = T.gfn[f];
+        to[gl].cnt = cnt;
+        to[gl].eta = (N2R)T.ang[(size_t)q * 15];
+        to[gl].q[l] = q;
+        to[gl].prog[l] = T.gprog[f];
+        to[gl].lam[l] = (N2R)T.ang[(size_t)q * 15 + 1];
+    }
+}
+
+// a record as uniform values
+__device__ __forceinline__ void n2_load_group(const N2Group &from, N2Group &G)
+{
+    G.cnt = __builtin_amdgcn_readfirstlane(from.cnt);
 #pragma unroll
     for (int l = 0; l < NNP2_GMAX; ++l) {
-        const int q = T.gfn[first + (l < cnt ? l : 0)];
-        G.q[l] = q;
-        G.lam[l] = T.ang[(size_t)q * 15 + 1];
-        G.zeta[l] = T.ang[(size_t)q * 15 + 2];
-    }
-    G.eta = T.ang[(size_t)T.gfn[first] * 15];
-}
-
-// cosine at c and exp(-eta (r_cj^2 + r_ck^2 + r_jk^2)) f_cj f_ck f_jk of triangle (c; j, k)
-// (SymmFunc.jl:184-202, Cutoff.jl:48-68)
-__device__ __forceinline__ void n2_tri_geom(const N2R *pc, const N2R *pj, const N2R *pk, N2R rcj,
-                                            N2R rck, N2R rjk, N2R fcj, N2R fck, N2R fjk, N2R eta,
-                                            N2R &cth, N2R &e)
-{
-    const N2R ux = pj[0] - pc[0], uy = pj[1] - pc[1], uz = pj[2] - pc[2];
-    const N2R wx = pk[0] - pc[0], wy = pk[1] - pc[1], wz = pk[2] - pc[2];
-    cth = (ux * wx + uy * wy + uz * wz) / (sqrt(rcj) * sqrt(rck));
-    e = exp(-eta * (rcj + rck + rjk)) * fcj * fck * fjk;
-}
-
-// acc[l] += e (1 + lambda_l cos)^zeta_l for the functions of the group
-__device__ __forceinline__ void n2_group_add(const N2Grp &G, N2R cth, N2R e, N2R (&acc)[NNP2_GMAX])
-{
-#pragma unroll
-    for (int l = 0; l < NNP2_GMAX; ++l)
-        if (l < G.cnt) acc[l] += e * n2_pow(N2R(1.0) + G.lam[l] * cth, G.zeta[l]);
-}
-
-// Radial sums of function q at centre c over the trial configuration:
-// s[0] partners of species 1, s[1] of species 2.
-__device__ void n2_radial_sums(const Nnp2Tables &T, const N2Lds &L, int N, int c, int q, N2R s[2])
-{
-    const int n1 = T.n1;
-    const N2R eta = (N2R)T.rad[(size_t)q * 9];
-    s[0] = s[1] = N2R(0.0);
-    for (int j = 0; j < N; ++j) {
-        if (j == c) continue;
-        s[j < n1 ? 0 : 1] += n2_rad(n2_rt(L, N, c, j), n2_ft(L, N, c, j), eta);
+        G.q[l] = __builtin_amdgcn_readfirstlane(from.q[l]);
+        G.prog[l] = __builtin_amdgcn_readfirstlane(from.prog[l]);
+        G.lam[l] = n2_uniform(from.lam[l]);
     }
 }
 
-// Angular sums of group g at centre c over the trial configuration XT, over
-// the partner pairs (j, k) with j = ch, ch + nch, ... (strided, so the
-// chunks mix near and far partners): out(l, row, v) adds v to row `row`
-// (partner pair 11 / 12 / 22) of the group's function l.  b is the other
-// moved atom of a swap (mb its row of RN / FN) or -1; the centre's own trial
-// row is read directly.
-template <typename Out>
-__device__ __forceinline__ void n2_group_sums(const Nnp2Tables &T, const N2Lds &L, const N2Grp &G, int N, int c, int b,
-                                              int mb, int ch, int nch, Out out)
+__device__ __forceinline__ N2R n2_group_eta(N2Tab &T, int g) { return (N2R)T.ang[(size_t)T.gfn[T.grp[2 * g]] * 15]; }
+
+// powers of NC cosines for every function of the group: use(l, p)
+template <bool POW, int NC, typename Use>
+__device__ __forceinline__ void n2_powers(N2Tab &T, const N2Group &G, const N2R (&c)[NC], Use use)
 {
-    const int n1 = T.n1;
-    const int mc = L.mi[c];
-    const N2R *rc_row = mc >= 0 ? &L.RN[mc * N] : &L.R2[c * N];
-    const N2R *fc_row = mc >= 0 ? &L.FN[mc * N] : &L.FC[c * N];
-    const N2R *pc = &L.XT[3 * c];
-    for (int j = ch; j < N; j += nch) {
-        if (j == c) continue;
-        const N2R fcj = fc_row[j];
-        if (fcj == N2R(0.0)) continue;
-        const N2R rcj = rc_row[j];
-        const int sj = j < n1 ? 0 : 1;
-        for (int blk = 0; blk < 2; ++blk) {
-            const int klo = blk ? (j + 1 > n1 ? j + 1 : n1) : j + 1, khi = blk ? N : n1;
-            if (klo >= khi) continue;
-            N2R acc[NNP2_GMAX];
+    N2R b[NC];
 #pragma unroll
-            for (int l = 0; l < NNP2_GMAX; ++l) acc[l] = N2R(0.0);
-            for (int k = klo; k < khi; ++k) {
-                if (k == c) continue;
-                const N2R fck = fc_row[k];
-                if (fck == N2R(0.0)) continue;
-                const N2R fjk = j == b ? L.FN[mb * N + k] : (k == b ? L.FN[mb * N + j] : L.FC[j * N + k]);
-                if (fjk == N2R(0.0)) continue;
-                const N2R rjk = j == b ? L.RN[mb * N + k] : (k == b ? L.RN[mb * N + j] : L.R2[j * N + k]);
-                N2R cth, e;
-                n2_tri_geom(pc, &L.XT[3 * j], &L.XT[3 * k], rcj, rc_row[k], rjk, fcj, fck, fjk, G.eta, cth, e);
-                n2_group_add(G, cth, e, acc);
+    for (int v = 0; v < NC; ++v) b[v] = N2R(1.0);
+#pragma unroll
+    for (int l = 0; l < NNP2_GMAX; ++l) {
+        if (l < G.cnt) {
+            const int pr = G.prog[l];
+            if (pr >= NNP2_FRESH) {
+#pragma unroll
+                for (int v = 0; v < NC; ++v) b[v] = fma_<N2R>(G.lam[l], c[v], N2R(1.0));
+                asm volatile("");  // a uniform branch, not two selects per power
             }
+            if (POW && pr == NNP2_POW) {
+                const N2R zeta = (N2R)T.ang[(size_t)G.q[l] * 15 + 2];
 #pragma unroll
-            for (int l = 0; l < NNP2_GMAX; ++l)
-                if (l < G.cnt) out(l, sj + blk, acc[l]);
+                for (int v = 0; v < NC; ++v) b[v] = n2_pow(b[v], zeta);
+            } else {
+                for (int q = pr & 15; q > 0; --q) {
+#pragma unroll
+                    for (int v = 0; v < NC; ++v) b[v] *= b[v];
+                }
+            }
+            use(l, b);
         }
     }
 }
 
-// scaled rows of radial function q / of the group at a centre of species sc
-__device__ __forceinline__ void n2_store_radial(const Nnp2Tables &T, N2R *Dc, int q, int sc, const N2R s[2])
+// inverse distances and the groups' P of the configuration X
+__device__ __forceinline__ void n2_tables(N2R *P, int N)
 {
-    const double *R = T.rad + (size_t)q * 9;
-    for (int r = 0; r < 2; ++r) Dc[2 * q + r] = s[r] * R[1 + 2 * sc + r] + R[5 + 2 * sc + r];
-}
-// radial rows of function q at an unmoved centre c: G plus the change of
-// every pair with a moved atom (ma[0..nm-1]), per-species scale
-__device__ void n2_delta_radial(const Nnp2Tables &T, const N2Lds &L, const N2R *Gc, int N, int c, int q, int nm,
-                                const int *ma)
-{
-    const int n1 = T.n1, sc = c < n1 ? 0 : 1;
-    const double *R = T.rad + (size_t)q * 9;
-    const N2R eta = R[0];
-    N2R acc[2] = {N2R(0.0), N2R(0.0)};
-    for (int m = 0; m < nm; ++m) {
-        const int a = ma[m];
-        acc[a < n1 ? 0 : 1] +=
-            n2_rad(L.RN[m * N + c], L.FN[m * N + c], eta) - n2_rad(L.R2[c * N + a], L.FC[c * N + a], eta);
-    }
-    N2R *Dc = &L.D[(size_t)c * T.ng];
-    for (int r = 0; r < 2; ++r) Dc[2 * q + r] = Gc[2 * q + r] + acc[r] * R[1 + 2 * sc + r];
-}
-
-// angular rows of group g at an unmoved centre c: G plus the change of every
-// triangle with a moved atom (new minus old), per-species scale, folded into
-// D block by block
-__device__ __forceinline__ void n2_delta_group(const Nnp2Tables &T, const N2Lds &L, const N2Grp &G, const N2R *Gc,
-                                               int N, int c, int nm, const int *ma)
-{
-    const int n1 = T.n1, sc = c < n1 ? 0 : 1;
-    const N2R *pc = &L.X[3 * c];
-    N2R *Dc = &L.D[(size_t)c * T.ng];
-#pragma unroll
-    for (int l = 0; l < NNP2_GMAX; ++l) {
-        if (l >= G.cnt) continue;
-        const int r = 2 * T.n_rad + 3 * G.q[l];
-        Dc[r] = Gc[r];
-        Dc[r + 1] = Gc[r + 1];
-        Dc[r + 2] = Gc[r + 2];
-    }
-    for (int m = 0; m < nm; ++m) {
-        const int a = ma[m], sa = a < n1 ? 0 : 1;
-        const N2R foca = L.FC[c * N + a], fnca = L.FN[m * N + c];
-        if (foca == N2R(0.0) && fnca == N2R(0.0)) continue;
-        const N2R roca = L.R2[c * N + a], rnca = L.RN[m * N + c];
-        for (int blk = 0; blk < 2; ++blk) {
-            N2R acc[NNP2_GMAX];
-#pragma unroll
-            for (int l = 0; l < NNP2_GMAX; ++l) acc[l] = N2R(0.0);
-            const int klo = blk ? n1 : 0, khi = blk ? N : n1;
-            for (int k = klo; k < khi; ++k) {
-                if (k == c || k == a) continue;
-                const int mk = L.mi[k];
-                if (mk >= 0 && mk < m) continue;  // the pair of two moved atoms counts once
-                N2R cth, e;
-                const N2R fck = L.FC[c * N + k];
-                if (foca != N2R(0.0) && fck != N2R(0.0)) {
-                    const N2R fak = L.FC[a * N + k];
-                    if (fak != N2R(0.0)) {
-                        n2_tri_geom(pc, &L.X[3 * a], &L.X[3 * k], roca, L.R2[c * N + k], L.R2[a * N + k], foca, fck,
-                                    fak, G.eta, cth, e);
-                        n2_group_add(G, cth, -e, acc);
-                    }
-                }
-                const N2R fnck = mk >= 0 ? L.FN[mk * N + c] : fck;
-                if (fnca != N2R(0.0) && fnck != N2R(0.0)) {
-                    const N2R fnak = L.FN[m * N + k];
-                    if (fnak != N2R(0.0)) {
-                        const N2R rnck = mk >= 0 ? L.RN[mk * N + c] : L.R2[c * N + k];
-                        n2_tri_geom(pc, &L.XT[3 * a], &L.XT[3 * k], rnca, rnck, L.RN[m * N + k], fnca, fnck, fnak,
-                                    G.eta, cth, e);
-                        n2_group_add(G, cth, e, acc);
-                    }
-                }
-            }
-            const int row = sa + blk;
-#pragma unroll
-            for (int l = 0; l < NNP2_GMAX; ++l) {
-                if (l >= G.cnt) continue;
-                const double *A = T.ang + (size_t)G.q[l] * 15;
-                Dc[2 * T.n_rad + 3 * G.q[l] + row] += acc[l] * A[3 + 3 * sc + row];
-            }
+    N2Tab &T = n2_fresh();
+    const N2Lds L = n2_lds(T, N);
+    for (int e = threadIdx.x; e < N * 64; e += NNP2_NT) {
+        const int k = e >> 6, j = e & 63;
+        N2R r2 = N2R(0.0), f = N2R(0.0);
+        if (j < N) {
+            const N2R pk[3] = {L.X[k], L.X[64 + k], L.X[128 + k]}, pj[3] = {L.X[j], L.X[64 + j], L.X[128 + j]};
+            r2 = n2_d2(pk, pj);
+            const N2R r = sqrt(r2);
+            f = j == k ? N2R(0.0) : n2_cut(r, (N2R)T.r_cut);
+            L.RI[k * N + j] = j == k ? N2R(0.0) : N2R(1.0) / r;
         }
+        for (int g = 0; g < T.n_groups; ++g)
+            P[((size_t)g * N + k) * 64 + j] = f != N2R(0.0) ? exp(-n2_group_eta(T, g) * r2) * f : N2R(0.0);
     }
 }
 
-__device__ __forceinline__ N2R n2_act(int code, N2R s) { return code == 2 ? tanh(s) : s; }
-
-// per-atom energies of the listed columns of D (RuNNer layout: per layer the
-// input-major weights, then the biases; one network per species)
-__device__ void n2_forward(const Nnp2Tables &T, const N2Lds &L, int N, int nc, const int *list)
+// sum of terms centred on an atom over the lanes j of species 1 or 2
+__device__ __forceinline__ N2R n2_species_sum(N2R v, int n1, int lane, bool second)
 {
-    const int tid = threadIdx.x, ng = T.ng, h1 = T.h1, h2 = T.h2, n1 = T.n1;
-    const size_t np = nnp2_params(ng, h1, h2);
-    N2R *H1 = L.S, *H2 = L.S + (size_t)N * h1;
-    for (int t = tid; t < nc * h1; t += NNP2_NT) {
-        const int ci = t / h1, j = t % h1, c = list[ci];
-        const N2R *p = c < n1 ? L.W : L.W + np;
-        const N2R *Dc = &L.D[(size_t)c * ng];
-        N2R s = N2R(0.0);
-        for (int k = 0; k < ng; ++k) s += Dc[k] * p[(size_t)k * h1 + j];
-        s += p[(size_t)ng * h1 + j];
-        H1[ci * h1 + j] = n2_act(T.act1, s);
-    }
-    __syncthreads();
-    const size_t o2 = (size_t)ng * h1 + h1;
-    for (int t = tid; t < nc * h2; t += NNP2_NT) {
-        const int ci = t / h2, j = t % h2, c = list[ci];
-        const N2R *p = (c < n1 ? L.W : L.W + np) + o2;
-        N2R s = N2R(0.0);
-        for (int k = 0; k < h1; ++k) s += H1[ci * h1 + k] * p[(size_t)k * h2 + j];
-        s += p[(size_t)h1 * h2 + j];
-        H2[ci * h2 + j] = n2_act(T.act2, s);
-    }
-    __syncthreads();
-    const size_t o3 = o2 + (size_t)h1 * h2 + h2;
-    for (int ci = tid; ci < nc; ci += NNP2_NT) {
-        const int c = list[ci];
-        const N2R *p = (c < n1 ? L.W : L.W + np) + o3;
-        N2R s = N2R(0.0);
-        for (int k = 0; k < h2; ++k) s += H2[ci * h2 + k] * p[k];
-        s += p[h2];
-        L.eatn[c] = n2_act(T.act3, s);
-    }
-    __syncthreads();
+    return n2_wave_sum((lane < n1) != second ? v : N2R(0.0));
 }
 
-// every column rebuilt from X (XT = X, nothing moved): D, eatn and the total
-__device__ double n2_rebuild(const Nnp2Tables &T, const N2Lds &L, int N, double *s_tot)
+// a and b exchanged across bit 5 or 4 of the lane and added: lanes with the
+// bit clear get a's sum over the two lanes, the others b's
+template <int ROW>
+__device__ __forceinline__ uint64_t n2_swap_words(uint32_t a, uint32_t b)
 {
-    for (int e = threadIdx.x; e < 3 * N; e += NNP2_NT) L.XT[e] = L.X[e];
-    __syncthreads();
-    const int nga = T.n_groups, nt = N * (nga + T.n_rad);
-    for (int t = threadIdx.x; t < nt; t += NNP2_NT) {
-        N2R *Dc;
-        if (t < N * nga) {
-            const int c = t / nga, g = t % nga;
-            N2Grp G;
-            n2_load_group(T, g, G);
-            Dc = &L.D[(size_t)c * T.ng];
-            const int sc = c < T.n1 ? 0 : 1;
-            // rows start at the offsets; each block adds its scaled sum
+    if constexpr (ROW == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+        return ((uint64_t)r[1] << 32) | r[0];
+    } else {
+        const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+        return ((uint64_t)r[1] << 32) | r[0];
+    }
+}
+template <int ROW>
+__device__ __forceinline__ float n2_merge(float a, float b)
+{
+    const uint64_t r = n2_swap_words<ROW>(__float_as_uint(a), __float_as_uint(b));
+    return __uint_as_float((uint32_t)r) + __uint_as_float((uint32_t)(r >> 32));
+}
+template <int ROW>
+__device__ __forceinline__ double n2_merge(double a, double b)
+{
+    const uint64_t x = (uint64_t)__double_as_longlong(a), y = (uint64_t)__double_as_longlong(b);
+    const uint64_t lo = n2_swap_words<ROW>((uint32_t)x, (uint32_t)y);
+    const uint64_t hi = n2_swap_words<ROW>((uint32_t)(x >> 32), (uint32_t)(y >> 32));
+    const uint64_t p = (hi << 32) | (uint32_t)lo, q = (hi & 0xffffffff00000000ull) | (lo >> 32);
+    return __longlong_as_double((long long)p) + __longlong_as_double((long long)q);
+}
+
+// Sums of eight values over the wave: lane l gets the sum of value 4 b5 + 2 b4
+// + b3 (bits of l).  The row swaps merge two values into one register per
+// step, 34 instructions in place of eight butterflies' 240.
+__device__ __forceinline__ N2R n2_sum8(const N2R (&v)[8], int lane)
+{
+    N2R a[4], b[2];
 #pragma unroll
-            for (int l = 0; l < NNP2_GMAX; ++l) {
-                if (l >= G.cnt) continue;
-                const double *A = T.ang + (size_t)G.q[l] * 15;
-                for (int r = 0; r < 3; ++r) Dc[2 * T.n_rad + 3 * G.q[l] + r] = A[9 + 3 * sc + r];
+    for (int i = 0; i < 4; ++i) a[i] = n2_merge<32>(v[i], v[i + 4]);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) b[i] = n2_merge<16>(a[i], a[i + 2]);
+    const bool odd = (lane & 8) != 0;
+    N2R s = (odd ? b[1] : b[0]) + dpp_perm<0x128>(odd ? b[0] : b[1]);  // row_ror 8: the lane across bit 3
+    s = s + dpp_perm<0xB1>(s);
+    s = s + dpp_perm<0x4E>(s);
+    return s + dpp_perm<0x141>(s);
+}
+
+// Visits of a wave: moved atom a (the m-th), partners k = part, part + 2, ...
+// of each species block, a lane per target j.  Changes of the rows of the
+// wave's group at the unmoved atoms: part 0 into D, part 1 into B (added to D
+// after a barrier); sums at the moved atom into S (both orders of an
+// equal-species pair are visited).  b: the other moved atom of a swap, a
+// partner at its trial position, or -1; the triangles with both moved atoms
+// count at j once (m = 0).
+template <bool POW, bool SWAP>
+__device__ __forceinline__ void n2_visits(const N2R *Pg, int N, int gl, int m, int a, int b, int part, int lane)
+{
+    N2Tab &T = n2_fresh();
+    const N2Lds L = n2_lds(T, N);
+    N2Group G;
+    n2_load_group(L.G[gl], G);
+    const int n1 = T.n1, lc = lane < N ? lane : N - 1;
+    const N2R *rec = L.rec + m * 64 * 8;
+    const N2R *pp = L.PP + (m * T.pass + gl) * 64 * 2;
+    const N2R *po = L.PP + ((1 - m) * T.pass + gl) * 64 * 2;  // of the other moved atom
+    const N2R xj = L.X[lc], yj = L.X[64 + lc], zj = L.X[128 + lc];
+    const N2R pnj = lane < N ? pp[2 * lc] : N2R(0.0), poj = lane < N ? -pp[2 * lc + 1] : N2R(0.0);
+    // unit vectors: trial moved atom -> j, and j -> old moved atom
+    const N2R vx = rec[8 * lc + 3], vy = rec[8 * lc + 4], vz = rec[8 * lc + 5];
+    const N2R rio = L.RI[a * N + lc];
+    const N2R ox = (L.X[a] - xj) * rio, oy = (L.X[64 + a] - yj) * rio, oz = (L.X[128 + a] - zj) * rio;
+    const bool still = lane < N && lane != a && lane != b;
+    const int sc = lane < n1 ? 0 : 1, sa = a < n1 ? 0 : 1;
+    // partners inside the cut-off of the trial or the old position (about two
+    // thirds of a 55-atom cluster); every other one is this wave's
+    uint64_t near = __ballot(lane < N && lane != a && (L.fn[m * 64 + lc] != N2R(0.0) || L.fo[m * 64 + lc] != N2R(0.0)));
+    const uint64_t first = n1 >= 64 ? ~0ull : (1ull << n1) - 1ull;
+    for (int blk = 0; blk < 2; ++blk) {
+        uint64_t left = near & (blk ? ~first : first);
+        if ((part ^ (blk ? __popcll(near & first) : 0)) & 1) left &= left - 1ull;
+        N2R accJ[NNP2_GMAX], own[NNP2_GMAX];
+#pragma unroll
+        for (int l = 0; l < NNP2_GMAX; ++l) accJ[l] = own[l] = N2R(0.0);
+        N2R pnext = left != 0ull ? Pg[__builtin_ctzll(left) * 64 + lane] : N2R(0.0);
+        while (left != 0ull) {
+            const int k = __builtin_ctzll(left);
+            left &= left - 1ull;
+            left &= left - 1ull;
+            const N2R p = pnext;
+            if (left != 0ull) pnext = Pg[__builtin_ctzll(left) * 64 + lane];
+            const N2R *rk = rec + 8 * k;
+            const N2R ri = L.RI[k * N + lc];
+            const N2R wx = rk[0] - xj, wy = rk[1] - yj, wz = rk[2] - zj;
+            N2R c[3];
+            c[0] = -fma_<N2R>(vz, wz, fma_<N2R>(vy, wy, vx * wx)) * ri;
+            c[1] = fma_<N2R>(oz, wz, fma_<N2R>(oy, wy, ox * wx)) * ri;
+            c[2] = fma_<N2R>(vz, rk[5], fma_<N2R>(vy, rk[4], vx * rk[3]));
+            N2R ea = p * pp[2 * k] * pnj;
+            N2R en = ea, eo = p * pp[2 * k + 1] * poj;
+            if constexpr (SWAP) {
+                if (k == b) {
+                    const N2R ux = L.X[b] - xj, uy = L.X[64 + b] - yj, uz = L.X[128 + b] - zj;
+                    c[0] = -fma_<N2R>(vz, wz, fma_<N2R>(vy, wy, vx * wx)) * L.rin[(1 - m) * 64 + lc];
+                    c[1] = fma_<N2R>(oz, uz, fma_<N2R>(oy, uy, ox * ux)) * ri;
+                    ea = po[2 * lc] * pp[2 * k] * pnj;
+                    en = m == 0 ? ea : N2R(0.0);
+                    if (m != 0) eo = N2R(0.0);
+                } else {
+                    ea = lane == b ? po[2 * k] * pp[2 * k] * pnj : ea;
+                }
             }
-            n2_group_sums(T, L, G, N, c, -1, 0, 0, 1, [&](int l, int row, N2R v) {
-                const double *A = T.ang + (size_t)G.q[l] * 15;
-                Dc[2 * T.n_rad + 3 * G.q[l] + row] += v * A[3 + 3 * sc + row];
+            n2_powers<POW, 3>(T, G, c, [&](int l, const N2R (&t)[3]) {
+                accJ[l] = fma_<N2R>(eo, t[1], fma_<N2R>(en, t[0], accJ[l]));
+                own[l] = fma_<N2R>(ea, t[2], own[l]);
             });
-        } else {
-            const int u = t - N * nga, c = u / T.n_rad, q = u % T.n_rad;
-            N2R s[2];
-            n2_radial_sums(T, L, N, c, q, s);
-            Dc = &L.D[(size_t)c * T.ng];
-            n2_store_radial(T, Dc, q, c < T.n1 ? 0 : 1, s);
+        }
+        // the scales first, so that their loads are in flight together
+        N2R sf[NNP2_GMAX];
+#pragma unroll
+        for (int l = 0; l < NNP2_GMAX; ++l) sf[l] = (N2R)T.ang[G.q[l] * 15 + 3 + 3 * sc + sa + blk];
+#pragma unroll
+        for (int l = 0; l < NNP2_GMAX; ++l) {
+            if (l < G.cnt) {
+                const int q = G.q[l];
+                if (still) {
+                    if (part == 0) L.D[(2 * T.n_rad + 3 * q + sa + blk) * N + lane] += accJ[l] * sf[l];
+                    else L.B[((gl * NNP2_GMAX + l) * 2 + blk) * N + lane] = accJ[l] * sf[l];
+                }
+            }
+        }
+        for (int sj = 0; sj <= blk; ++sj) {  // j of species 1, then of species 2 with k of species 2
+            N2R v[8] = {N2R(0.0), N2R(0.0), N2R(0.0), N2R(0.0), N2R(0.0), N2R(0.0), N2R(0.0), N2R(0.0)};
+#pragma unroll
+            for (int l = 0; l < NNP2_GMAX; ++l) v[l] = (lane < n1) == (sj == 0) ? own[l] : N2R(0.0);
+            const N2R sum = n2_sum8(v, lane);
+            const int l = (lane >> 5) * 4 + ((lane >> 4) & 1) * 2 + ((lane >> 3) & 1);
+            if ((lane & 7) == 0 && l < G.cnt)
+                L.S[((m * T.n_ang + L.G[gl].q[l]) * 3 + blk + sj) * 2 + part] = blk == sj ? N2R(0.5) * sum : sum;
         }
     }
-    for (int c = threadIdx.x; c < N; c += NNP2_NT) L.chg[c] = c;
-    __syncthreads();
-    n2_forward(T, L, N, N, L.chg);
-    if (threadIdx.x == 0) {
-        double tot = 0.0;
-        for (int c = 0; c < N; ++c) tot += (double)L.eatn[c];
-        *s_tot = tot;
+}
+static_assert(NNP2_GMAX <= 8, "n2_sum8 covers a group");
+
+__device__ __forceinline__ N2R n2_act(int code, N2R s) { return code == 2 ? n2_tanh(s) : s; }
+
+typedef N2R n2_x4 __attribute__((ext_vector_type(4)));
+typedef double n2_d4 __attribute__((ext_vector_type(4)));
+typedef float n2_f4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ n2_d4 n2_mfma(double a, double b, n2_d4 c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ n2_f4 n2_mfma(float a, float b, n2_f4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// One hidden layer of all atoms, out[h][N] = act(in[n][N] W + b), as 16 x 16
+// tiles (atoms x outputs) on the matrix cores: a wave per (species, tile) that
+// holds atoms of the species, whose rows it keeps.  Lane l holds A[row l % 16]
+// [k l / 16], B[k l / 16][column l % 16]; of the product value v belongs to
+// row 4 v + l / 16 (FP64) or 4 (l / 16) + v (binary32).  The weights come from
+// LDS where they were staged, else from L2, eight steps of k in flight.  The
+// activations follow over all threads: a tile's own lanes would spend the
+// padding's share on tanh too (20 outputs of 32).
+// lw: the layer's weights in LDS per species, or -1.
+__device__ __forceinline__ void n2_layer(const N2R *in, N2R *out, int N, int n, int h, int o, int act, const N2R *Wl,
+                                         int lw0, int lw1)
+{
+    N2Tab &T = n2_fresh();
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lr = lane & 15, lk = lane >> 4, n1 = T.n1;
+    // tiles of species 1 (atoms 0 .. n1 - 1), then of species 2
+    const int nct = (h + 15) / 16, nt1 = (n1 + 15) / 16 * nct, r2 = n1 / 16;
+    const int nt = nt1 + (n1 < N ? ((N + 15) / 16 - r2) * nct : 0);
+    for (int task = w; task < nt; task += N2_NW) {
+        const bool s = task >= nt1;
+        const int tt = s ? task - nt1 : task, rt = tt / nct + (s ? r2 : 0), ct = tt % nct;
+        const int lo = s ? n1 : 0, hi = s ? N : n1, lw = s ? lw1 : lw0;
+        const double *W = (s ? T.p2 : T.p1) + o;
+        const int at = min(16 * rt + lr, N - 1), j = min(16 * ct + lr, h - 1);
+        n2_x4 acc = {N2R(0.0), N2R(0.0), N2R(0.0), N2R(0.0)};
+        auto steps = [&](auto weight) {
+            const N2R *xp = in + lk * N + at;
+            int e = lk * h + j, k0 = 0;
+            for (; k0 + 32 <= n; k0 += 32, xp += 32 * N, e += 32 * h) {
+                N2R x[8], y[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    y[u] = weight(e + 4 * u * h);
+                    x[u] = xp[4 * u * N];
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u) acc = n2_mfma(x[u], y[u], acc);
+            }
+            for (; k0 < n; k0 += 4, xp += 4 * N, e += 4 * h) {
+                const bool in_row = k0 + lk < n;
+                const N2R y = weight(in_row ? e : j), x = in_row ? *xp : N2R(0.0);
+                acc = n2_mfma(x, y, acc);
+            }
+        };
+        if (lw >= 0) steps([&](int e) { return Wl[lw + e]; });
+        else steps([&](int e) { return (N2R)W[e]; });
+        if (16 * ct + lr < h) {
+            const N2R bias = lw >= 0 ? Wl[lw + n * h + j] : (N2R)W[n * h + j];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int row = 16 * rt + (sizeof(N2R) == 8 ? 4 * v + lk : 4 * lk + v);
+                if (row >= lo && row < hi) out[j * N + row] = acc[v] + bias;
+            }
+        }
     }
+    __syncthreads();
+    for (int e = threadIdx.x; e < h * N; e += NNP2_NT) out[e] = n2_act(act, out[e]);
+    __syncthreads();
+}
+
+// per-atom energies of D into eatn (RuNNer layout: per layer the input-major
+// weights, then the biases; one network per species); returns the FP64 total
+// in wave 0
+__device__ __forceinline__ double n2_forward(int N)
+{
+    N2Tab &T = n2_fresh();
+    const N2Lds L = n2_lds(T, N);
+    const int tid = threadIdx.x, lane = tid & 63, ng = T.ng, h1 = T.h1, h2 = T.h2;
+    // LDS holds (as T.stage says) layers 2 and 3 of both species, then layer 1
+    // of species 1, or of species 1 and 2
+    const int o2 = ng * h1 + h1, n23 = h1 * h2 + h2 + h2 + 1, st = T.stage;
+    n2_layer(L.D, L.H1, N, ng, h1, 0, T.act1, L.W, st > 1 ? 2 * n23 : -1, st > 2 ? 2 * n23 + o2 : -1);
+    n2_layer(L.H1, L.H2, N, h1, h2, o2, T.act2, L.W, st > 0 ? 0 : -1, st > 0 ? n23 : -1);
+    double tot = 0.0;
+    if (tid < 64) {
+        const int lc = lane < N ? lane : N - 1;
+        auto output = [&](auto weight) {
+            N2R s = N2R(0.0);
+#pragma unroll 8
+            for (int k = 0; k < h2; ++k) s = fma_<N2R>(L.H2[k * N + lc], weight(k), s);
+            return s + weight(h2);
+        };
+        N2R y;
+        if (st > 0) {
+            const N2R *p = L.W + (lc < T.n1 ? 0 : n23) + h1 * h2 + h2;
+            y = output([&](int k) { return p[k]; });
+        } else {
+            const double *p = (lc < T.n1 ? T.p1 : T.p2) + o2 + h1 * h2 + h2;
+            y = output([&](int k) { return (N2R)p[k]; });
+        }
+        y = n2_act(T.act3, y);
+        if (lane < N) {
+            L.eatn[lane] = y;
+            tot = (double)y;
+        }
+        tot = group_sum<16>(tot);
+        tot = tot + row_xor<16>(tot);
+        tot = tot + row_xor<32>(tot);
+    }
+    return tot;
+}
+
+// every column rebuilt from X: P, RI, D, eatn and the total
+template <bool POW>
+__device__ __forceinline__ double n2_rebuild(N2R *P, int N, double *s_tot)
+{
+    N2Tab &T = n2_fresh();
+    const N2Lds L = n2_lds(T, N);
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n1 = T.n1, lc = lane < N ? lane : N - 1;
+    __syncthreads();
+    n2_tables(P, N);
+    for (int g0 = 0; g0 == 0 || g0 < T.n_groups; g0 += T.pass) {
+        n2_stage_groups(T, L.G, g0);
+        __syncthreads();
+        // columns x (groups of the pass, then the radial functions)
+        const int ngp = min(T.pass, T.n_groups - g0);
+        for (int u = w; u < N * (ngp + (g0 == 0 ? T.n_rad : 0)); u += N2_NW) {
+            const int c = u % N, gl = u / N, g = g0 + gl, sc = c < n1 ? 0 : 1;
+            const N2R x = L.X[c], y = L.X[64 + c], z = L.X[128 + c];
+            if (gl >= ngp) {
+                const int q = gl - ngp;
+                const double *R = T.rad + (size_t)q * 9;
+                const N2R pc[3] = {x, y, z}, pj[3] = {L.X[lc], L.X[64 + lc], L.X[128 + lc]};
+                const N2R r2 = n2_d2(pc, pj);
+                const N2R v = lane < N && lane != c ? n2_rad(r2, n2_cut(sqrt(r2), (N2R)T.r_cut), (N2R)R[0]) : N2R(0.0);
+                for (int r = 0; r < 2; ++r) {
+                    const N2R s = n2_wave_sum((lane < n1) == (r == 0) ? v : N2R(0.0));
+                    if (lane == 0) L.D[(size_t)(2 * q + r) * N + c] = s * (N2R)R[1 + 2 * sc + r] + (N2R)R[5 + 2 * sc + r];
+                }
+                continue;
+            }
+            N2Group G;
+            n2_load_group(L.G[gl], G);
+            const N2R *Pg = P + (size_t)g * N * 64;
+            const N2R rj = L.RI[c * N + lc], pj = lane < N ? Pg[(size_t)c * 64 + lane] : N2R(0.0);
+            const N2R vx = (L.X[lc] - x) * rj, vy = (L.X[64 + lc] - y) * rj, vz = (L.X[128 + lc] - z) * rj;
+            for (int blk = 0; blk < 2; ++blk) {
+                N2R own[NNP2_GMAX];
+#pragma unroll
+                for (int l = 0; l < NNP2_GMAX; ++l) own[l] = N2R(0.0);
+                for (int k = blk ? n1 : 0; k < (blk ? N : n1); ++k) {
+                    const N2R e = Pg[(size_t)k * 64 + lane] * Pg[(size_t)c * 64 + k] * pj, rk = L.RI[c * N + k];
+                    const N2R wx = (L.X[k] - x) * rk, wy = (L.X[64 + k] - y) * rk, wz = (L.X[128 + k] - z) * rk;
+                    const N2R cs[1] = {fma_<N2R>(vz, wz, fma_<N2R>(vy, wy, vx * wx))};
+                    n2_powers<POW, 1>(T, G, cs, [&](int l, const N2R (&t)[1]) { own[l] = fma_<N2R>(e, t[0], own[l]); });
+                }
+#pragma unroll
+                for (int l = 0; l < NNP2_GMAX; ++l) {
+                    if (l < G.cnt) {
+                        const int q = G.q[l];
+                        auto store = [&](int row, N2R v) {
+                            const double *A = T.ang + (size_t)q * 15 + 3 * sc + row;
+                            if (lane == 0) L.D[(size_t)(2 * T.n_rad + 3 * q + row) * N + c] = v * (N2R)A[3] + (N2R)A[9];
+                        };
+                        // both orders of an equal-species pair were visited
+                        const N2R v = n2_species_sum(own[l], n1, lane, false);
+                        store(blk, blk ? v : N2R(0.5) * v);
+                        if (blk) store(2, N2R(0.5) * n2_species_sum(own[l], n1, lane, true));
+                    }
+                }
+            }
+        }
+        __syncthreads();
+    }
+    const double tot = n2_forward(N);
+    if (threadIdx.x == 0) *s_tot = tot;
     __syncthreads();
     return *s_tot;
 }
 
-__device__ void n2_load_x(const SweepArgs &a, const N2Lds &L, int slot, int N)
+__device__ __forceinline__ void n2_load_x(N2Args &a, const N2Lds &L, int slot, int N)
 {
     const N2R *gX = reinterpret_cast<const N2R *>(a.coords) + (size_t)slot * 3 * NNP_NP;
-    for (int e = threadIdx.x; e < 3 * N; e += NNP2_NT) {
-        const int j = e / 3, c = e % 3;
-        L.X[e] = gX[c * NNP_NP + j];
-        L.XT[e] = L.X[e];
-    }
-    for (int e = threadIdx.x; e < N; e += NNP2_NT) L.mi[e] = -1;
-    // both networks, staged once per launch
-    const Nnp2Tables &T = a.nnp2;
-    const int np = (int)nnp2_params(T.ng, T.h1, T.h2);
-    for (int e = threadIdx.x; e < 2 * np; e += NNP2_NT) L.W[e] = e < np ? T.p1[e] : T.p2[e - np];
+    for (int e = threadIdx.x; e < 3 * N; e += NNP2_NT) L.X[(e / N) * 64 + e % N] = gX[(e / N) * NNP_NP + e % N];
+}
+
+// the weights T.stage says, once per launch
+__device__ __forceinline__ void n2_stage_weights(N2Tab &T, N2R *W)
+{
+    const int o2 = T.ng * T.h1 + T.h1, n23 = T.h1 * T.h2 + T.h2 + T.h2 + 1;
+    if (T.stage > 0)
+        for (int e = threadIdx.x; e < 2 * n23; e += NNP2_NT) W[e] = (N2R)(e < n23 ? T.p1[o2 + e] : T.p2[o2 + e - n23]);
+    for (int s = 0; s + 2 <= T.stage; ++s)
+        for (int e = threadIdx.x; e < o2; e += NNP2_NT) W[2 * n23 + s * o2 + e] = (N2R)(s ? T.p2 : T.p1)[e];
+}
+
+__device__ __forceinline__ N2R *n2_pairs(N2Tab &T, int slot, int N)
+{
+    return reinterpret_cast<N2R *>(T.pair) + (size_t)slot * T.n_groups * N * 64;
 }
 
 // set_variables + initialise_energy (src/EnergyEvaluation.jl:1824-1856, :1748-1768)
-__global__ void __launch_bounds__(NNP2_NT) nnp2_init_kernel(SweepArgs a)
+template <bool POW>
+__global__ void __launch_bounds__(NNP2_NT) nnp2_init_kernel(SweepArgs)
 {
-    extern __shared__ __align__(16) unsigned char lds_raw[];
+    N2Args &a = n2_args();
     __shared__ double s_tot;
     const int slot = blockIdx.x;
     if (a.init_run >= 0 && a.slot_run[slot] != a.init_run) return;  // whole workgroup
-    const Nnp2Tables &T = a.nnp2;
+    N2Tab &T = a.nnp2;
     const int N = a.runs[a.slot_run[slot]].n_atoms;
-    const N2Lds L = n2_lds(lds_raw, N, T.ng, T.n_rad + T.n_ang, T.h1, T.h2);
+    const N2Lds L = n2_lds(T, N);
     n2_load_x(a, L, slot, N);
-    __syncthreads();
-    n2_tables(L, N, T.r_cut);
-    __syncthreads();
-    const double E = n2_rebuild(T, L, N, &s_tot);
+    n2_stage_weights(T, L.W);
+    const double E = n2_rebuild<POW>( n2_pairs(T, slot, N), N, &s_tot);
     N2R *gG = reinterpret_cast<N2R *>(T.feat) + (size_t)slot * NNP_NP * T.ng;
     for (int e = threadIdx.x; e < N * T.ng; e += NNP2_NT) gG[e] = L.D[e];
-    for (int e = threadIdx.x; e < NNP_NP; e += NNP2_NT) reinterpret_cast<N2R *>(T.eatom)[(size_t)slot * NNP_NP + e] = e < N ? L.eatn[e] : N2R(0.0);
+    for (int e = threadIdx.x; e < NNP_NP; e += NNP2_NT)
+        reinterpret_cast<N2R *>(T.eatom)[(size_t)slot * NNP_NP + e] = e < N ? L.eatn[e] : N2R(0.0);
     if (threadIdx.x == 0) a.slot_en[slot] = E;
+}
+
+// the moved atoms of a move (b = -1: one) and the trial position of one
+struct N2Move {
+    int a, b;
+    bool swap;
+    N2R tr[3];
+    __device__ int atom(int m) const { return m ? b : a; }
+    __device__ int other(int m) const { return m ? a : b; }
+};
+
+// Rows of the moved atoms: distances, cutoffs and unit vectors in the trial
+// configuration (waves 0, 1), distances and cutoffs in the old one (waves 2, 3).
+__device__ __forceinline__ void n2_rows(const N2Lds &L, const N2Move &mv, int N, int w, int lane, N2R rcut)
+{
+    const int mm = w & 1, aa = mv.atom(mm);
+    if (w >= 4 || (mm && !mv.swap) || lane >= N) return;
+    auto pos = [&](int j, N2R (&x)[3]) {
+        const bool now = w < 2;
+        const int i = now && mv.swap ? (j == mv.a ? mv.b : (j == mv.b ? mv.a : j)) : j;
+        const bool moved = now && !mv.swap && j == mv.a;
+        for (int k = 0; k < 3; ++k) x[k] = moved ? mv.tr[k] : L.X[64 * k + i];
+    };
+    N2R xa[3], xj[3];
+    pos(aa, xa);
+    pos(lane, xj);
+    const N2R r2 = lane == aa ? N2R(0.0) : n2_d2(xa, xj);
+    const N2R r = sqrt(r2), f = n2_cut(r, rcut);
+    if (w < 2) {
+        const N2R iv = lane == aa ? N2R(0.0) : N2R(1.0) / r;
+        L.r2n[mm * 64 + lane] = r2;
+        L.fn[mm * 64 + lane] = f;
+        L.rin[mm * 64 + lane] = iv;
+        N2R *rk = L.rec + (mm * 64 + lane) * 8;
+        for (int k = 0; k < 3; ++k) {
+            rk[k] = xj[k];
+            rk[3 + k] = (xj[k] - xa[k]) * iv;
+        }
+    } else {
+        L.r2o[mm * 64 + lane] = r2;
+        L.fo[mm * 64 + lane] = f;
+    }
+}
+
+// trial P of atom aa (the mm-th moved one) at eta, lane j; zero at itself
+__device__ __forceinline__ N2R n2_trial_pair(const N2Lds &L, N2R eta, int mm, int aa, int lane)
+{
+    const N2R f = L.fn[mm * 64 + lane];
+    return lane != aa && f != N2R(0.0) ? exp(-eta * L.r2n[mm * 64 + lane]) * f : N2R(0.0);
+}
+
+// Radial rows of moved atom mm, function q by the wave: changes at the
+// unmoved atoms, rebuilt entries at the moved one.
+__device__ __forceinline__ void n2_radial(int q, const N2Move &mv, int mm, int N, int lane)
+{
+    N2Tab &T = n2_fresh();
+    const N2Lds L = n2_lds(T, N);
+    const int n1 = T.n1, lc = lane < N ? lane : N - 1, aa = mv.atom(mm), sa = aa < n1 ? 0 : 1, sc = lane < n1 ? 0 : 1;
+    const double *R = T.rad + (size_t)q * 9;
+    const N2R eta = (N2R)R[0];
+    const N2R vn = lane < N ? n2_rad(L.r2n[mm * 64 + lc], L.fn[mm * 64 + lc], eta) : N2R(0.0);
+    if (lane < N && lane != mv.a && lane != mv.b) {
+        const N2R vo = n2_rad(L.r2o[mm * 64 + lc], L.fo[mm * 64 + lc], eta);
+        L.D[(2 * q + sa) * N + lane] += (vn - vo) * (N2R)R[1 + 2 * sc + sa];
+    }
+    for (int r = 0; r < 2; ++r) {
+        const N2R v = n2_species_sum(vn, n1, lane, r == 1);
+        if (lane == 0) L.D[(2 * q + r) * N + aa] = v * (N2R)R[1 + 2 * sa + r] + (N2R)R[5 + 2 * sa + r];
+    }
+}
+
+// Angular and radial rows of the trial features: the groups T.pass at a
+// time, two waves each; all threads call.
+template <bool POW>
+__device__ __forceinline__ void n2_features(const N2Move &mv, N2R *P, int N, int w, int lane)
+{
+    const int nm = mv.swap ? 2 : 1, gl = w >> 1, part = w & 1;
+    for (int g0 = 0; g0 == 0 || g0 < n2_fresh().n_groups; g0 += n2_fresh().pass) {
+        const int ngp = min(n2_fresh().pass, n2_fresh().n_groups - g0);
+        if (g0 > 0) __syncthreads();
+        {
+            // P of the moved atoms, trial and old
+            N2Tab &T = n2_fresh();
+            const N2Lds L = n2_lds(T, N);
+            if (T.n_groups > T.pass) n2_stage_groups(T, L.G, g0);
+            if (T.n_groups > T.pass) __syncthreads();
+            for (int u = w; u < nm * ngp; u += N2_NW) {
+                const int mm = u >= ngp, g = mm ? u - ngp : u, aa = mv.atom(mm);
+                if (lane < N) {
+                    N2R *pp = L.PP + ((mm * T.pass + g) * 64 + lane) * 2;
+                    const N2R old = P[((size_t)(g0 + g) * N + aa) * 64 + lane];
+                    pp[0] = n2_trial_pair(L, L.G[g].eta, mm, aa, lane);
+                    pp[1] = old;
+                }
+            }
+        }
+        __syncthreads();
+        for (int mm = 0; mm < nm; ++mm) {
+            const int aa = mv.atom(mm);
+            if (gl < ngp) {
+                const N2R *Pg = P + (size_t)(g0 + gl) * N * 64;
+                if (mv.swap) n2_visits<POW, true>(Pg, N, gl, mm, aa, mv.other(mm), part, lane);
+                else n2_visits<POW, false>(Pg, N, gl, mm, aa, -1, part, lane);
+            }
+            // radial functions, by the waves without a group if there are any
+            const int idle = N2_NW - 2 * ngp;
+            if (g0 == 0 && (idle == 0 || w >= 2 * ngp))
+                for (int q = idle ? w - 2 * ngp : w; q < n2_fresh().n_rad; q += idle ? idle : N2_NW)
+                    n2_radial(q, mv, mm, N, lane);
+            __syncthreads();
+            N2Tab &T = n2_fresh();
+            const N2Lds L = n2_lds(T, N);
+            const int sa = aa < T.n1 ? 0 : 1;
+            for (int u = w; u < ngp * 2 * NNP2_GMAX; u += N2_NW) {
+                const int g = u / (2 * NNP2_GMAX), l = u % (2 * NNP2_GMAX) / 2, blk = u & 1;
+                if (l < L.G[g].cnt && lane < N && lane != mv.a && lane != mv.b)
+                    L.D[(2 * T.n_rad + 3 * L.G[g].q[l] + sa + blk) * N + lane] += L.B[u * N + lane];
+            }
+            if (mm + 1 < nm) __syncthreads();
+        }
+    }
+    __syncthreads();
+    N2Tab &T = n2_fresh();
+    const N2Lds L = n2_lds(T, N);
+    for (int u = threadIdx.x; u < nm * T.n_ang * 3; u += NNP2_NT) {
+        const int mm = u >= T.n_ang * 3, v = mm ? u - T.n_ang * 3 : u, q = v / 3, row = v % 3, aa = mv.atom(mm);
+        const double *A = T.ang + (size_t)q * 15 + 3 * (aa < T.n1 ? 0 : 1) + row;
+        L.D[(2 * T.n_rad + 3 * q + row) * N + aa] = (L.S[2 * u] + L.S[2 * u + 1]) * (N2R)A[3] + (N2R)A[9];
+    }
+    __syncthreads();
+}
+
+// An accepted move: positions, distances, pair factors, features, energies
+// (swap_atom_config! / swap_move_config! with swap_vars!(NNPVariables2a)).
+__device__ __forceinline__ void n2_commit(const N2Move &mv, N2R *P, N2R *gG, int N, int w, int lane)
+{
+    N2Tab &T = n2_fresh();
+    const N2Lds L = n2_lds(T, N);
+    const int nm = mv.swap ? 2 : 1, tid = threadIdx.x;
+    if (w < nm && lane < N) {
+        const int aa = mv.atom(w);
+        const N2R v = L.rin[w * 64 + lane];
+        L.RI[aa * N + lane] = v;
+        L.RI[lane * N + aa] = v;
+    }
+    for (int u = w; u < nm * T.n_groups; u += N2_NW) {
+        const int mm = u >= T.n_groups, g = mm ? u - T.n_groups : u, aa = mv.atom(mm);
+        if (lane < N) {
+            const N2R v = T.n_groups <= T.pass ? L.PP[((mm * T.pass + g) * 64 + lane) * 2]
+                                               : n2_trial_pair(L, n2_group_eta(T, g), mm, aa, lane);
+            P[((size_t)g * N + aa) * 64 + lane] = v;
+            P[((size_t)g * N + lane) * 64 + aa] = v;
+        }
+    }
+    for (int e = tid; e < N * T.ng; e += NNP2_NT) gG[e] = L.D[e];
+    if (tid < 3 * nm) {
+        const int mm = tid >= 3, k = mm ? tid - 3 : tid, aa = mv.atom(mm);
+        L.X[k * 64 + aa] = L.rec[(mm * 64 + aa) * 8 + k];
+    }
+    if (tid < N) L.eat[tid] = L.eatn[tid];
 }
 
 // One cycle (N + n_swaps moves) of one configuration per workgroup
 // (mc_step! / mc_move!, src/MCRun.jl:142-182, with get_energy!(NNVT) :87-112).
-__global__ void __launch_bounds__(NNP2_NT) N2_SWEEP_ATTR nnp2_sweep_kernel(SweepArgs a)
+template <bool POW>
+__global__ void __launch_bounds__(NNP2_NT) nnp2_sweep_kernel(SweepArgs)
 {
-    extern __shared__ __align__(16) unsigned char lds_raw[];
-    __shared__ int s_err, s_nc, s_next;
+    __shared__ int s_err, s_acc;
     __shared__ double s_en;
-    const Nnp2Tables &T = a.nnp2;
-    const int slot = blockIdx.x, tid = threadIdx.x;
+    const int slot = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    N2Args &a = n2_args();
     const RunInfo &ri = a.runs[a.slot_run[slot]];
-    const int N = ri.n_atoms, n1 = T.n1, ng = T.ng, nfn = T.n_rad + T.n_ang;
-    const uint32_t nsteps = (uint32_t)(N + T.n_swaps);
-    const int t = a.slot_temp[slot];
-    const int Tg = ri.temp_base + t;
-    const uint32_t sweep = (uint32_t)a.sweep0;
+    const int N = __builtin_amdgcn_readfirstlane(ri.n_atoms);
+    const uint32_t nsteps = (uint32_t)(N + a.nnp2.n_swaps), sweep = (uint32_t)a.sweep0;
+    const uint32_t run_key = __builtin_amdgcn_readfirstlane(ri.run_key);
+    const int t = __builtin_amdgcn_readfirstlane(a.slot_temp[slot]);
+    const int Tg = __builtin_amdgcn_readfirstlane(ri.temp_base + t);
     const double beta = a.t_beta[Tg];
-    const N2R delta_r = (N2R)a.t_displ[2 * Tg];
-    const N2R radius2 = (N2R)ri.radius2;
-    const N2Lds L = n2_lds(lds_raw, N, ng, nfn, T.h1, T.h2);
-    N2R *gG = reinterpret_cast<N2R *>(T.feat) + (size_t)slot * NNP_NP * ng;
-
-    n2_load_x(a, L, slot, N);
-    for (int e = tid; e < N; e += NNP2_NT) L.eat[e] = reinterpret_cast<const N2R *>(T.eatom)[(size_t)slot * NNP_NP + e];
-    if (tid == 0) s_err = 0;
-    double E = a.slot_en[slot];
+    const N2R delta_r = n2_uniform((N2R)a.t_displ[2 * Tg]), radius2 = n2_uniform((N2R)ri.radius2);
+    N2R *gG = reinterpret_cast<N2R *>(a.nnp2.feat) + (size_t)slot * NNP_NP * a.nnp2.ng;  // [ng][N]
+    N2R *P = n2_pairs(a.nnp2, slot, N);
+    {
+        const N2Lds L = n2_lds(a.nnp2, N);
+        n2_load_x(a, L, slot, N);
+        n2_stage_groups(a.nnp2, L.G, 0);
+        n2_stage_weights(a.nnp2, L.W);
+        if (tid < N) L.eat[tid] = reinterpret_cast<const N2R *>(a.nnp2.eatom)[(size_t)slot * NNP_NP + tid];
+        if (tid == 0) {
+            s_err = 0;
+            s_en = a.slot_en[slot];
+        }
+    }
     __syncthreads();
-    n2_tables(L, N, T.r_cut);
-    __syncthreads();
-    long long nacc = 0, nsw = 0, nsw_acc = 0;
+    n2_tables(P, N);
+    double E = s_en;
+    int nacc = 0, nsw = 0, nsw_acc = 0;
 
     for (uint32_t m = 0; m < nsteps; ++m) {
-        // draws (every thread the same): the move index as mc_move! draws it
-        // (src/MCRun.jl:145), then the trial position (src/MCMoves.jl:115-135)
-        // or one atom of each species (src/MCMoves.jl:363-370)
-        const MoveDraw<N2R> d0 = move_draw<N2R>(a.seed, ri.run_key, (uint32_t)t, sweep, m, 0u, nsteps);
-        const bool swap = d0.index >= (uint32_t)N;
-        int ma[2] = {(int)d0.index, -1};
-        N2R tx = N2R(0.0), ty = N2R(0.0), tz = N2R(0.0);
-        if (swap) {
-            const u32x4 S = draw(a.seed, ri.run_key, RNG_MOVE, 254u, (uint32_t)t, sweep, m);
-            ma[0] = (int)below(S.x, (uint32_t)n1);
-            ma[1] = n1 + (int)below(S.y, (uint32_t)(N - n1));
-        } else {
-            const int i = ma[0];
-            make_trial<N2R, BC_SPHERE, false>(L.X[3 * i], L.X[3 * i + 1], L.X[3 * i + 2], d0, delta_r, N2R(0.0), N2R(0.0),
-                                                 tx, ty, tz);
-            int count = 0;
-            uint32_t attempt = 0;
-            while (outside_sphere<N2R>(tx, ty, tz, radius2)) {
-                count += 1;
-                if (count == 50) {
-                    // recentre! (src/Configurations.jl:79-85)
-                    __syncthreads();
-                    if (tid == 0) {
-                        double cm[3] = {0.0, 0.0, 0.0};
-                        for (int b = 0; b < N; ++b)
-                            for (int k = 0; k < 3; ++k) cm[k] += L.X[3 * b + k];
-                        for (int k = 0; k < 3; ++k) cm[k] /= (double)N;
-                        for (int b = 0; b < N; ++b)
-                            for (int k = 0; k < 3; ++k) L.X[3 * b + k] = (N2R)((double)L.X[3 * b + k] - cm[k]);
+        N2Move mv;
+        {
+            N2Args &a = n2_args();
+            N2Tab &T = a.nnp2;
+            const N2Lds L = n2_lds(T, N);
+            // the draws of 64 moves at a time, one lane each: the move index as
+            // mc_move! draws it (src/MCRun.jl:145), a trial displacement and the
+            // atoms of a swap (src/MCMoves.jl:363-370)
+            if (m % NNP2_DRAWS == 0) {
+                if (tid < NNP2_DRAWS && m + tid < nsteps) {
+                    N2Draw r;
+                    r.d = move_draw<N2R>(a.seed, run_key, (uint32_t)t, sweep, m + tid, 0u, nsteps);
+                    r.p = r.q = 0;
+                    if (r.d.index >= (uint32_t)N) {
+                        const u32x4 S = draw(a.seed, run_key, RNG_MOVE, 254u, (uint32_t)t, sweep, m + tid);
+                        r.p = (int)below(S.x, (uint32_t)T.n1);
+                        r.q = T.n1 + (int)below(S.y, (uint32_t)(N - T.n1));
                     }
-                    __syncthreads();
-                } else {
-                    attempt += 1;
-                    const MoveDraw<N2R> dd =
-                        move_draw<N2R>(a.seed, ri.run_key, (uint32_t)t, sweep, m, attempt, nsteps);
-                    make_trial<N2R, BC_SPHERE, false>(L.X[3 * i], L.X[3 * i + 1], L.X[3 * i + 2], dd, delta_r,
-                                                         N2R(0.0), N2R(0.0), tx, ty, tz);
-                    if (count == 100) {
-                        if (tid == 0) s_err = 1;
-                        break;
+                    L.dr[tid] = r;
+                }
+                __syncthreads();
+            }
+            const N2Draw &dr = L.dr[m % NNP2_DRAWS];
+            mv.swap = __builtin_amdgcn_readfirstlane((int)(dr.d.index >= (uint32_t)N)) != 0;
+            mv.a = __builtin_amdgcn_readfirstlane(mv.swap ? dr.p : (int)dr.d.index);
+            mv.b = __builtin_amdgcn_readfirstlane(mv.swap ? dr.q : -1);
+            mv.tr[0] = mv.tr[1] = mv.tr[2] = N2R(0.0);
+            if (!mv.swap) {
+                // trial position (src/MCMoves.jl:115-135), every thread the same
+                const int i = mv.a;
+                make_trial<N2R, BC_SPHERE, false>(L.X[i], L.X[64 + i], L.X[128 + i], dr.d, delta_r, N2R(0.0), N2R(0.0),
+                                                  mv.tr[0], mv.tr[1], mv.tr[2]);
+                int count = 0;
+                uint32_t attempt = 0;
+                while (outside_sphere<N2R>(mv.tr[0], mv.tr[1], mv.tr[2], radius2)) {
+                    count += 1;
+                    if (count == 50) {
+                        // recentre! (src/Configurations.jl:79-85)
+                        __syncthreads();
+                        if (tid < 3) {
+                            double cm = 0.0;
+                            for (int b = 0; b < N; ++b) cm += L.X[tid * 64 + b];
+                            cm /= (double)N;
+                            for (int b = 0; b < N; ++b) L.X[tid * 64 + b] = (N2R)((double)L.X[tid * 64 + b] - cm);
+                        }
+                        __syncthreads();
+                    } else {
+                        attempt += 1;
+                        const MoveDraw<N2R> dd = move_draw<N2R>(a.seed, run_key, (uint32_t)t, sweep, m, attempt, nsteps);
+                        make_trial<N2R, BC_SPHERE, false>(L.X[i], L.X[64 + i], L.X[128 + i], dd, delta_r, N2R(0.0),
+                                                          N2R(0.0), mv.tr[0], mv.tr[1], mv.tr[2]);
+                        if (count == 100) {
+                            if (tid == 0) s_err = 1;
+                            break;
+                        }
                     }
                 }
             }
-        }
-        const int nm = swap ? 2 : 1;
-        // trial positions and the moved set
-        for (int e = tid; e < 3 * N; e += NNP2_NT) {
-            const int j = e / 3, k = e % 3;
-            N2R v = L.X[e];
-            if (!swap && j == ma[0]) v = k == 0 ? tx : (k == 1 ? ty : tz);
-            if (swap && j == ma[0]) v = L.X[3 * ma[1] + k];
-            if (swap && j == ma[1]) v = L.X[3 * ma[0] + k];
-            L.XT[e] = v;
-        }
-        if (tid == 0) {
-            L.mi[ma[0]] = 0;
-            if (swap) L.mi[ma[1]] = 1;
-            s_next = NNP2_NT;
-        }
-        __syncthreads();
-        // distances and cutoffs of the moved atoms in the trial configuration
-        for (int e = tid; e < nm * N; e += NNP2_NT) {
-            const int mm = e / N, k = e % N, aa = ma[mm];
-            const N2R r2 = k == aa ? N2R(0.0) : n2_d2(&L.XT[3 * aa], &L.XT[3 * k]);
-            L.RN[e] = r2;
-            L.FN[e] = n2_cut(sqrt(r2), T.r_cut);
-        }
-        __syncthreads();
-        // changed columns: the moved atoms and every atom within the cutoff
-        // of an old or new position of one
-        auto changed = [&](int c) {
-            if (L.mi[c] >= 0) return true;
-            for (int mm = 0; mm < nm; ++mm)
-                if (L.FC[c * N + ma[mm]] != N2R(0.0) || L.FN[mm * N + c] != N2R(0.0)) return true;
-            return false;
-        };
-        if (tid < 64) {
-            const bool f = tid < N && changed(tid);
-            const uint64_t b = __ballot(f);
-            if (f) L.chg[__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u))] = tid;
-            if (tid == 0) s_nc = __builtin_popcountll(b);
-        }
-        // trial features from a queue of tasks, heaviest first: angular groups
-        // of unmoved changed columns (delta) and chunks of the moved columns
-        // (partial sums), then the radial functions of both
-        const int nga = T.n_groups, nAg = N * nga, nBg = nm * nga * NNP2_NCH, nAr = N * T.n_rad;
-        const int ntask = nAg + nBg + nAr + nm * T.n_rad;
-        for (int u = tid; u < ntask; u = atomicAdd(&s_next, 1)) {
-            if (u < nAg) {
-                // group-major: the lanes of a wave mostly share one group
-                const int g = u / N, c = u % N;
-                if (L.mi[c] >= 0 || !changed(c)) continue;  // moved: rebuilt below; unchanged: not read
-                N2Grp G;
-                n2_load_group(T, g, G);
-                n2_delta_group(T, L, G, gG + (size_t)c * ng, N, c, nm, ma);
-            } else if (u < nAg + nBg) {
-                const int v = u - nAg, mm = v / (nga * NNP2_NCH), g = (v / NNP2_NCH) % nga, ch = v % NNP2_NCH;
-                N2Grp G;
-                n2_load_group(T, g, G);
+            // D = G, eight loads in flight over the rows of the moved atoms
+            const int nd = N * T.ng;
+            N2R g[8];
 #pragma unroll
-                for (int l = 0; l < NNP2_GMAX; ++l) {
-                    if (l >= G.cnt) continue;
-                    N2R *P = &L.S[(((size_t)mm * nfn + T.n_rad + G.q[l]) * NNP2_NCH + ch) * 3];
-                    P[0] = P[1] = P[2] = N2R(0.0);
-                }
-                const int other = nm == 2 ? ma[1 - mm] : -1;
-                n2_group_sums(T, L, G, N, ma[mm], other, 1 - mm, ch, NNP2_NCH, [&](int l, int row, N2R v) {
-                    L.S[(((size_t)mm * nfn + T.n_rad + G.q[l]) * NNP2_NCH + ch) * 3 + row] += v;
-                });
-            } else if (u < nAg + nBg + nAr) {
-                const int v = u - nAg - nBg, c = v / T.n_rad, q = v % T.n_rad;
-                if (L.mi[c] >= 0 || !changed(c)) continue;
-                n2_delta_radial(T, L, gG + (size_t)c * ng, N, c, q, nm, ma);
-            } else {
-                const int v = u - nAg - nBg - nAr, mm = v / T.n_rad, q = v % T.n_rad;
-                N2R s2[2];
-                n2_radial_sums(T, L, N, ma[mm], q, s2);
-                N2R *P = &L.S[((size_t)mm * nfn + q) * NNP2_NCH * 3];
-                P[0] = s2[0];
-                P[1] = s2[1];
-                P[2] = N2R(0.0);
-                for (int e = 3; e < 3 * NNP2_NCH; ++e) P[e] = N2R(0.0);
-            }
+            for (int u = 0; u < 8; ++u) g[u] = gG[min(tid + u * NNP2_NT, nd - 1)];
+            n2_rows(L, mv, N, w, lane, (N2R)T.r_cut);
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (tid + u * NNP2_NT < nd) L.D[tid + u * NNP2_NT] = g[u];
+            for (int e = tid + 8 * NNP2_NT; e < nd; e += NNP2_NT) L.D[e] = gG[e];
         }
         __syncthreads();
-        for (int u = tid; u < nm * nfn; u += NNP2_NT) {
-            const int mm = u / nfn, fn = u % nfn, c = ma[mm];
-            N2R sum[3] = {N2R(0.0), N2R(0.0), N2R(0.0)};
-            const N2R *P = &L.S[((size_t)mm * nfn + fn) * NNP2_NCH * 3];
-            for (int ch = 0; ch < NNP2_NCH; ++ch)
-                for (int r = 0; r < 3; ++r) sum[r] += P[3 * ch + r];
-            N2R *Dc = &L.D[(size_t)c * ng];
-            const int sc = c < n1 ? 0 : 1;
-            if (fn < T.n_rad) {
-                n2_store_radial(T, Dc, fn, sc, sum);
-            } else {
-                const double *A = T.ang + (size_t)(fn - T.n_rad) * 15;
-                for (int r = 0; r < 3; ++r)
-                    Dc[2 * T.n_rad + 3 * (fn - T.n_rad) + r] = sum[r] * A[3 + 3 * sc + r] + A[9 + 3 * sc + r];
-            }
-        }
-        __syncthreads();
-        const int nc = s_nc;
-        n2_forward(T, L, N, nc, L.chg);
-        if (tid == 0) {
-            double tot = 0.0;
-            int q = 0;
-            for (int c = 0; c < N; ++c) {
-                if (q < nc && L.chg[q] == c) {
-                    tot += L.eatn[c];
-                    ++q;
-                } else {
-                    tot += L.eat[c];
+        n2_features<POW>(mv, P, N, w, lane);
+        const double new_en = n2_forward(N);
+        // Metropolis on the energy change (src/Exchange.jl:53-57, :74-83), by wave 0
+        if (w == 0) {
+            N2Args &a = n2_args();
+            const N2Lds L = n2_lds(a.nnp2, N);
+            const double dd = new_en - E;
+            const bool ok = (dd <= 0.0) || (det_exp(-dd * beta) >= L.dr[m % NNP2_DRAWS].d.umet);
+            if (tid == 0) {
+                s_acc = ok;
+                s_en = new_en;
+                if (a.trace_de != nullptr && a.trace_cycle < a.trace_cycles) {
+                    const size_t ti = ((size_t)Tg * a.trace_cycles + a.trace_cycle) * nsteps + m;
+                    a.trace_de[ti] = dd;
+                    a.trace_acc[ti] = (int8_t)ok;
+                    a.trace_idx[ti] = mv.swap ? N + mv.a * N + mv.b : mv.a;
                 }
             }
-            s_en = tot;
         }
         __syncthreads();
-        // Metropolis on the energy change (src/Exchange.jl:53-57, :74-83)
-        const double new_en = s_en;
-        const double dd = new_en - E;
-        const bool accept = (dd <= 0.0) || (det_exp(-dd * beta) >= d0.umet);
-        if (tid == 0 && a.trace_de != nullptr && a.trace_cycle < a.trace_cycles) {
-            const size_t ti = ((size_t)Tg * a.trace_cycles + a.trace_cycle) * nsteps + m;
-            a.trace_de[ti] = dd;
-            a.trace_acc[ti] = (int8_t)accept;
-            a.trace_idx[ti] = swap ? N + ma[0] * N + ma[1] : ma[0];
-        }
-        if (swap) nsw += 1;
-        if (accept) {
-            // swap_atom_config! / swap_move_config! with swap_vars!(NNPVariables2a)
-            for (int e = tid; e < 3 * N; e += NNP2_NT) L.X[e] = L.XT[e];
-            for (int e = tid; e < nm * N; e += NNP2_NT) {
-                const int mm = e / N, k = e % N, aa = ma[mm];
-                L.R2[aa * N + k] = L.RN[e];
-                L.R2[k * N + aa] = L.RN[e];
-                L.FC[aa * N + k] = L.FN[e];
-                L.FC[k * N + aa] = L.FN[e];
-            }
-            for (int e = tid; e < nc * ng; e += NNP2_NT) {
-                const int c = L.chg[e / ng], r = e % ng;
-                gG[(size_t)c * ng + r] = L.D[(size_t)c * ng + r];
-            }
-            for (int e = tid; e < nc; e += NNP2_NT) L.eat[L.chg[e]] = L.eatn[L.chg[e]];
-            E = new_en;
-            if (swap) nsw_acc += 1;
+        if (mv.swap) nsw += 1;
+        if (__builtin_amdgcn_readfirstlane(s_acc)) {
+            n2_commit(mv, P, gG, N, w, lane);
+            E = s_en;
+            if (mv.swap) nsw_acc += 1;
             else nacc += 1;
-        }
-        if (tid == 0) {
-            L.mi[ma[0]] = -1;
-            if (swap) L.mi[ma[1]] = -1;
         }
         __syncthreads();
     }
 
+    N2Args &z = n2_args();
+    const N2Lds L = n2_lds(z.nnp2, N);
     // periodic full rebuild bounds the drift of the incremental features
-    if (a.recompute_every > 0 && ((long long)sweep + 1) % a.recompute_every == 0) {
+    if (z.recompute_every > 0 && ((long long)sweep + 1) % z.recompute_every == 0) {
         __shared__ double s_tot;
-        const double Er = n2_rebuild(T, L, N, &s_tot);
+        const double Er = n2_rebuild<POW>(P, N, &s_tot);
         const double dr = __builtin_fabs(E - Er);
-        if (tid == 0 && dr > a.slot_drift[slot]) a.slot_drift[slot] = dr;
-        for (int e = tid; e < N * ng; e += NNP2_NT) gG[e] = L.D[e];
-        for (int e = tid; e < N; e += NNP2_NT) L.eat[e] = L.eatn[e];
+        if (tid == 0 && dr > z.slot_drift[slot]) z.slot_drift[slot] = dr;
+        for (int e = tid; e < N * z.nnp2.ng; e += NNP2_NT) gG[e] = L.D[e];
+        if (tid < N) L.eat[tid] = L.eatn[tid];
         E = Er;
         __syncthreads();
     }
 
-    N2R *gX = reinterpret_cast<N2R *>(a.coords) + (size_t)slot * 3 * NNP_NP;
-    for (int e = tid; e < 3 * N; e += NNP2_NT) gX[(e % 3) * NNP_NP + e / 3] = L.X[e];
-    for (int e = tid; e < N; e += NNP2_NT) reinterpret_cast<N2R *>(T.eatom)[(size_t)slot * NNP_NP + e] = L.eat[e];
+    N2R *gX = reinterpret_cast<N2R *>(z.coords) + (size_t)slot * 3 * NNP_NP;
+    for (int e = tid; e < 3 * N; e += NNP2_NT) gX[(e / N) * NNP_NP + e % N] = L.X[(e / N) * 64 + e % N];
+    if (tid < N) reinterpret_cast<N2R *>(z.nnp2.eatom)[(size_t)slot * NNP_NP + tid] = L.eat[tid];
     if (tid == 0) {
-        a.slot_en[slot] = E;
-        a.t_count_atom[2 * Tg] += nacc;
-        a.t_count_atom[2 * Tg + 1] += nacc;
-        a.t_count_vol[2 * Tg] += nsw_acc;
-        a.t_count_vol[2 * Tg + 1] += nsw;
-        if (s_err) a.run_error[a.slot_run[slot]] = 1;
+        z.slot_en[slot] = E;
+        z.t_count_atom[2 * Tg] += nacc;
+        z.t_count_atom[2 * Tg + 1] += nacc;
+        z.t_count_vol[2 * Tg] += nsw_acc;
+        z.t_count_vol[2 * Tg + 1] += nsw;
+        if (s_err) z.run_error[z.slot_run[slot]] = 1;
     }
 }
 
@@ -687,7 +993,7 @@ __global__ void __launch_bounds__(NNP2_NT) N2_SWEEP_ATTR nnp2_sweep_kernel(Sweep
 
 using SweepFn = void (*)(SweepArgs);
 
-SweepFn N2_SWEEP_FN() { return &nnp2_sweep_kernel; }
-SweepFn N2_INIT_FN() { return &nnp2_init_kernel; }
+SweepFn N2_SWEEP_FN(bool pow) { return pow ? &nnp2_sweep_kernel<true> : &nnp2_sweep_kernel<false>; }
+SweepFn N2_INIT_FN(bool pow) { return pow ? &nnp2_init_kernel<true> : &nnp2_init_kernel<false>; }
 
 }  // namespace ptmc

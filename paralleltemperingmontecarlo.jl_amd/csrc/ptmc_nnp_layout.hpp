@@ -84,30 +84,26 @@ __host__ __device__ inline size_t sur_lds_floats()
            3 * SUR_H + 4 * NNP_NP;
 }
 
-// Two-species NNVT kernels: threads per workgroup, chunks of the partner
-// pairs of a fully rebuilt feature column, and the LDS layout in doubles:
-// X[N][3] | XT[N][3] | R2[N][N] | FC[N][N] | RN[2][N] | FN[2][N] |
-// D[N][ng] | eat[N] | eatn[N] | W[2][n_params] (both networks) | scratch
-// (layer activations, or the partial sums of rebuilt columns) | ints:
-// moved index[N], changed list[N]
-constexpr int NNP2_NT = 512;
-constexpr int NNP2_NCH = 20;
-constexpr int NNP2_GMAX = 6;  // angular functions per eta group (larger groups are split)
-__host__ __device__ inline size_t nnp2_scratch_doubles(int N, int nfn, int h1, int h2)
+// Two-species NNVT kernels: threads per workgroup, angular functions per eta
+// group (larger groups are split), groups of one pass of a move (two waves
+// each), moves drawn together and the bytes of a draw record.
+constexpr int NNP2_NT = 1024;
+constexpr int NNP2_GMAX = 6;
+constexpr int NNP2_GP = NNP2_NT / 128;
+constexpr int NNP2_CHAIN = 0, NNP2_FRESH = 16, NNP2_POW = 32;  // how a function takes its power (+ squarings)
+constexpr int NNP2_DRAWS = 64;
+constexpr int NNP2_DRAW_BYTES = 48;
+constexpr int NNP2_GROUP_BYTES = 112;  // an angular group's record
+// LDS in bytes: rec[2][64][8] | draws | group records | X[3][64] | five rows [2][64] | eat,
+// eatn [64] | RI[N][N] | PP[2][pass][64][2] | D[ng][N] | H1[h1][N] and
+// H2[h2][N], or changes [pass][NNP2_GMAX][2][N] | S[2][n_ang][3][2]; esz: bytes
+// per element (8 for the FP64 kernels, 4 for binary32)
+__host__ __device__ inline size_t nnp2_lds_bytes(int N, int ng, int n_ang, int pass, int h1, int h2, int esz)
 {
-    const size_t act = (size_t)N * (h1 + h2), part = (size_t)2 * nfn * NNP2_NCH * 3;
-    return act > part ? act : part;
-}
-__host__ __device__ inline size_t nnp2_params(int ng, int h1, int h2)
-{
-    return (size_t)ng * h1 + h1 + (size_t)h1 * h2 + h2 + h2 + 1;
-}
-// esz: bytes per element (8 for the FP64 kernels, 4 for binary32)
-__host__ __device__ inline size_t nnp2_lds_bytes(int N, int ng, int nfn, int h1, int h2, int esz)
-{
-    const size_t d = (size_t)6 * N + 2 * (size_t)N * N + 4 * (size_t)N + (size_t)N * ng + 2 * (size_t)N +
-                     2 * nnp2_params(ng, h1, h2) + nnp2_scratch_doubles(N, nfn, h1, h2);
-    return d * (size_t)esz + 2 * (size_t)N * sizeof(int);
+    const size_t act = (size_t)h1 + h2, chg = 2 * NNP2_GMAX * (size_t)pass;
+    const size_t d = 64 * (size_t)(16 + 3 + 10 + 2 + 4 * pass) + (size_t)N * (N + ng + (act > chg ? act : chg)) +
+                     12 * (size_t)n_ang;
+    return d * (size_t)esz + (size_t)NNP2_DRAWS * NNP2_DRAW_BYTES + (size_t)NNP2_GP * NNP2_GROUP_BYTES;
 }
 
 }  // namespace ptmc

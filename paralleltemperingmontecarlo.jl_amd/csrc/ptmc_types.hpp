@@ -103,11 +103,14 @@ struct Nnp2Tables {
     double r_cut;
     const double *rad;         // n_rad x 9: eta, norm[4], offset[4]
     const double *ang;         // n_ang x 15: eta, lambda, zeta, tpz[6], offset[6]
-    int32_t n_groups;          // angular functions grouped by eta
+    int32_t n_groups, pass;    // angular functions grouped by eta; groups of one pass of a move
+    int32_t stage;             // weights in LDS: 1 layers 2 and 3; 2, 3: and layer 1 of species 1, of both
     const int32_t *grp;        // n_groups x 2: first entry in gfn, count
     const int32_t *gfn;        // n_ang angular function indices, group by group
+    const int32_t *gprog;      // n_ang: how each takes its power of 1 + lambda cos
     const double *p1, *p2;     // networks of species 1 and 2 (RuNNer layout)
-    double *feat;              // per slot [NNP_NP][ng] features, atom-major
+    double *feat;              // per slot [ng][N] features (room for NNP_NP atoms)
+    double *pair;              // per slot [n_groups][N][64] pair factors (scratch of a launch)
     double *eatom;             // per slot [NNP_NP] per-atom energies
 };
 
