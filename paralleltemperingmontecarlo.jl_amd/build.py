@@ -36,10 +36,11 @@ CFLAGS = [
 ]
 
 
-# The two-species move runs as one long loop with many phases: constants of
-# every phase's polynomials hoisted out of it spill to scratch (16 VGPRs and
-# 141 SGPRs spilled with hoisting, none and 104 without).
-NO_MACHINE_LICM = ("ptmc_nnp2_mc", "ptmc_nnp2_mc_f32")
+# The moves of the network potentials run as one long loop with many phases:
+# constants of every phase's polynomials hoisted out of it spill to scratch
+# (two species: 16 VGPRs and 141 SGPRs spilled with hoisting, none and 104
+# without; one species: 22 VGPRs with hoisting, none without).
+NO_MACHINE_LICM = ("ptmc_nnp", "ptmc_nnp2_mc", "ptmc_nnp2_mc_f32")
 
 
 def _compile(src: pathlib.Path) -> tuple[pathlib.Path, str]:

@@ -204,6 +204,22 @@ __device__ __forceinline__ float row_pair_sum(float v)
         return __uint_as_float(r[0]) + __uint_as_float(r[1]);
     }
 }
+// Two values merged across the row boundary: lanes of the even rows (the
+// lower half) get a + (a across the boundary), lanes of the odd rows (the
+// upper half) the same of b.
+template <int ROW>
+__device__ __forceinline__ float row_merge(float a, float b)
+{
+    const uint32_t x = __float_as_uint(a), y = __float_as_uint(b);
+    if constexpr (ROW == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    } else {
+        static_assert(ROW == 32, "row swap of 16 or 32 lanes");
+        const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+}
 template <int ROW>
 __device__ __forceinline__ double row_xor(double v)
 {

@@ -72,12 +72,11 @@ __device__ __forceinline__ void nnp_theta3(float lam, float kpow, float c0, floa
     }
 }
 
-// cosine of the angle at c between c->p and c->q (Cutoff.jl:48-58)
-__device__ __forceinline__ float nnp_cos(const float *c, const float *p, const float *q, float dcp, float dcq)
+// 1 / sqrt(x): the hardware's value (1 ulp) and one Newton step
+__device__ __forceinline__ float nnp_rsq(float x)
 {
-    const float ux = p[0] - c[0], uy = p[1] - c[1], uz = p[2] - c[2];
-    const float wx = q[0] - c[0], wy = q[1] - c[1], wz = q[2] - c[2];
-    return (ux * wx + uy * wy + uz * wz) / (dcp * dcq);
+    const float y = __builtin_amdgcn_rsqf(x);
+    return y * __builtin_fmaf(-0.5f * x * y, y, 1.5f);
 }
 
 // number of set bits of a 64-lane mask below this lane
@@ -123,49 +122,19 @@ __device__ __forceinline__ float row_sum16(float v)
     return v;
 }
 
-// Sum over all 64 lanes, complete in lane 63: row sums, then the last lane
-// of rows 0 and 2 broadcast into rows 1 and 3, then lane 31 into rows 2 and 3.
-__device__ __forceinline__ float wave_sum_last(float v)
-{
-    v = row_sum16(v);
-    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x142, 0xa, 0xf, false));
-    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x143, 0xc, 0xf, false));
-    return v;
-}
-
-
-// Accumulate e_new (1 + lam c_new)^(2^k) + e_old (1 + lam c_old)^(2^k) into
-// acc[S0 + k] for k = 0..kmax (kmax uniform; -1: no function of this lambda).
-// eo carries the sign of the old term.
-template <int S0>
-__device__ __forceinline__ void nnp_chain(int kmax, float lam, float cn, float co, float en, float eo, float *acc)
-{
-    if (kmax < 0) return;
-    float pn = 1.0f + lam * cn, po = 1.0f + lam * co;
-#pragma unroll
-    for (int k = 0; k < NNP_KSLOT; ++k) {
-        if (k <= kmax) {
-            acc[S0 + k] = __builtin_fmaf(en, pn, acc[S0 + k]);
-            acc[S0 + k] = __builtin_fmaf(eo, po, acc[S0 + k]);
-            pn *= pn;
-            po *= po;
-        }
-    }
-}
-
 // One eta group of angular functions as the move update reads it: e^{-eta x}
-// = 2^{-eta2 x}; slots (lambda, k) = (+1, 0..4), (-1, 0..4); kp / km the
-// largest k per lambda (-1: none); per slot tpz and the row (-1: none).
+// = 2^{-eta2 x}; slots (lambda, k) = (+1, 0..4), (-1, 0..4); per slot tpz and
+// the row (-1: none).
 struct NnpGroup {
     float eta2;
-    int row0, kp, km;
+    int row0;
+    int top[2];  // per lambda: 1 + the highest power with a function (0: none)
     int rk[NNP_GMAX];
     float tpz[NNP_GMAX];
     __device__ void none()
     {
         eta2 = 0.0f;
-        row0 = 0;
-        kp = km = -1;
+        row0 = top[0] = top[1] = 0;
 #pragma unroll
         for (int q = 0; q < NNP_GMAX; ++q) {
             rk[q] = -1;
@@ -188,39 +157,87 @@ __device__ __forceinline__ void nnp_group(const int32_t *gd, int g, NnpGroup &G)
     }
     G.eta2 = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(dw[0]));
     G.row0 = __builtin_amdgcn_readfirstlane(dw[1]);
-    G.kp = __builtin_amdgcn_readfirstlane(dw[2]);
-    G.km = __builtin_amdgcn_readfirstlane(dw[3]);
+    G.top[0] = G.top[1] = 0;
 #pragma unroll
     for (int q = 0; q < NNP_GMAX; ++q) {
         G.tpz[q] = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(dw[4 + q]));
         G.rk[q] = __builtin_amdgcn_readfirstlane(dw[4 + NNP_GMAX + q]);
+        if (G.rk[q] >= 0) G.top[q / NNP_KSLOT] = q % NNP_KSLOT + 1;
     }
 }
 
-// One visit (j, k) for one group: the terms centred on j into aj and, for
-// own visits, those centred on i into ai (per slot, tpz applied at the store).
-__device__ __forceinline__ void nnp_visit(const NnpGroup &G, float rsn, float rso, float fpn, float fpo, float cjn,
-                                          float cjo, float cin, float cio, bool own, float *aj, float *ai)
+// Terms of one visit centred on one atom, both groups of the wave: e_new
+// (1 + lambda c_new)^(2^k) + e_old (1 + lambda c_old)^(2^k) into slot (lambda,
+// k) of a0 (a1), one squaring chain per lambda for both groups (eo carries the
+// sign of the old term).  Every slot up to the highest power is added to: one
+// without a function is never read, and a test per slot costs more than its
+// two fma (a select each, its mask in a spilled scalar pair).
+template <bool TWO>
+__device__ __forceinline__ void nnp_terms(int top_p, int top_m, float cn, float co, float en0, float eo0, float en1,
+                                          float eo1, float *a0, float *a1)
 {
-    const float en = __builtin_amdgcn_exp2f(-G.eta2 * rsn) * fpn;
-    const float eo = -(__builtin_amdgcn_exp2f(-G.eta2 * rso) * fpo);
-    nnp_chain<0>(G.kp, 1.0f, cjn, cjo, en, eo, aj);
-    nnp_chain<NNP_KSLOT>(G.km, -1.0f, cjn, cjo, en, eo, aj);
-    if (own) {
-        nnp_chain<0>(G.kp, 1.0f, cin, cio, en, eo, ai);
-        nnp_chain<NNP_KSLOT>(G.km, -1.0f, cin, cio, en, eo, ai);
+#pragma unroll
+    for (int v = 0; v < 2; ++v) {
+        const int top = v ? top_m : top_p;
+        float pn = v ? 1.0f - cn : 1.0f + cn, po = v ? 1.0f - co : 1.0f + co;
+#pragma unroll
+        for (int k = 0; k < NNP_KSLOT; ++k) {
+            if (k >= top) break;
+            if (k > 0) {
+                pn *= pn;
+                po *= po;
+            }
+            const int q = v * NNP_KSLOT + k;
+            a0[q] = __builtin_fmaf(en0, pn, a0[q]);
+            a0[q] = __builtin_fmaf(eo0, po, a0[q]);
+            if (TWO) {
+                a1[q] = __builtin_fmaf(en1, pn, a1[q]);
+                a1[q] = __builtin_fmaf(eo1, po, a1[q]);
+            }
+        }
     }
 }
 
-// Stores of one group: the 2^lp lanes of a target (an aligned block)
-// combine their parts by quad exchanges and the half-row mirror, the first
-// writes the target's entry; the wave's sum of the terms centred on i goes
-// to the moved atom's column (added to the earlier chunks' sum when the
-// targets come in several chunks of 64).  All lanes call.
+// m without its n lowest set bits (n up to their number): the position by
+// halving over the bit counts
+__device__ __forceinline__ uint64_t nnp_drop(uint64_t m, int n)
+{
+    int p = 0;
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) {
+        const int c = __popcll((m >> p) & ((1ull << s) - 1ull));
+        const bool up = n >= c;
+        n = up ? n - c : n;
+        p = up ? p + s : p;
+    }
+    m = (m >> p) << p;
+    return n > 0 ? m & (m - 1ull) : m;
+}
+
+// Adds one group's changes to the trial features D (which start as the
+// current ones).  The 2^lp lanes of a target (an aligned block) combine their
+// parts by quad exchanges and the half-row mirror, the first writes the
+// target's entry.  The wave's sums of the terms centred on i go to the moved
+// atom's column: the two row swaps merge the ten slots' registers into three
+// (lambda by lane bit 5, the power's low bit by bit 4), so three row sums do
+// for ten and one lane per slot writes.  Every old value is read before the
+// first is written: the reads are in flight together.  All lanes call.
+static_assert(NNP_KSLOT == 5, "slots (k, k + 1) of each lambda in three registers");
 template <int NP>
-__device__ __forceinline__ void nnp_store(const NnpGroup &G, int lp, bool writer, int j, int i, int lane, float *Dp,
-                                          float *aj, float *ai, bool first)
+__device__ __forceinline__ void nnp_store(const NnpGroup &G, const int32_t *gd, int lp, bool writer, int j, int i,
+                                          int lane, float *Dp, const float *aj, const float *ai)
 {
+    // the slot whose sum this lane writes
+    const int kq = 2 * (lane & 3) + ((lane >> 4) & 1), qi = NNP_KSLOT * (lane >> 5) + kq;
+    const bool iw = (lane & 15) < 3 && kq < NNP_KSLOT;
+    const int qc = iw ? qi : 0;
+    const int irk = gd[4 + NNP_GMAX + qc];
+    const float itpz = __int_as_float(gd[4 + qc]);
+    float old[NNP_GMAX];
+#pragma unroll
+    for (int q = 0; q < NNP_GMAX; ++q) old[q] = Dp[(G.row0 + (G.rk[q] < 0 ? 0 : G.rk[q])) * NP + j];
+    float *di = Dp + (G.row0 + (irk < 0 ? 0 : irk)) * NP + i;
+    const float oldi = *di;
 #pragma unroll
     for (int q = 0; q < NNP_GMAX; ++q) {
         if (G.rk[q] >= 0) {
@@ -231,12 +248,17 @@ __device__ __forceinline__ void nnp_store(const NnpGroup &G, int lp, bool writer
             v = lp >= 2 ? v + t2 : v;
             const float t3 = dpp_f<0x141>(v);
             v = lp >= 3 ? v + t3 : v;
-            float *Dr = Dp + (G.row0 + G.rk[q]) * NP;
-            if (writer) Dr[j] = v * G.tpz[q];
-            const float vi = wave_sum_last(ai[q]);
-            if (lane == 63) Dr[i] = first ? vi * G.tpz[q] : Dr[i] + vi * G.tpz[q];
+            if (writer) Dp[(G.row0 + G.rk[q]) * NP + j] = __builtin_fmaf(v, G.tpz[q], old[q]);
         }
     }
+    float h[NNP_KSLOT];
+#pragma unroll
+    for (int k = 0; k < NNP_KSLOT; ++k) h[k] = row_merge<32>(ai[k], ai[NNP_KSLOT + k]);
+    const float s0 = row_sum16(row_merge<16>(h[0], h[1]));
+    const float s1 = row_sum16(row_merge<16>(h[2], h[3]));
+    const float s2 = row_sum16(row_pair_sum<16>(h[4]));
+    const float s = (lane & 3) == 0 ? s0 : ((lane & 3) == 1 ? s1 : s2);
+    if (iw && irk >= 0) *di = __builtin_fmaf(s, itpz, oldi);
 }
 
 // Full feature matrix from positions into Gout (total_symm_calc,
@@ -315,25 +337,58 @@ __device__ void nnp_full_build(const NnpTables &T, const NnpLds &L, float *Gout,
     __syncthreads();
 }
 
-typedef float nnp_f32x16 __attribute__((ext_vector_type(16)));
+typedef float nnp_f32x4 __attribute__((ext_vector_type(4)));
 
-// tanh x = 1 - 2 / (1 + e^{2x}), e^{2x} = 2^{2 log2(e) x}: absolute error below
-// about 4e-7 over the whole range (the limits +-1 come out exactly)
+// tanh x = 1 - 2 / (1 + e^{2x}), e^{2x} = 2^{2 log2(e) x} with the rounding
+// of the argument put back (e^d = 1 + d) and the reciprocal refined by one
+// Newton step: absolute error below 1.5e-7 over the whole range.  Past |x| =
+// 40 the value is +-1 in binary32 at any rate; the clamp keeps e finite there.
 __device__ __forceinline__ float nnp_tanh(float x)
 {
-    const float e = __builtin_amdgcn_exp2f(x * 2.8853900817779268f);
-    return __builtin_fmaf(-2.0f, __builtin_amdgcn_rcpf(1.0f + e), 1.0f);
+    const float c = 2.8853900817779268f, x1 = x > 40.0f ? 40.0f : (x < -40.0f ? -40.0f : x);
+    const float t = x1 * c, d = __builtin_fmaf(x1, c, -t) * 0.6931471805599453f;
+    float e = __builtin_amdgcn_exp2f(t);
+    e = __builtin_fmaf(e, d, e) + 1.0f;
+    const float y = __builtin_amdgcn_rcpf(e);
+    return __builtin_fmaf(-2.0f, __builtin_fmaf(__builtin_fmaf(-e, y, 1.0f), y, y), 1.0f);
+}
+
+// One 16 x 16 tile (atoms r0 .., outputs c0 ..) of a layer's product over n
+// inputs, binary32 on the matrix cores: lane l feeds A[row l % 16][k l / 16]
+// from x(k, row) and B[k l / 16][column l % 16] from w(k, column); value v of
+// the result belongs to row 4 (l / 16) + v, column l % 16.  Four partial sums:
+// independent steps, and a quarter of the terms in each rounding chain.
+template <typename X, typename W>
+__device__ __forceinline__ nnp_f32x4 nnp_tile(int n, X x, W w)
+{
+    const int lk = (threadIdx.x & 63) >> 4;
+    nnp_f32x4 z[4] = {};
+    int k0 = 0;
+    for (; k0 + 16 <= n; k0 += 16) {
+        float a[4], b[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            a[u] = x(k0 + 4 * u + lk);
+            b[u] = w(k0 + 4 * u + lk);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) z[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u], b[u], z[u], 0, 0, 0);
+    }
+    for (; k0 < n; k0 += 4) {
+        const int k = k0 + lk, kc = k < n ? k : n - 1;
+        const float m = k < n ? 1.0f : 0.0f;
+        z[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(x(kc) * m, w(kc) * m, z[3], 0, 0, 0);
+    }
+    return (z[0] + z[1]) + (z[2] + z[3]);
 }
 
 // Per-atom network energies of the features Gin into out[N]
 // (n_features -> tanh h1 -> tanh h2 -> linear 1, ForwardPass.jl:23-39).
-// The two hidden layers are NP x 32 products on the matrix cores in binary32
-// (v_mfma_f32_32x32x2_f32; wave w takes atoms 32w to 32w + 31, two
-// accumulators over alternating k pairs); lane layout: A[row l%32][k l/32],
-// B[k l/32][col l%32], output value v of lane l at row 8(v/4) + 4(l/32) + v%4,
-// column l%32.  The output layer is one dot product per atom; the FP64 total
-// is a butterfly over each wave of 64 atoms, then the waves' sums in order.
-// All threads call.
+// The two hidden layers are products on the matrix cores in binary32, a 16 x 16
+// tile per wave (64 atoms x 32 outputs are eight tiles; two waves with 32 x 32
+// tiles left the other six waiting for 44 steps of 64 cycles).  The
+// output layer's dot product is a row sum per tile; the FP64 total is a sum
+// over each wave of 64 atoms (DPP and row swaps), then the waves' sums in order.  All threads call.
 template <int NP>
 __device__ void nnp_forward(const NnpTables &T, const NnpLds &L, const float *Gin, int N, float *out,
                             double *total = nullptr)
@@ -342,54 +397,38 @@ __device__ void nnp_forward(const NnpTables &T, const NnpLds &L, const float *Gi
     __shared__ double s_fpart[NNP_NP_WIDE / 64];
     const int tid = threadIdx.x, l = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lr = l & 31, lh = l >> 5;
+    const int lr = l & 15, lk = l >> 4;
     const int nf = T.nf, h1 = T.h1, h2 = T.h2;
-    if (w < NP / 32) {
-        const int r0 = 32 * w;
-        const int c1 = lr < h1 ? lr : 0;
-        const float m1 = lr < h1 ? 1.0f : 0.0f;
-        nnp_f32x16 za = {}, zb = {};
-        for (int kk = 0; kk < nf; kk += 4) {
-            const int ka = kk + lh, kb = kk + 2 + lh;
-            const int kac = ka < nf ? ka : nf - 1, kbc = kb < nf ? kb : nf - 1;
-            const float ma = ka < nf ? 1.0f : 0.0f, mb = kb < nf ? 1.0f : 0.0f;
-            const float xa = Gin[kac * NP + r0 + lr] * ma, xb = Gin[kbc * NP + r0 + lr] * mb;
-            const float wa = L.W1[kac * h1 + c1] * m1, wb = L.W1[kbc * h1 + c1] * m1;
-            za = __builtin_amdgcn_mfma_f32_32x32x2f32(xa, wa, za, 0, 0, 0);
-            zb = __builtin_amdgcn_mfma_f32_32x32x2f32(xb, wb, zb, 0, 0, 0);
-        }
-        if (lr < h1) {
-            const float bias = L.B[lr];
+    for (int t = w; t < 2 * (NP / 16); t += NNP_NT / 64) {
+        const int r0 = 16 * (t % (NP / 16)), c0 = 16 * (t / (NP / 16));
+        if (r0 >= N || c0 >= h1) continue;
+        const int c = c0 + lr, cc = c < h1 ? c : h1 - 1;
+        const nnp_f32x4 z = nnp_tile(nf, [&](int k) { return Gin[k * NP + r0 + lr]; },
+                                     [&](int k) { return L.W1[k * h1 + cc]; });
+        if (c < h1) {
+            const float bias = L.B[c];
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int row = r0 + 8 * (v >> 2) + 4 * lh + (v & 3);
-                L.H1[row * NNP_HS + lr] = nnp_tanh(za[v] + zb[v] + bias);
-            }
+            for (int v = 0; v < 4; ++v) L.H1[(r0 + 4 * lk + v) * NNP_HS + c] = nnp_tanh(z[v] + bias);
         }
     }
     __syncthreads();
-    if (w < NP / 32) {
-        const int r0 = 32 * w;
-        const int c2 = lr < h2 ? lr : 0;
-        const float m2 = lr < h2 ? 1.0f : 0.0f;
-        nnp_f32x16 za = {}, zb = {};
-        for (int kk = 0; kk < h1; kk += 4) {
-            const int ka = kk + lh, kb = kk + 2 + lh;
-            const int kac = ka < h1 ? ka : h1 - 1, kbc = kb < h1 ? kb : h1 - 1;
-            const float ma = ka < h1 ? 1.0f : 0.0f, mb = kb < h1 ? 1.0f : 0.0f;
-            const float xa = L.H1[(r0 + lr) * NNP_HS + kac] * ma, xb = L.H1[(r0 + lr) * NNP_HS + kbc] * mb;
-            const float wa = L.W2[kac * h2 + c2] * m2, wb = L.W2[kbc * h2 + c2] * m2;
-            za = __builtin_amdgcn_mfma_f32_32x32x2f32(xa, wa, za, 0, 0, 0);
-            zb = __builtin_amdgcn_mfma_f32_32x32x2f32(xb, wb, zb, 0, 0, 0);
+    for (int t = w; t < 2 * (NP / 16); t += NNP_NT / 64) {
+        const int r0 = 16 * (t % (NP / 16)), c0 = 16 * (t / (NP / 16));
+        if (r0 >= N || c0 >= h2) continue;
+        const int c = c0 + lr, cc = c < h2 ? c : h2 - 1;
+        const nnp_f32x4 z = nnp_tile(h1, [&](int k) { return L.H1[(r0 + lr) * NNP_HS + k]; },
+                                     [&](int k) { return L.W2[k * h2 + cc]; });
+        float bias = 0.0f, w3 = 0.0f;
+        if (c < h2) {
+            bias = L.B[NNP_MAXH + c];
+            w3 = L.B[2 * NNP_MAXH + c];
         }
-        if (lr < h2) {
-            // second hidden layer times the output weights
-            const float bias = L.B[NNP_MAXH + lr], w3 = L.B[2 * NNP_MAXH + lr];
+        // second hidden layer times the output weights, summed over the tile's
+        // columns (w3 = 0 past the last)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int row = r0 + 8 * (v >> 2) + 4 * lh + (v & 3);
-                L.H2[row * NNP_HS + lr] = nnp_tanh(za[v] + zb[v] + bias) * w3;
-            }
+        for (int v = 0; v < 4; ++v) {
+            const float y = row_sum16(nnp_tanh(z[v] + bias) * w3);
+            if (lr == 0) L.H2[(c0 >> 4) * NP + r0 + 4 * lk + v] = y;
         }
     }
     __syncthreads();
@@ -397,15 +436,17 @@ __device__ void nnp_forward(const NnpTables &T, const NnpLds &L, const float *Gi
         const int at = 64 * w + l;
         float y = 0.0f;
         if (at < N) {
-            for (int k = 0; k < h2; ++k) y += L.H2[at * NNP_HS + k];
+            y = L.H2[at];
+            if (h2 > 16) y += L.H2[NP + at];
             y += T.b3;
             out[at] = y;
         }
-        // FP64 total of the atomic energies (a butterfly over the wave)
+        // FP64 total of the atomic energies
         if (total != nullptr) {
             double t = at < N ? (double)y : 0.0;
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
+            t = group_sum<16>(t);
+            t += row_xor<16>(t);
+            t += row_xor<32>(t);
             if (NW == 1 && l == 0) *total = t;
             if (NW > 1 && l == 0) s_fpart[w] = t;
         }
@@ -478,6 +519,17 @@ __global__ void __launch_bounds__(NNP_NT) nnp_init_kernel(SweepArgs a)
 // slot, 64 (two workgroups per CU) or 128 (one; the near atoms of a move are
 // then up to 127, their partner masks two words, and the angular targets are
 // taken in chunks of 64 lanes).
+//
+// Bound by instruction issue in the angular visits (a 55-atom move visits about
+// 1000 triangles from two of their atoms, once per wave): 28,000 of a move's
+// 51,000 cycles with one workgroup on a CU.  A visit's instructions went from
+// about 330 to 190: the lane's share of the partners is cut from the mask once
+// per target (not popped past on every visit), cosines from unit vectors in
+// place of IEEE divides and roots, one squaring chain for both groups of a
+// wave, no select per slot.  Store: sums merged across rows before they are
+// summed, 20 wave sums as 6 row sums.  Cycle of 40 temperatures x 55 atoms
+// (8 + 80 functions) 2.07 ms -> 1.21, of 1280 configurations 6.9 -> 4.0, of 20 x
+// 78 atoms 3.0 -> 1.97.
 template <bool DA, int NP>
 __global__ void __launch_bounds__(NNP_NT) __attribute__((amdgpu_waves_per_eu((DA || NP > NNP_NP) ? 2 : 4)))
 nnp_sweep_kernel(SweepArgs a)
@@ -548,9 +600,21 @@ nnp_sweep_kernel(SweepArgs a)
     // current features and the scratch that becomes the trial features; an
     // accepted move swaps the two (swap_vars!(NNPVariables), src/swap_config.jl:213-221)
     float *Gp = L.G, *Dp = L.D;
-    float4 *nb_a = reinterpret_cast<float4 *>((reinterpret_cast<uintptr_t>(L.H2) + 15) & ~(uintptr_t)15);
-    float4 *nb_b = nb_a + NP;
-    float *nb_fo = reinterpret_cast<float *>(nb_b + NP);
+    // 16-byte aligned by its offset, so that the compiler still sees an LDS
+    // address (a pointer through an integer is read with flat loads)
+    float *nb_base = reinterpret_cast<float *>(lds_raw) + (((int)(L.H2 - reinterpret_cast<float *>(lds_raw)) + 3) & ~3);
+    float4 *nb_a = reinterpret_cast<float4 *>(nb_base);
+    float4 *nb_b = nb_a + NP, *nb_u = nb_b + NP, *nb_v = nb_u + NP;
+    // near atom q of the list (atom j): {x, y, z, f_new}, {r2_new, r2_old,
+    // f_old, -} and the unit vectors from the moved atom's new and old position
+    auto pack = [&](int q, int j, const float (&pt)[3], const float (&po)[3]) {
+        const float x = L.X[j], y = L.X[NP + j], z = L.X[2 * NP + j], rn = L.rn2[j], ro = L.ro2[j];
+        const float un = nnp_rsq(rn), uo = nnp_rsq(ro);
+        nb_a[q] = make_float4(x, y, z, L.fn[j]);
+        nb_b[q] = make_float4(rn, ro, L.fo[j], 0.0f);
+        nb_u[q] = make_float4((x - pt[0]) * un, (y - pt[1]) * un, (z - pt[2]) * un, 0.0f);
+        nb_v[q] = make_float4((x - po[0]) * uo, (y - po[1]) * uo, (z - po[2]) * uo, 0.0f);
+    };
 
     for (uint32_t m = 0; m < nsteps; ++m) {
         // draws and trial position (every thread the same), src/MCMoves.jl:115-135
@@ -621,13 +685,10 @@ nnp_sweep_kernel(SweepArgs a)
             const uint64_t b = __ballot(near);
             if constexpr (NW == 1) {
                 if (near) {
-                    // packed per near atom for the angular visits (in the H2 scratch):
-                    // {x, y, z, f_new}, {r2_new, r2_old, r_new, r_old}, f_old
+                    // packed per near atom for the angular visits (in the H2 scratch)
                     const int q = mbcnt64(b);
                     s_near[q] = (uint8_t)j;
-                    nb_a[q] = make_float4(L.X[j], L.X[NP + j], L.X[2 * NP + j], L.fn[j]);
-                    nb_b[q] = make_float4(L.rn2[j], L.ro2[j], sqrtf(L.rn2[j]), sqrtf(L.ro2[j]));
-                    nb_fo[q] = L.fo[j];
+                    pack(q, j, pt, po);
                 }
                 if (lane == 0) s_nnear = __popcll(b);
             } else {
@@ -645,9 +706,7 @@ nnp_sweep_kernel(SweepArgs a)
                     int q = mbcnt64(b);
                     for (int v = 0; v < (tid >> 6); ++v) q += __popcll(s_wmask[v]);
                     s_near[q] = (uint8_t)j;
-                    nb_a[q] = make_float4(L.X[j], L.X[NP + j], L.X[2 * NP + j], L.fn[j]);
-                    nb_b[q] = make_float4(L.rn2[j], L.ro2[j], sqrtf(L.rn2[j]), sqrtf(L.ro2[j]));
-                    nb_fo[q] = L.fo[j];
+                    pack(q, j, pt, po);
                 }
             }
             if (tid == 0) {
@@ -656,7 +715,10 @@ nnp_sweep_kernel(SweepArgs a)
                 s_nnear = t;
             }
         }
-        for (int e = tid; e < T.nf * NP; e += NNP_NT) Dp[e] = 0.0f;
+        // trial features start as the current ones; every changed entry is
+        // written once, as current plus change
+        for (int e = tid; e < T.nf * NP / 4; e += NNP_NT)
+            reinterpret_cast<float4 *>(Dp)[e] = reinterpret_cast<const float4 *>(Gp)[e];
         if (da && tid < SUR_K) s_acci[tid] = 0.0f;
         __syncthreads();
         // delayed acceptance, stage 1: Metropolis on the surrogate energy change
@@ -699,12 +761,7 @@ nnp_sweep_kernel(SweepArgs a)
         if (stage1 && !s_flag) {
             if constexpr (DA) {
                 // the surrogate's layer scratch covered the packed near-atom data
-                if (tid < s_nnear) {
-                    const int j = s_near[tid];
-                    nb_a[tid] = make_float4(L.X[j], L.X[NP + j], L.X[2 * NP + j], L.fn[j]);
-                    nb_b[tid] = make_float4(L.rn2[j], L.ro2[j], sqrtf(L.rn2[j]), sqrtf(L.ro2[j]));
-                    nb_fo[tid] = L.fo[j];
-                }
+                if (tid < s_nnear) pack(tid, s_near[tid], pt, po);
                 __syncthreads();
             }
             // radial changes, DeltaMatrix.jl:794-822: one wave per function,
@@ -719,11 +776,11 @@ nnp_sweep_kernel(SweepArgs a)
                     float d = 0.0f;
                     if (at < N && at != i)
                         d = expf(-eta * L.rn2[at]) * (L.fn[at] * norm) + expf(-eta * L.ro2[at]) * (-L.fo[at] * norm);
-                    if (at < N && at != i) Dp[row * NP + at] = d;
+                    if (at < N && at != i) Dp[row * NP + at] = Gp[row * NP + at] + d;
                     dsum += d;
                 }
                 const float s = wave_sum(dsum);
-                if (lane == 0) Dp[row * NP + i] = s;
+                if (lane == 0) Dp[row * NP + i] = Gp[row * NP + i] + s;
             }
             // angular changes, DeltaMatrix.jl:827-872.  Every partner pair
             // (j, k) of the moved atom i whose triangle lies inside the cut-off
@@ -740,14 +797,14 @@ nnp_sweep_kernel(SweepArgs a)
             const float rc2 = T.r_cut * T.r_cut * 1.0001f;  // loose: the cut-off function decides below
             for (int a = tid >> 6; a < n_near; a += NNP_NT / 64) {
                 const float4 pa = nb_a[a];
-                const float foa = nb_fo[a];
+                const float foa = nb_b[a].z;
 #pragma unroll
                 for (int v = 0; v < NW; ++v) {
                     const int b = 64 * v + lane;
                     bool act = false;
                     if (b < n_near && b != a) {
                         const float4 pb = nb_a[b];
-                        if (pa.w * pb.w != 0.0f || foa * nb_fo[b] != 0.0f) {
+                        if (pa.w * pb.w != 0.0f || foa * nb_b[b].z != 0.0f) {
                             const float dx = pa.x - pb.x, dy = pa.y - pb.y, dz = pa.z - pb.z;
                             act = dx * dx + dy * dy + dz * dz < rc2;
                         }
@@ -778,21 +835,19 @@ nnp_sweep_kernel(SweepArgs a)
 #pragma unroll
                     for (int v = 0; v < NW; ++v) La += __popcll(s_mask[(64 * c + lane) * NW + v]);
                 }
+                // lanes of a target at load T: 1 up to T visits, 2 up to 2 T,
+                // 4 up to 4 T, else 8; their sum over the targets
                 auto lanes_for = [&](int load) {
-                    if (lane >= nc) return 0;
-                    const int q = (La + load - 1) / load;
-                    return q <= 1 ? 1 : (q <= 2 ? 2 : (q <= 4 ? 4 : 8));
+                    return lane >= nc ? 0 : (La <= load ? 1 : (La <= 2 * load ? 2 : (La <= 4 * load ? 4 : 8)));
                 };
-                auto lanes_used = [&](int pa) {
-                    int t = 0;
-#pragma unroll
-                    for (int cc = 0; cc < 4; ++cc) t += __popcll(__ballot(pa == (1 << cc))) << cc;
-                    return t;
+                auto lanes_used = [&](int load) {
+                    return nc + __popcll(__ballot(La > load)) + 2 * __popcll(__ballot(La > 2 * load)) +
+                           4 * __popcll(__ballot(La > 4 * load));
                 };
                 int lo = 1, hi = 64 * NW;
                 while (lo < hi) {
                     const int mid = (lo + hi) >> 1;
-                    if (lanes_used(lanes_for(mid)) <= 64) hi = mid;
+                    if (lanes_used(mid) <= 64) hi = mid;
                     else lo = mid + 1;
                 }
                 const int Pa = lanes_for(lo);
@@ -808,21 +863,19 @@ nnp_sweep_kernel(SweepArgs a)
                 }
                 used_c[c] = used;
             }
-            // this lane's target in chunk c: lanes, part, atom, partner masks
-            // (and those of larger list index, the visits that also carry the
+            // this lane's target in chunk c: lanes, part, atom, the partners of
+            // its part (and those of larger list index, the visits that also carry the
             // terms centred on i), packed data
             struct Target {
-                int lp, P, part, j;
+                int lp, part, j;
                 bool tact;
                 uint64_t m0, m1, after0, after1;
-                float4 ja, jb;
-                float jfo;
+                float4 ja, jb, ju, jv;
             };
             auto target = [&](int c) {
                 Target g;
                 const int ent = lane < used_c[c] ? (int)s_lt[64 * c + lane] : 0;
                 g.lp = ent >> 9;
-                g.P = 1 << g.lp;
                 const int ta = 64 * c + (ent & 63);
                 g.part = (ent >> 6) & 7;
                 g.tact = lane < used_c[c];
@@ -836,82 +889,100 @@ nnp_sweep_kernel(SweepArgs a)
                     const int sh = ta - 64;
                     g.after1 = sh < 0 ? ~0ull : (sh < 63 ? ~((2ull << sh) - 1ull) : 0ull);
                 }
+                // the part's share: equal counts, by rank among the partners
+                const int n0 = __popcll(g.m0), n = n0 + (NW > 1 ? __popcll(g.m1) : 0);
+                const int r0 = (g.part * n) >> g.lp, r1 = ((g.part + 1) * n) >> g.lp;
+                auto cut_word = [](uint64_t m, int c, int a, int b) {  // bits of rank a .. b - 1 of c
+                    a = a < 0 ? 0 : (a < c ? a : c);
+                    b = b < 0 ? 0 : (b < c ? b : c);
+                    return nnp_drop(m, a) & ~nnp_drop(m, b);
+                };
+                if constexpr (NW > 1) g.m1 = cut_word(g.m1, n - n0, r0 - n0, r1 - n0);
+                g.m0 = cut_word(g.m0, n0, r0, r1);
                 g.ja = nb_a[ta];
                 g.jb = nb_b[ta];
-                g.jfo = nb_fo[ta];
+                g.ju = nb_u[ta];
+                g.jv = nb_v[ta];
                 return g;
             };
             Target t1{};
             if constexpr (NW == 1) t1 = target(0);  // one chunk: read once for all group passes
-            const int w = tid >> 6;
-            const int ngw = L.wg[w * (NNP_WG + 1)];
+            // uniform over the wave, and said so: the functions' masks then
+            // branch instead of selecting every accumulator
+            const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+            const int ngw = __builtin_amdgcn_readfirstlane(L.wg[w * (NNP_WG + 1)]);
             for (int gi = 0; gi < ngw; gi += 2) {
                 // up to two groups per pass over the visits
-                const int ga = L.wg[w * (NNP_WG + 1) + 1 + gi];
-                const int gb = gi + 1 < ngw ? L.wg[w * (NNP_WG + 1) + 2 + gi] : -1;
+                const int ga = __builtin_amdgcn_readfirstlane(L.wg[w * (NNP_WG + 1) + 1 + gi]);
+                const int gb = gi + 1 < ngw ? __builtin_amdgcn_readfirstlane(L.wg[w * (NNP_WG + 1) + 2 + gi]) : -1;
                 NnpGroup G0, G1;
                 nnp_group(L.gd, ga, G0);
                 if (gb >= 0) nnp_group(L.gd, gb, G1);
                 else G1.none();
+                const int top_p = G0.top[0] > G1.top[0] ? G0.top[0] : G1.top[0];
+                const int top_m = G0.top[1] > G1.top[1] ? G0.top[1] : G1.top[1];
 #pragma unroll
                 for (int c = 0; c < NW; ++c) {
                     if (c >= nch) continue;
                     const Target tg = NW == 1 ? t1 : target(c);
-                    const int lp = tg.lp, P = tg.P, part = tg.part, j = tg.j;
-                    const bool tact = tg.tact;
-                    uint64_t m0 = tg.m0, m1 = tg.m1;
-                    const uint64_t after0 = tg.after0, after1 = tg.after1;
-                    const float4 ja = tg.ja, jb = tg.jb;
-                    const float jfo = tg.jfo;
-                    const float pj3[3] = {ja.x, ja.y, ja.z};
-                    const float dijn = jb.z, dijo = jb.w;
+                    const float4 ja = tg.ja, jb = tg.jb, ju = tg.ju, jv = tg.jv;
                     float aj0[NNP_GMAX], ai0[NNP_GMAX], aj1[NNP_GMAX], ai1[NNP_GMAX];
 #pragma unroll
                     for (int q = 0; q < NNP_GMAX; ++q) aj0[q] = ai0[q] = aj1[q] = ai1[q] = 0.0f;
-                    auto pop = [&]() {  // drop the lowest partner
-                        if constexpr (NW == 1) {
-                            m0 &= m0 - 1ull;
-                        } else {
-                            if (m0 != 0ull) m0 &= m0 - 1ull;
-                            else m1 &= m1 - 1ull;
+                    auto visits = [&](auto two) {
+                        constexpr bool TWO = decltype(two)::value;
+                        uint64_t m0 = tg.m0, m1 = tg.m1;
+                        while (NW == 1 ? m0 != 0ull : (m0 | m1) != 0ull) {
+                            int bk;
+                            bool own;
+                            if (NW == 1 || m0 != 0ull) {
+                                bk = __builtin_ctzll(m0);
+                                m0 &= m0 - 1ull;
+                                own = ((tg.after0 >> bk) & 1ull) != 0ull;
+                            } else {
+                                bk = __builtin_ctzll(m1);
+                                m1 &= m1 - 1ull;
+                                own = ((tg.after1 >> bk) & 1ull) != 0ull;
+                                bk += 64;
+                            }
+                            const float4 ka = nb_a[bk], kb = nb_b[bk];
+                            const float dx = ja.x - ka.x, dy = ja.y - ka.y, dz = ja.z - ka.z;
+                            const float rjk = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
+                            const float ijk = nnp_rsq(rjk);
+                            const float fjk = nnp_cutoff(rjk * ijk, T.r_cut);
+                            const float fpn = ja.w * ka.w * fjk, fpo = jb.z * kb.z * fjk;
+                            if (fpn == 0.0f && fpo == 0.0f) continue;
+                            const float rsn = jb.x + kb.x + rjk, rso = jb.y + kb.y + rjk;
+                            // cosines at j, new and old, from the unit vectors i -> j and k -> j
+                            const float cjn = __builtin_fmaf(ju.z, dz, __builtin_fmaf(ju.y, dy, ju.x * dx)) * ijk;
+                            const float cjo = __builtin_fmaf(jv.z, dz, __builtin_fmaf(jv.y, dy, jv.x * dx)) * ijk;
+                            const float en0 = __builtin_amdgcn_exp2f(-G0.eta2 * rsn) * fpn;
+                            const float eo0 = -(__builtin_amdgcn_exp2f(-G0.eta2 * rso) * fpo);
+                            float en1 = 0.0f, eo1 = 0.0f;
+                            if (TWO) {
+                                en1 = __builtin_amdgcn_exp2f(-G1.eta2 * rsn) * fpn;
+                                eo1 = -(__builtin_amdgcn_exp2f(-G1.eta2 * rso) * fpo);
+                            }
+                            nnp_terms<TWO>(top_p, top_m, cjn, cjo, en0, eo0, en1, eo1, aj0, aj1);
+                            if (own) {
+                                // and at i
+                                const float4 ku = nb_u[bk], kv = nb_v[bk];
+                                const float cin = __builtin_fmaf(ju.z, ku.z, __builtin_fmaf(ju.y, ku.y, ju.x * ku.x));
+                                const float cio = __builtin_fmaf(jv.z, kv.z, __builtin_fmaf(jv.y, kv.y, jv.x * kv.x));
+                                nnp_terms<TWO>(top_p, top_m, cin, cio, en0, eo0, en1, eo1, ai0, ai1);
+                            }
                         }
                     };
-                    for (int t = 0; t < part; ++t) pop();  // this lane's first partner
-                    while (NW == 1 ? m0 != 0ull : (m0 | m1) != 0ull) {
-                        const int bk = (NW == 1 || m0 != 0ull) ? __builtin_ctzll(m0) : 64 + __builtin_ctzll(m1);
-                        for (int t = 0; t < P; ++t) pop();  // next partner of this lane
-                        const bool own = (NW == 1 || bk < 64) ? ((after0 >> bk) & 1ull) != 0ull
-                                                              : ((after1 >> (bk - 64)) & 1ull) != 0ull;
-                        const float4 ka = nb_a[bk], kb = nb_b[bk];
-                        const float kfo = nb_fo[bk];
-                        const float pk3[3] = {ka.x, ka.y, ka.z};
-                        const float dx = pj3[0] - pk3[0], dy = pj3[1] - pk3[1], dz = pj3[2] - pk3[2];
-                        const float rjk = dx * dx + dy * dy + dz * dz;
-                        const float djk = sqrtf(rjk);
-                        const float fjk = nnp_cutoff(djk, T.r_cut);
-                        const float fpn = ja.w * ka.w * fjk, fpo = jfo * kfo * fjk;
-                        if (fpn == 0.0f && fpo == 0.0f) continue;
-                        const float rsn = jb.x + kb.x + rjk, rso = jb.y + kb.y + rjk;
-                        // cosines at j (and at i), new and old
-                        float cjn = 0.0f, cjo = 0.0f, cin = 0.0f, cio = 0.0f;
-                        const float dikn = kb.z, diko = kb.w;
-                        if (fpn != 0.0f) {
-                            cjn = nnp_cos(pj3, pt, pk3, dijn, djk);
-                            if (own) cin = nnp_cos(pt, pj3, pk3, dijn, dikn);
-                        }
-                        if (fpo != 0.0f) {
-                            cjo = nnp_cos(pj3, po, pk3, dijo, djk);
-                            if (own) cio = nnp_cos(po, pj3, pk3, dijo, diko);
-                        }
-                        nnp_visit(G0, rsn, rso, fpn, fpo, cjn, cjo, cin, cio, own, aj0, ai0);
-                        if (gb >= 0) nnp_visit(G1, rsn, rso, fpn, fpo, cjn, cjo, cin, cio, own, aj1, ai1);
+                    const bool writer = tg.tact && tg.part == 0;
+                    if (gb >= 0) {
+                        visits(std::true_type{});
+                        nnp_store<NP>(G1, L.gd + NNP_GD * gb, tg.lp, writer, tg.j, i, lane, Dp, aj1, ai1);
+                    } else {
+                        visits(std::false_type{});
                     }
-                    nnp_store<NP>(G0, lp, tact && part == 0, j, i, lane, Dp, aj0, ai0, c == 0);
-                    if (gb >= 0) nnp_store<NP>(G1, lp, tact && part == 0, j, i, lane, Dp, aj1, ai1, c == 0);
+                    nnp_store<NP>(G0, L.gd + NNP_GD * ga, tg.lp, writer, tg.j, i, lane, Dp, aj0, ai0);
                 }
             }
-            __syncthreads();
-            for (int e = tid; e < T.nf * NP; e += NNP_NT) Dp[e] += Gp[e];
             __syncthreads();
             nnp_forward<NP>(T, L, Dp, N, L.eatn, &s_en);
             new_en = s_en;
