@@ -9,6 +9,7 @@
 #include <cstdio>
 #include <cstring>
 #include <map>
+#include <mutex>
 #include <random>
 #include <string>
 #include <vector>
@@ -96,6 +97,52 @@ struct DevBuf {
     }
 };
 
+// ---- read-back -------------------------------------------------------------
+// A run's state is gathered by one kernel straight into pinned host memory and
+// waited for once.  Bound by latency: a copy of a few kB to pageable memory
+// takes 12 us and a run needed four of them, and one more per workgroup of a
+// ladder spread over workgroups (state() of 44 temperatures x 64 atoms 164 us,
+// of 48 x 256 atoms on 48 workgroups 750; 22 and 90 so).
+
+constexpr int RB_HEAD = 4;       // words before a slot's coordinates: label, energy, box length, height
+constexpr int RB_NT = 256;
+constexpr int RB_ARRAYS = 5;
+constexpr size_t RB_BYTES = (size_t)1 << 20;  // staging of a handle (at least one slot): larger runs are read in pieces
+
+// Words of slots s0 .. s0 + gridDim.x: head, then x, y, z of the n_atoms atoms
+// in FP64.  Atom j of a slot lies at off[slot] + ((j / kl) 3 + c) stride + j %
+// kl (a slot layout of np atoms: kl = stride = np).  Writes run along the
+// buffer, so that they leave the chip as whole lines; the scattered reads hit
+// the caches.
+template <typename T>
+__global__ void __launch_bounds__(RB_NT) state_gather_kernel(const T *coords, const int64_t *off, const int32_t *label,
+                                                             const double *en, const double *box, const double *boxh,
+                                                             int s0, int n_atoms, int kl, int stride, double *out)
+{
+    const int s = s0 + (int)blockIdx.x;
+    double *o = out + (size_t)blockIdx.x * (RB_HEAD + 3 * (size_t)n_atoms);
+    if (threadIdx.x == 0) {
+        o[0] = (double)label[s];
+        o[1] = en[s];
+        o[2] = box[s];
+        o[3] = boxh[s];
+    }
+    for (int e = threadIdx.x; e < 3 * n_atoms; e += RB_NT) {
+        const int j = e / 3, c = e - 3 * j;
+        o[RB_HEAD + e] = (double)coords[off[s] + ((int64_t)(j / kl) * 3 + c) * stride + j % kl];
+    }
+}
+
+// n 8-byte words from each of gridDim.y arrays, one array after the other
+struct WordArrays {
+    const uint64_t *p[RB_ARRAYS];
+};
+__global__ void __launch_bounds__(RB_NT) word_gather_kernel(WordArrays a, int n, uint64_t *out)
+{
+    const int e = (int)(blockIdx.x * RB_NT + threadIdx.x);
+    if (e < n) out[(size_t)blockIdx.y * n + e] = a.p[blockIdx.y][e];
+}
+
 }  // namespace
 
 struct ptmc_engine {
@@ -119,6 +166,12 @@ struct ptmc_engine {
     std::vector<hipEvent_t> ev_pool;  // every timing event created (destroyed with the handle)
     std::vector<hipEvent_t> ev_free;  // those not attached to a pending launch
     std::vector<LaunchTiming> pending;
+
+    // read-back: pinned staging (rb_bytes) and where each slot's coordinates start
+    std::mutex rb_mutex;
+    double *rb = nullptr;
+    size_t rb_bytes = 0;
+    DevBuf<int64_t> d_slot_off;
 
     // plan
     std::vector<TileInfo> tiles;
@@ -1165,6 +1218,9 @@ int ptmc_destroy(ptmc_handle h)
     h->d_runs.free_();
     h->d_run_list.free_();
     h->d_slot_run.free_();
+    h->d_slot_off.free_();
+    if (h->rb) (void)hipHostFree(h->rb);
+    h->rb = nullptr;
     h->d_slot_temp.free_();
     h->d_run_error.free_();
     h->d_slot_en.free_();
@@ -1631,6 +1687,7 @@ int ptmc_prepare(ptmc_handle h)
 
     std::vector<RunInfo> infos;
     std::vector<int32_t> slot_run(h->n_slots), slot_temp(h->n_slots);
+    std::vector<int64_t> slot_off(h->n_slots);
     std::vector<double> slot_en(h->n_slots, 0.0), slot_box(h->n_slots, 1.0), slot_boxh(h->n_slots, 1.0);
     std::vector<double> beta, displ, maxbox, maxboxh, lh, displ_sep;
     const bool pbc = h->cfg.boundary != BC_SPHERE;
@@ -1653,6 +1710,7 @@ int ptmc_prepare(ptmc_handle h)
         for (int t = 0; t < rh.d.n_temps; ++t) {
             slot_run[ri.slot_base + t] = r;
             slot_temp[ri.slot_base + t] = t;
+            if (is_slot(h)) slot_off[ri.slot_base + t] = (int64_t)(ri.slot_base + t) * 3 * slot_np(h);
             const double bl = pbc ? rh.d.box_length : 1.0, bh = has_h ? rh.d.box_height : bl;
             slot_box[ri.slot_base + t] = bl;
             slot_boxh[ri.slot_base + t] = bh;
@@ -1667,6 +1725,10 @@ int ptmc_prepare(ptmc_handle h)
             displ_sep.push_back(rh.d.max_displ_vol);  // max_displ[3] (xy) and [4] (z): the reference default 0.1 each
             displ_sep.push_back(rh.d.max_displ_vol);
         }
+        if (!is_slot(h))
+            for (const Seg &g : rh.segs)
+                for (int k = 0; k < g.count; ++k)
+                    slot_off[ri.slot_base + g.t0 + k] = h->tiles[g.tile].coord_off + (int64_t)(g.local0 + k) * rh.kl;
         tb += rh.d.n_temps;
     }
     h->n_temps = tb;
@@ -1681,6 +1743,14 @@ int ptmc_prepare(ptmc_handle h)
     if ((rc = upload(h, h->d_runs, infos))) return rc;
     if ((rc = upload(h, h->d_slot_run, slot_run))) return rc;
     if ((rc = upload(h, h->d_slot_temp, slot_temp))) return rc;
+    if ((rc = upload(h, h->d_slot_off, slot_off))) return rc;
+    if (!h->rb) {
+        size_t bytes = RB_BYTES;
+        for (const RunHost &rh : h->runs)
+            bytes = std::max(bytes, (RB_HEAD + 3 * (size_t)rh.d.n_atoms) * sizeof(double));
+        HIPCHK(h, hipHostMalloc((void **)&h->rb, bytes, hipHostMallocDefault));
+        h->rb_bytes = bytes;
+    }
     if ((rc = upload(h, h->d_slot_en, slot_en))) return rc;
     if ((rc = upload(h, h->d_slot_box, slot_box))) return rc;
     if ((rc = upload(h, h->d_slot_boxh, slot_boxh))) return rc;
@@ -1960,18 +2030,43 @@ int ptmc_reset_counters(ptmc_handle h)
     return PTMC_OK;
 }
 
+// A run's temperature labels, energies, box lengths and heights by slot, and
+// its coordinates by temperature ([temperature][atom][3]); null: not wanted.  Pieces of whole
+// slots where the run is larger than the staging.
 static int fetch_slots(ptmc_engine *h, int run, std::vector<int32_t> &temp, std::vector<double> &en,
-                       std::vector<double> &box)
+                       std::vector<double> &box, std::vector<double> *boxh = nullptr, double *x = nullptr)
 {
     const RunHost &rh = h->runs[run];
-    const int R = rh.d.n_temps, s0 = rh.info.slot_base;
+    const int R = rh.d.n_temps, N = x ? rh.d.n_atoms : 0;
+    const int kl = is_slot(h) ? slot_np(h) : rh.kl, stride = is_slot(h) ? slot_np(h) : rh.lanes;
+    const bool f32 = is_slot(h) ? slot_f32(h) : h->cfg.precision != 0;
+    const size_t words = RB_HEAD + 3 * (size_t)N;
+    const int piece = (int)std::min<size_t>(R, h->rb_bytes / (words * sizeof(double)));
     temp.resize(R);
     en.resize(R);
     box.resize(R);
-    HIPCHK(h, hipStreamSynchronize(h->stream));
-    HIPCHK(h, hipMemcpy(temp.data(), h->d_slot_temp.p + s0, R * sizeof(int32_t), hipMemcpyDeviceToHost));
-    HIPCHK(h, hipMemcpy(en.data(), h->d_slot_en.p + s0, R * sizeof(double), hipMemcpyDeviceToHost));
-    HIPCHK(h, hipMemcpy(box.data(), h->d_slot_box.p + s0, R * sizeof(double), hipMemcpyDeviceToHost));
+    if (boxh) boxh->resize(R);
+    std::lock_guard<std::mutex> lock(h->rb_mutex);
+    for (int s0 = 0; s0 < R; s0 += piece) {
+        const int ns = std::min(piece, R - s0), first = rh.info.slot_base + s0;
+        if (f32)
+            state_gather_kernel<float><<<ns, RB_NT, 0, h->stream>>>((const float *)h->d_coords.p, h->d_slot_off.p,
+                h->d_slot_temp.p, h->d_slot_en.p, h->d_slot_box.p, h->d_slot_boxh.p, first, N, kl, stride, h->rb);
+        else
+            state_gather_kernel<double><<<ns, RB_NT, 0, h->stream>>>((const double *)h->d_coords.p, h->d_slot_off.p,
+                h->d_slot_temp.p, h->d_slot_en.p, h->d_slot_box.p, h->d_slot_boxh.p, first, N, kl, stride, h->rb);
+        HIPCHK(h, hipGetLastError());
+        HIPCHK(h, hipStreamSynchronize(h->stream));
+        for (int s = s0; s < s0 + ns; ++s) {
+            const double *o = h->rb + (size_t)(s - s0) * words;
+            temp[s] = (int32_t)o[0];
+            en[s] = o[1];
+            box[s] = o[2];
+            if (boxh) (*boxh)[s] = o[3];
+            if (temp[s] < 0 || temp[s] >= R) return fail(h, PTMC_E_DEVICE, "corrupt temperature label");
+            if (x) memcpy(x + (size_t)temp[s] * N * 3, o + RB_HEAD, (size_t)N * 3 * sizeof(double));
+        }
+    }
     return PTMC_OK;
 }
 
@@ -1986,17 +2081,12 @@ int ptmc_get_state(ptmc_handle h, int32_t run, double *x, double *en, double *bo
     if (rc) return rc;
     HIPCHK(h, hipSetDevice(h->cfg.device));
     std::vector<int32_t> temp;
-    std::vector<double> e, b;
-    if ((rc = fetch_slots(h, run, temp, e, b))) return rc;
-    const RunHost &rh = h->runs[run];
-    const int R = rh.d.n_temps, N = rh.d.n_atoms;
+    std::vector<double> e, b, bh;
+    if ((rc = fetch_slots(h, run, temp, e, b, &bh, x))) return rc;
+    const int R = h->runs[run].d.n_temps;
     const bool has_h = h->cfg.boundary == BC_RECT || h->cfg.boundary == BC_RHOMB;
-    std::vector<double> bh(R, 0.0);
-    if (box && has_h)
-        HIPCHK(h, hipMemcpy(bh.data(), h->d_slot_boxh.p + rh.info.slot_base, R * sizeof(double), hipMemcpyDeviceToHost));
     for (int s = 0; s < R; ++s) {
         const int t = temp[s];
-        if (t < 0 || t >= R) return fail(h, PTMC_E_DEVICE, "corrupt temperature label");
         if (en) en[t] = e[s];
         if (box && has_h) {
             box[2 * t] = b[s];
@@ -2005,50 +2095,35 @@ int ptmc_get_state(ptmc_handle h, int32_t run, double *x, double *en, double *bo
             box[t] = b[s];
         }
     }
-    if (x && slot_f32(h)) {
-        const int np = slot_np(h);
-        std::vector<float> blk((size_t)R * 3 * np);
-        HIPCHK(h, hipMemcpy(blk.data(), h->d_coords.p + (size_t)rh.info.slot_base * 3 * np * sizeof(float),
-                            blk.size() * sizeof(float), hipMemcpyDeviceToHost));
-        for (int s = 0; s < R; ++s)
-            for (int j = 0; j < N; ++j)
-                for (int c = 0; c < 3; ++c)
-                    x[((size_t)temp[s] * N + j) * 3 + c] = blk[((size_t)s * 3 + c) * np + j];
-    } else if (x && is_nnp2(h)) {
-        std::vector<double> blk((size_t)R * 3 * NNP_NP);
-        HIPCHK(h, hipMemcpy(blk.data(), h->d_coords.p + (size_t)rh.info.slot_base * 3 * NNP_NP * sizeof(double),
-                            blk.size() * sizeof(double), hipMemcpyDeviceToHost));
-        for (int s = 0; s < R; ++s)
-            for (int j = 0; j < N; ++j)
-                for (int c = 0; c < 3; ++c)
-                    x[((size_t)temp[s] * N + j) * 3 + c] = blk[((size_t)s * 3 + c) * NNP_NP + j];
-    } else if (x) {
-      for (const Seg &g : rh.segs) {
-        const TileInfo &ti = h->tiles[g.tile];
-        const int A = ti.n_slab, kl = rh.kl;
-        const size_t rsize = h->cfg.precision == 0 ? 8 : 4;
-        const size_t nblk = (size_t)3 * A * rh.lanes;
-        std::vector<unsigned char> blk(nblk * rsize);
-        HIPCHK(h, hipMemcpy(blk.data(), h->d_coords.p + (size_t)ti.coord_off * rsize, blk.size(), hipMemcpyDeviceToHost));
-        for (int s = g.t0; s < g.t0 + g.count; ++s) {
-            const int t = temp[s], lg = g.local0 + (s - g.t0);
-            for (int j = 0; j < N; ++j) {
-                const int sl = j / kl, lane = lg * kl + j % kl;
-                for (int c = 0; c < 3; ++c) {
-                    const size_t e_ = ((size_t)sl * 3 + c) * rh.lanes + lane;
-                    double v;
-                    if (rsize == 8) memcpy(&v, &blk[e_ * 8], 8);
-                    else {
-                        float f;
-                        memcpy(&f, &blk[e_ * 4], 4);
-                        v = f;
-                    }
-                    x[((size_t)t * N + j) * 3 + c] = v;
-                }
-            }
+    return PTMC_OK;
+}
+
+// n words from each of the device arrays into the host arrays (null: not
+// wanted), by way of the staging
+static int fetch_words(ptmc_engine *h, size_t n, int count, const void *const *src, void *const *dst)
+{
+    WordArrays a{};
+    void *to[RB_ARRAYS];
+    int m = 0;
+    for (int k = 0; k < count; ++k)
+        if (dst[k]) {
+            a.p[m] = (const uint64_t *)src[k];
+            to[m++] = dst[k];
         }
-      }
+    if (m == 0 || n == 0) {
+        HIPCHK(h, hipStreamSynchronize(h->stream));
+        return PTMC_OK;
     }
+    if (m * n * 8 > h->rb_bytes) {
+        HIPCHK(h, hipStreamSynchronize(h->stream));
+        for (int k = 0; k < m; ++k) HIPCHK(h, hipMemcpy(to[k], a.p[k], n * 8, hipMemcpyDeviceToHost));
+        return PTMC_OK;
+    }
+    std::lock_guard<std::mutex> lock(h->rb_mutex);
+    word_gather_kernel<<<dim3((unsigned)((n + RB_NT - 1) / RB_NT), m), RB_NT, 0, h->stream>>>(a, (int)n, (uint64_t *)h->rb);
+    HIPCHK(h, hipGetLastError());
+    HIPCHK(h, hipStreamSynchronize(h->stream));
+    for (int k = 0; k < m; ++k) memcpy(to[k], (const char *)h->rb + (size_t)k * n * 8, n * 8);
     return PTMC_OK;
 }
 
@@ -2058,15 +2133,12 @@ int ptmc_get_counters(ptmc_handle h, int32_t run, double *max_displ, int64_t *co
     int rc = check_run(h, run);
     if (rc) return rc;
     HIPCHK(h, hipSetDevice(h->cfg.device));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
     const RunHost &rh = h->runs[run];
     const size_t off = (size_t)2 * rh.info.temp_base, n = (size_t)2 * rh.d.n_temps;
-    if (max_displ) HIPCHK(h, hipMemcpy(max_displ, h->d_displ.p + off, n * 8, hipMemcpyDeviceToHost));
-    if (count_atom) HIPCHK(h, hipMemcpy(count_atom, h->d_count_atom.p + off, n * 8, hipMemcpyDeviceToHost));
-    if (count_vol) HIPCHK(h, hipMemcpy(count_vol, h->d_count_vol.p + off, n * 8, hipMemcpyDeviceToHost));
-    if (count_exc) HIPCHK(h, hipMemcpy(count_exc, h->d_count_exc.p + off, n * 8, hipMemcpyDeviceToHost));
-    if (ham) HIPCHK(h, hipMemcpy(ham, h->d_ham.p + off, n * 8, hipMemcpyDeviceToHost));
-    return PTMC_OK;
+    const void *src[] = {h->d_displ.p + off, h->d_count_atom.p + off, h->d_count_vol.p + off, h->d_count_exc.p + off,
+                         h->d_ham.p + off};
+    void *dst[] = {max_displ, count_atom, count_vol, count_exc, ham};
+    return fetch_words(h, n, 5, src, dst);
 }
 
 int ptmc_get_counters_sep(ptmc_handle h, int32_t run, double *max_displ_sep, int64_t *count_vol_xy,
@@ -2075,13 +2147,11 @@ int ptmc_get_counters_sep(ptmc_handle h, int32_t run, double *max_displ_sep, int
     int rc = check_run(h, run);
     if (rc) return rc;
     HIPCHK(h, hipSetDevice(h->cfg.device));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
     const RunHost &rh = h->runs[run];
     const size_t off = (size_t)2 * rh.info.temp_base, n = (size_t)2 * rh.d.n_temps;
-    if (max_displ_sep) HIPCHK(h, hipMemcpy(max_displ_sep, h->d_displ_sep.p + off, n * 8, hipMemcpyDeviceToHost));
-    if (count_vol_xy) HIPCHK(h, hipMemcpy(count_vol_xy, h->d_count_volxy.p + off, n * 8, hipMemcpyDeviceToHost));
-    if (count_vol_z) HIPCHK(h, hipMemcpy(count_vol_z, h->d_count_volz.p + off, n * 8, hipMemcpyDeviceToHost));
-    return PTMC_OK;
+    const void *src[] = {h->d_displ_sep.p + off, h->d_count_volxy.p + off, h->d_count_volz.p + off};
+    void *dst[] = {max_displ_sep, count_vol_xy, count_vol_z};
+    return fetch_words(h, n, 3, src, dst);
 }
 
 int ptmc_set_counters_sep(ptmc_handle h, int32_t run, const double *max_displ_sep, const int64_t *count_vol_xy,
