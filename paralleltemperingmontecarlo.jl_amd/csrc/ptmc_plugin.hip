@@ -4,7 +4,8 @@
 // once per call (one thread per matrix element), then the potential's
 // kernels run one thread per (configuration, atom) or per (configuration,
 // feature, atom), and every total is summed by one thread per configuration
-// in the reference's order.  The order of every sum follows the reference:
+// in the reference's order.  The order of the sums follows the reference, the
+// moved-atom update of the angular features excepted (noted there):
 //   dimer_energy_config       pairs i < j, row i then j (src/EnergyEvaluation.jl:378-396)
 //   dimer_energy_update!      sum over j != i of the new row minus the old (:313-336, :804-821)
 //   calc_components           row sums with the diagonal (:1105-1148)
@@ -12,12 +13,13 @@
 //   total_symm_calc           per atom: partners / partner triples in the
 //                             reference's pair and triple order
 //                             (MachineLearningPotential/SymmFunc.jl:259-312, :494-510)
-//   total_thr_symm!           per atom: the moved atom's pairs / pair couples in order
+//   total_thr_symm!           per atom: the moved atom's pairs / pair couples
 //                             (MachineLearningPotential/DeltaMatrix.jl:794-872, :933-975)
 // so pair potentials reproduce the reference's arithmetic operation by
 // operation; the EAM and network results differ from it only by the device's
 // pow / exp / cos / tanh against the host library's.
 #include "ptmc_plugin.hpp"
+#include "ptmc_nnp_layout.hpp"
 #include "ptmc_sweep.hpp"
 
 namespace ptmc {
@@ -25,12 +27,14 @@ namespace {
 
 constexpr int PT = 256;  // threads per workgroup
 
+constexpr int PLUGIN_ROWS = 6;
+
 struct WS {
     double *d2;    // squared distances
     double *m1;    // network: cut-off function; ELJB / LUT: xy extent^2
     double *m2;    // ELJB / LUT: z extent
     double *pe;    // pair energies
-    double *rows;  // update: per (configuration, partner) values, 4 rows of N
+    double *rows;  // update: per (configuration, partner) values, 4 rows of N (network 6)
     double *flag;  // network update: 1 = the hard-core test failed
 };
 
@@ -56,7 +60,7 @@ __host__ __device__ inline WS ws_of(const PluginJob &j)
         w.pe = j.ws + CM;
     }
     w.rows = j.ws + (size_t)plugin_mats(j.kind) * CM;
-    w.flag = w.rows + (size_t)4 * j.n_conf * j.N;
+    w.flag = w.rows + (size_t)PLUGIN_ROWS * j.n_conf * j.N;
     return w;
 }
 
@@ -459,36 +463,44 @@ __global__ void __launch_bounds__(PT) plugin_nnp_feature_kernel(PluginJob j)
     j.vars_out[((size_t)c * N + a) * nf + q] = g;
 }
 
-// forward pass of one atom: [nf] -> h1 (tanh) -> h2 (tanh) -> 1 (linear),
-// RuNNer parameter order (each layer's input-major weights, then its
-// biases); skipped where the hard-core test failed
+// forward pass: [nf] -> h1 (tanh) -> h2 (tanh) -> 1 (linear), RuNNer parameter
+// order (each layer's input-major weights, then its biases); skipped where the
+// hard-core test failed.  A thread per (atom, output of a layer), four atoms a
+// workgroup: every dot product in order, as one thread per atom would take it,
+// but the outputs of a layer at once (one thread per atom waited for 88 x 20
+// loads in a row: 0.29 ms for 40 x 55 atoms, 0.02 so).
+constexpr int NET_ATOMS = PT / PLUGIN_MAXH;
 __global__ void __launch_bounds__(PT) plugin_nnp_network_kernel(PluginJob j)
 {
-    const int N = j.N, nf = plugin_nf(j);
-    const size_t t = (size_t)blockIdx.x * PT + threadIdx.x;
-    if (t >= (size_t)j.n_conf * N) return;
-    const int c = (int)(t / N);
-    if (ws_of(j).flag[c] != 0.0) return;
-    const double *g = j.vars_out + t * nf;
+    __shared__ double a1[NET_ATOMS][PLUGIN_MAXH], a2[NET_ATOMS][PLUGIN_MAXH];
+    const int nf = plugin_nf(j), la = threadIdx.x / PLUGIN_MAXH, o = threadIdx.x % PLUGIN_MAXH;
+    const size_t t = (size_t)blockIdx.x * NET_ATOMS + la;
+    const bool in = t < (size_t)j.n_conf * j.N && ws_of(j).flag[t / j.N] == 0.0;
     const double *W1 = j.w, *B1 = W1 + (size_t)nf * j.h1, *W2 = B1 + j.h1, *B2 = W2 + (size_t)j.h1 * j.h2;
     const double *W3 = B2 + j.h2, *B3 = W3 + j.h2;
-    double a1[PLUGIN_MAXH], a2[PLUGIN_MAXH];
-    for (int o = 0; o < j.h1; ++o) {
+    if (in && o < j.h1) {
+        const double *g = j.vars_out + t * nf;
         double s = 0.0;
+#pragma unroll 8
         for (int k = 0; k < nf; ++k) s += g[k] * W1[(size_t)k * j.h1 + o];
         s += B1[o];
-        a1[o] = tanh(s);
+        a1[la][o] = tanh(s);
     }
-    for (int o = 0; o < j.h2; ++o) {
+    __syncthreads();
+    if (in && o < j.h2) {
         double s = 0.0;
-        for (int k = 0; k < j.h1; ++k) s += a1[k] * W2[(size_t)k * j.h2 + o];
+#pragma unroll 4
+        for (int k = 0; k < j.h1; ++k) s += a1[la][k] * W2[(size_t)k * j.h2 + o];
         s += B2[o];
-        a2[o] = tanh(s);
+        a2[la][o] = tanh(s);
     }
-    double s = 0.0;
-    for (int k = 0; k < j.h2; ++k) s += a2[k] * W3[k];
-    s += B3[0];
-    j.en_atom[t] = s;
+    __syncthreads();
+    if (in && o == 0) {
+        double s = 0.0;
+        for (int k = 0; k < j.h2; ++k) s += a2[la][k] * W3[k];
+        s += B3[0];
+        j.en_atom[t] = s;
+    }
 }
 
 // sum of the per-atom energies in order; 100 where the hard-core test
@@ -507,8 +519,8 @@ __global__ void __launch_bounds__(PT) plugin_nnp_sum_kernel(PluginJob j)
 }
 
 // energy_update!(RuNNerPotential), per partner k of the moved atom i: new
-// and old squared distances and cut-off functions (rows 0-3); a partner
-// inside the hard-core distance marks the configuration
+// and old squared distances, cut-off functions and distances (rows 0-5); a
+// partner inside the hard-core distance marks the configuration
 __global__ void __launch_bounds__(PT) plugin_nnp_row_kernel(PluginJob j)
 {
     const int N = j.N;
@@ -520,95 +532,207 @@ __global__ void __launch_bounds__(PT) plugin_nnp_row_kernel(PluginJob j)
     const BoxC<double> B = box_of(j, c, l, h);
     const double rn = k == i ? 0.0 : geom(j, j.trial + 3 * (size_t)c, j.x + ((size_t)c * N + k) * 3, B, dxy, dz);
     const size_t ik = (size_t)c * N * N + (size_t)i * N + k;
-    double *R = w.rows + (size_t)c * 4 * N;
+    double *R = w.rows + (size_t)c * PLUGIN_ROWS * N;
+    const double dn = sqrt(rn);
     R[k] = rn;
     R[N + k] = w.d2[ik];
-    R[2 * N + k] = fcut(sqrt(rn), j.r_cut);
+    R[2 * N + k] = fcut(dn, j.r_cut);
     R[3 * N + k] = w.m1[ik];
+    R[4 * N + k] = dn;
+    R[5 * N + k] = sqrt(w.d2[ik]);
     if (k != i && rn < j.hardcore2) w.flag[c] = 1.0;
 }
 
-// total_thr_symm!: one thread per (configuration, function, atom) adds the
-// atom's share of the change, in the reference's order: radial, the pair
-// with the moved atom (new term, then the old one subtracted as a negative
-// term); angular, the partner couples (k, l), k < l, both != i, that hold
-// the atom (all of them for the moved atom), each adding the new triple's
-// value and subtracting the old one.  Where the hard-core test failed the
-// features are copied.
+// p^(2^sq) by squarings that carry each product's rounding (h + l), rounded
+// once at the end
+__device__ __forceinline__ double square_up(double p, int sq)
+{
+    double h = p, l = 0.0;
+    for (int k = 0; k < sq; ++k) {
+        const double q = h * h;
+        l = fma(2.0 * h, l, fma(h, h, -q));
+        h = q;
+    }
+    return h + l;
+}
+
+// sum over the workgroup, on every thread, in a fixed order
+__device__ __forceinline__ double block_sum(double v, double *red)
+{
+    v = group_sum<16>(v);
+    v += row_xor<16>(v);
+    v += row_xor<32>(v);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double s = red[0];
+    for (int k = 1; k < PT / 64; ++k) s += red[k];
+    return s;
+}
+
+// total_thr_symm!: the change of every function at every atom, new terms added
+// and old ones subtracted; radial, the pair with the moved atom i; angular, the
+// partner couples (k, l) that hold the atom (all of them for the moved atom).
+// Where the hard-core test failed the features are copied.
+//
+// One workgroup per (configuration, function).  The angular functions of one eta
+// are done by the first of them (the other workgroups end at once), DU at a time,
+// so a couple's two exponentials and four cosines are taken once for all; S lanes
+// share the partners of a target atom, and the couple's term centred on i is
+// added where the target is the smaller of the two.  The sums at an atom are
+// taken by lane and then over the lanes, those at i over the workgroup, both in
+// a fixed order.  Before, a thread took one (function, atom) with a pow per
+// term: the moved atom's thread went through 1431 couples in a row, 4.9 ms for
+// 40 x 55 atoms x 88 functions whatever else ran; 0.14 ms so.  Bound by the FP64
+// instructions of a couple (about 700 for eight functions).
+constexpr int DU = 8;
 __global__ void __launch_bounds__(PT) plugin_nnp_delta_kernel(PluginJob j)
 {
-    const int N = j.N, nf = plugin_nf(j);
-    const size_t t = (size_t)blockIdx.x * PT + threadIdx.x;
-    if (t >= (size_t)j.n_conf * nf * N) return;
-    const int c = (int)(t / ((size_t)nf * N)), rem = (int)(t % ((size_t)nf * N)), q = rem / N, a = rem % N;
+    __shared__ uint64_t s_same[2];
+    __shared__ int s_idx[DU];
+    __shared__ double s_par[DU][2], red[PT / 64];
+    __shared__ int s_sq[DU];
+    const int N = j.N, nf = plugin_nf(j), tid = threadIdx.x;
+    const int c = (int)(blockIdx.x / (unsigned)nf), q = (int)(blockIdx.x % (unsigned)nf);
     const WS w = ws_of(j);
-    const size_t out = ((size_t)c * N + a) * nf + q;
-    double v = j.vars_in[out];
-    if (w.flag[c] != 0.0) {
-        j.vars_out[out] = v;
+    const size_t base = (size_t)c * N * nf;
+    const double *in = j.vars_in + base;
+    double *out = j.vars_out + base;
+    const bool rad = q < j.n_rad;
+    const double *A = rad ? j.rad + 4 * q : j.ang + 6 * (q - j.n_rad);
+    if (w.flag[c] != 0.0 || A[rad ? 3 : 5] == 0.0) {
+        for (int a = tid; a < N; a += PT) out[(size_t)a * nf + q] = in[(size_t)a * nf + q];
         return;
     }
     const int i = j.index[c];
-    const double *R = w.rows + (size_t)c * 4 * N;
-    const double *rn = R, *ro = R + N, *fn = R + 2 * N, *fo = R + 3 * N;
-    if (q < j.n_rad) {
-        const double *Rd = j.rad + 4 * q;
-        if (Rd[3] != 0.0) {
-            const double eta = Rd[0], norm = Rd[1];
-            if (a != i) {
-                v += exp(-eta * rn[a]) * (fn[a] * norm);
-                v += exp(-eta * ro[a]) * (-fo[a] * norm);
-            } else {
-                for (int k = 0; k < N; ++k) {
-                    if (k == i) continue;
-                    v += exp(-eta * rn[k]) * (fn[k] * norm);
-                    v += exp(-eta * ro[k]) * (-fo[k] * norm);
+    const double *R = w.rows + (size_t)c * PLUGIN_ROWS * N;
+    const double *rn = R, *ro = R + N, *fn = R + 2 * N, *fo = R + 3 * N, *dn = R + 4 * N, *dold = R + 5 * N;
+    if (rad) {
+        const double eta = A[0], norm = A[1];
+        double sum = 0.0;
+        for (int a = tid; a < N; a += PT) {
+            if (a == i) continue;
+            const double tn = exp(-eta * rn[a]) * (fn[a] * norm), to = exp(-eta * ro[a]) * (-fo[a] * norm);
+            const double v = in[(size_t)a * nf + q] + tn;
+            out[(size_t)a * nf + q] = v + to;
+            sum += tn;
+            sum += to;
+        }
+        sum = block_sum(sum, red);
+        if (tid == 0) out[(size_t)i * nf + q] = in[(size_t)i * nf + q] + sum;
+        return;
+    }
+    // the active functions of this eta (at most 128 functions in all); the first does them
+    const int qa = q - j.n_rad;
+    const double eta = A[0];
+    if (tid < 128) {
+        const bool same = tid < j.n_ang && j.ang[6 * tid + 5] != 0.0 && (j.ang[6 * tid] == eta || tid == qa);
+        const uint64_t b = __ballot(same);
+        if ((tid & 63) == 0) s_same[tid >> 6] = b;
+    }
+    __syncthreads();
+    uint64_t same[2] = {s_same[0], s_same[1]};
+    if ((qa < 64 ? same[0] & ((1ull << qa) - 1) : same[0] | (same[1] & ((1ull << (qa - 64)) - 1))) != 0) return;
+    int S = 1;  // lanes of a target: as many as the workgroup has for N targets, up to a row
+    while (S < 16 && 2 * S * N <= PT) S *= 2;
+    const int part = tid & (S - 1);
+    const double *r2 = w.d2 + (size_t)c * N * N, *f = w.m1 + (size_t)c * N * N;
+    const double *X = j.x + (size_t)c * N * 3, *T = j.trial + 3 * (size_t)c, *Xi = X + 3 * i;
+    while ((same[0] | same[1]) != 0) {
+        __syncthreads();
+        int cnt = 0;
+        for (; cnt < DU && (same[0] | same[1]) != 0; ++cnt) {
+            const int h = same[0] != 0 ? 0 : 1, u = 64 * h + __builtin_ctzll(same[h]);
+            same[h] &= same[h] - 1;
+            if (tid == cnt) {
+                s_idx[cnt] = j.n_rad + u;
+                s_par[cnt][0] = j.ang[6 * u + 1];
+                s_par[cnt][1] = j.ang[6 * u + 3];
+                s_sq[cnt] = ilogb(j.ang[6 * u + 2]);  // zeta is a power of two
+            }
+        }
+        __syncthreads();
+        double vi[DU];
+#pragma unroll
+        for (int u = 0; u < DU; ++u) vi[u] = 0.0;
+        for (int a0 = 0; a0 < N; a0 += PT / S) {
+            const int a = a0 + tid / S;
+            double va[DU];
+#pragma unroll
+            for (int u = 0; u < DU; ++u) va[u] = 0.0;
+            if (a < N && a != i) {
+                const double *Xa = X + 3 * a;
+                for (int b = part; b < N; b += S) {
+                    if (b == i || b == a) continue;
+                    const int k = a < b ? a : b, l = a < b ? b : a;
+                    const double fkl = f[(size_t)k * N + l];
+                    const double pn = fn[k] * fn[l] * fkl, po = fo[k] * fo[l] * fkl;
+                    if (pn == 0.0 && po == 0.0) continue;
+                    const double rkl = r2[(size_t)k * N + l], dkl = sqrt(rkl);
+                    const double en = exp(-eta * (rn[k] + rn[l] + rkl)) * fn[k] * fn[l] * fkl;
+                    const double eo = exp(-eta * (ro[k] + ro[l] + rkl)) * fo[k] * fo[l] * fkl;
+                    const double *Xb = X + 3 * b;
+                    const double abx = Xa[0] - Xb[0], aby = Xa[1] - Xb[1], abz = Xa[2] - Xb[2];
+                    const double tn = theta(Xa[0] - T[0], Xa[1] - T[1], Xa[2] - T[2], abx, aby, abz, dn[a], dkl);
+                    const double to = theta(Xa[0] - Xi[0], Xa[1] - Xi[1], Xa[2] - Xi[2], abx, aby, abz, dold[a], dkl);
+#pragma unroll
+                    for (int u = 0; u < DU; ++u)
+                        if (u < cnt) {
+                            const double lam = s_par[u][0], tpz = s_par[u][1];
+                            va[u] += en * square_up(1.0 + lam * tn, s_sq[u]) * tpz;
+                            va[u] -= eo * square_up(1.0 + lam * to, s_sq[u]) * tpz;
+                        }
+                    if (a < b) {
+                        const double in_ = theta(T[0] - Xa[0], T[1] - Xa[1], T[2] - Xa[2], T[0] - Xb[0], T[1] - Xb[1],
+                                                 T[2] - Xb[2], dn[a], dn[b]);
+                        const double io = theta(Xi[0] - Xa[0], Xi[1] - Xa[1], Xi[2] - Xa[2], Xi[0] - Xb[0],
+                                                Xi[1] - Xb[1], Xi[2] - Xb[2], dold[a], dold[b]);
+#pragma unroll
+                        for (int u = 0; u < DU; ++u)
+                            if (u < cnt) {
+                                const double lam = s_par[u][0], tpz = s_par[u][1];
+                                vi[u] += en * square_up(1.0 + lam * in_, s_sq[u]) * tpz;
+                                vi[u] -= eo * square_up(1.0 + lam * io, s_sq[u]) * tpz;
+                            }
+                    }
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < DU; ++u) {
+                if (u >= cnt) break;
+                double v = va[u];
+                if (S >= 2) v += dpp_perm<0xB1>(v);
+                if (S >= 4) v += dpp_perm<0x4E>(v);
+                if (S >= 8) v += dpp_perm<0x141>(v);
+                if (S >= 16) v += dpp_perm<0x140>(v);
+                if (part == 0 && a < N && a != i) {
+                    const size_t o = (size_t)a * nf + s_idx[u];
+                    out[o] = in[o] + v;
                 }
             }
         }
-    } else {
-        const double *A = j.ang + 6 * (q - j.n_rad);
-        if (A[5] != 0.0) {
-            const double eta = A[0], lam = A[1], zeta = A[2], tpz = A[3];
-            const double *r2 = w.d2 + (size_t)c * N * N, *f = w.m1 + (size_t)c * N * N;
-            const double *X = j.x + (size_t)c * N * 3, *T = j.trial + 3 * (size_t)c, *Xi = X + 3 * i;
-            auto couple = [&](int k, int l, int vtx) {
-                const double fkl = f[(size_t)k * N + l];
-                const double pn = fn[k] * fn[l] * fkl, po = fo[k] * fo[l] * fkl;
-                if (pn == 0.0 && po == 0.0) return;
-                const double rkl = r2[(size_t)k * N + l];
-                const double en = exp(-eta * (rn[k] + rn[l] + rkl)) * fn[k] * fn[l] * fkl;
-                const double eo = exp(-eta * (ro[k] + ro[l] + rkl)) * fo[k] * fo[l] * fkl;
-                const double tn = cos_at(vtx, T, X + 3 * k, X + 3 * l, rn[k], rn[l], rkl);
-                const double to = cos_at(vtx, Xi, X + 3 * k, X + 3 * l, ro[k], ro[l], rkl);
-                v += en * pow(1.0 + lam * tn, zeta) * tpz;
-                v -= eo * pow(1.0 + lam * to, zeta) * tpz;
-            };
-            if (a != i) {
-                for (int k = 0; k < a; ++k)
-                    if (k != i) couple(k, a, 2);
-                for (int l = a + 1; l < N; ++l)
-                    if (l != i) couple(a, l, 1);
-            } else {
-                for (int k = 0; k < N; ++k) {
-                    if (k == i) continue;
-                    for (int l = k + 1; l < N; ++l)
-                        if (l != i) couple(k, l, 0);
-                }
+#pragma unroll
+        for (int u = 0; u < DU; ++u) {
+            if (u >= cnt) break;
+            const double v = block_sum(vi[u], red);
+            if (tid == 0) {
+                const size_t o = (size_t)i * nf + s_idx[u];
+                out[o] = in[o] + v;
             }
         }
     }
-    j.vars_out[out] = v;
 }
+static_assert(NNP_MAXF <= 128, "the functions of one eta in two masks");
 
 inline unsigned blocks(size_t n) { return (unsigned)((n + PT - 1) / PT); }
+inline unsigned net_blocks(size_t n) { return (unsigned)((n + NET_ATOMS - 1) / NET_ATOMS); }
 
 }  // namespace
 
 size_t plugin_workspace_doubles(const PluginJob &j)
 {
     const size_t C = (size_t)j.n_conf, N = (size_t)j.N;
-    return C * N * N * plugin_mats(j.kind) + 4 * C * N + C;
+    return C * N * N * plugin_mats(j.kind) + PLUGIN_ROWS * C * N + C;
 }
 
 hipError_t plugin_initialise(const PluginJob &j, hipStream_t s)
@@ -620,7 +744,7 @@ hipError_t plugin_initialise(const PluginJob &j, hipStream_t s)
         hipLaunchKernelGGL(plugin_eam_energy_kernel, dim3(blocks(C)), dim3(PT), 0, s, j);
     } else if (j.kind == POT_NNP) {
         hipLaunchKernelGGL(plugin_nnp_feature_kernel, dim3(blocks(C * plugin_nf(j) * N)), dim3(PT), 0, s, j);
-        hipLaunchKernelGGL(plugin_nnp_network_kernel, dim3(blocks(C * N)), dim3(PT), 0, s, j);
+        hipLaunchKernelGGL(plugin_nnp_network_kernel, dim3(net_blocks(C * N)), dim3(PT), 0, s, j);
         hipLaunchKernelGGL(plugin_nnp_sum_kernel, dim3(blocks(C)), dim3(PT), 0, s, j);
     } else {
         hipLaunchKernelGGL(plugin_pair_kernel, dim3(blocks(C * N * N)), dim3(PT), 0, s, j);
@@ -638,8 +762,8 @@ hipError_t plugin_update(const PluginJob &j, hipStream_t s)
     } else if (j.kind == POT_NNP) {
         hipLaunchKernelGGL(plugin_geom_kernel, dim3(blocks(C * N * N)), dim3(PT), 0, s, j);
         hipLaunchKernelGGL(plugin_nnp_row_kernel, dim3(blocks(C * N)), dim3(PT), 0, s, j);
-        hipLaunchKernelGGL(plugin_nnp_delta_kernel, dim3(blocks(C * plugin_nf(j) * N)), dim3(PT), 0, s, j);
-        hipLaunchKernelGGL(plugin_nnp_network_kernel, dim3(blocks(C * N)), dim3(PT), 0, s, j);
+        hipLaunchKernelGGL(plugin_nnp_delta_kernel, dim3((unsigned)(C * plugin_nf(j))), dim3(PT), 0, s, j);
+        hipLaunchKernelGGL(plugin_nnp_network_kernel, dim3(net_blocks(C * N)), dim3(PT), 0, s, j);
         hipLaunchKernelGGL(plugin_nnp_sum_kernel, dim3(blocks(C)), dim3(PT), 0, s, j);
     } else {
         hipLaunchKernelGGL(plugin_pair_row_kernel, dim3(blocks(C * N)), dim3(PT), 0, s, j);
