@@ -311,6 +311,26 @@ int default_lanes(int n_atoms, int precision)
     return kl;
 }
 
+// Lanes of a FP64 ladder for which none are asked.  A move is a serial chain of
+// pair terms, bound by the latency of its FP64 instructions, so while the chip
+// has idle SIMDs a configuration gains from more lanes than default_lanes, up
+// to one wave on each SIMD: 256 lanes of a ladder (one workgroup) and 256 lanes
+// a CU over the whole batch.  us per cycle at default_lanes / so: 32
+// temperatures x 13 atoms 40 / 14, x 20 45 / 23, x 38 90 / 60, 8 x 55 107 / 81;
+// 32 atoms in a cubic box at constant pressure, 32 temperatures 488 / 216; 1024
+// ladders of 32 x 13 39 / 28.  Past it waves share a SIMD and the exchange of
+// partial sums is paid for nothing (1024 x 32 x 13: 2 and 4 lanes 28, 8 37, 16 56;
+// one ladder of 32 x 13 on 16 lanes 15, on 8 14).  Binary32 keeps its widths:
+// the order of its sums decides between trajectories; so does the reference
+// pair form, whose sums are the reference's only in sequence.
+int fp64_lanes(int n_atoms, int n_temps, int64_t all_slots, int cus)
+{
+    int kl = default_lanes(n_atoms, 0);
+    while (kl < 16 && kl < n_atoms && 2 * kl * n_temps <= LANES_SMALL && 2 * kl * all_slots <= (int64_t)LANES_SMALL * cus)
+        kl *= 2;
+    return kl;
+}
+
 // bc is the configured boundary: rectangular boxes run the cubic kernels
 KernelPair lookup(int precision, int bc, int ens, int pot, int pk, int kc, int kl, int lanes)
 {
@@ -616,6 +636,11 @@ int plan(ptmc_engine *h)
     int max_lds = 0;
     HIPCHK(h, hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
 
+    int cus = 0;
+    HIPCHK(h, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    int64_t all_slots = 0;
+    for (const RunHost &rh : h->runs) all_slots += rh.d.n_temps;
+
     // group runs by (lanes per configuration, workgroup width, N)
     std::map<std::tuple<int, int, int>, std::vector<int>> groups;
     for (int r = 0; r < (int)h->runs.size(); ++r) {
@@ -623,6 +648,7 @@ int plan(ptmc_engine *h)
         const int N = rh.d.n_atoms, R = rh.d.n_temps;
         const int req = rh.d.lanes_per_replica > 0 ? rh.d.lanes_per_replica
                         : h->cfg.lanes_per_replica > 0 ? h->cfg.lanes_per_replica
+                        : prec == 0 && !eam && h->cfg.pair_form == 0 ? fp64_lanes(N, R, all_slots, cus)
                                                        : default_lanes(N, prec);
         if (req > 16)
             return fail(h, PTMC_E_UNSUPPORTED, "run %d: %d lanes per configuration need the spread layout "
