@@ -23,11 +23,11 @@
 using namespace ptmc;
 
 namespace ptmc {
-SweepFn nnp_sweep_fn(int np);
+SweepFn nnp_sweep_fn(int np, int nt);
 SweepFn nnp_sweep_da_fn();
 bool pair_slot_fns(int pk, int kc, bool da, SweepFn *sweep, SweepFn *init);
 size_t pair_slot_lds_bytes(bool da);
-SweepFn nnp_init_fn(int np);
+SweepFn nnp_init_fn(int np, int nt);
 SweepFn nnp2_sweep_fn(bool pow);
 SweepFn nnp2_init_fn(bool pow);
 SweepFn nnp2_sweep_fn_f32(bool pow);
@@ -229,6 +229,7 @@ struct ptmc_engine {
     NnpTables nnp_dev{};
     size_t nnp_lds = 0;
     int nnp_np = NNP_NP;  // atoms per slot of the network-potential engine (64 or 128)
+    int nnp_nt = NNP_NT;  // threads per slot (NNP_NT or twice that)
 
     // two-species network potential, NNVT (one workgroup per slot, FP64)
     bool nnvt = false;
@@ -1023,6 +1024,17 @@ int prepare_nnp2(ptmc_engine *h)
 
 // Slots of a neural-network engine: one workgroup per slot, slots of a run
 // consecutive, temperature t of run r starting in slot slot_base + t.
+// Threads of a slot.  Slots of 128 atoms have a CU to themselves (LDS) and take
+// 1024 threads, and so do slots of 64 while there are no more of them than CUs
+// (us per cycle on 512 / 1024 threads: 40 x 55 atoms 1224 / 1121, 40 x 33 618 /
+// 602, 256 x 55 1248 / 1150).  Past that two slots of 512 share a CU and hide
+// each other's barriers (264 x 55 1624 / 2129, 1280 x 55 3950 / 5348), and small
+// clusters do not fill 16 waves (40 x 13 201 / 221).
+int nnp_threads(int np, int n_max, int64_t slots, int cus)
+{
+    return np > NNP_NP || (slots <= cus && n_max > NNP_NP / 2) ? 2 * NNP_NT : NNP_NT;
+}
+
 int prepare_nnp(ptmc_engine *h)
 {
     if (h->cfg.precision != 1) return fail(h, PTMC_E_UNSUPPORTED, "the network potential runs in binary32 (precision 1)");
@@ -1041,15 +1053,23 @@ int prepare_nnp(ptmc_engine *h)
     if ((long long)h->nnp_lds > max_lds)
         return fail(h, PTMC_E_UNSUPPORTED, "network tables for %d-atom slots need %zu B of LDS (%d available)", h->nnp_np,
                     h->nnp_lds, max_lds);
-    const void *fs = (const void *)nnp_sweep_fn(h->nnp_np), *fi = (const void *)nnp_init_fn(h->nnp_np);
+    int64_t slots = 0;
+    for (const RunHost &rh : h->runs) slots += rh.d.n_temps;
+    int cus = 0;
+    HIPCHK(h, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    h->nnp_nt = nnp_threads(h->nnp_np, n_max, slots, cus);
+    const void *fs = (const void *)nnp_sweep_fn(h->nnp_np, h->nnp_nt), *fi = (const void *)nnp_init_fn(h->nnp_np, h->nnp_nt);
     HIPCHK(h, hipFuncSetAttribute(fs, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->nnp_lds));
     HIPCHK(h, hipFuncSetAttribute(fi, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->nnp_lds));
+    // delayed acceptance initialises on NNP_NT threads
+    HIPCHK(h, hipFuncSetAttribute((const void *)nnp_init_fn(h->nnp_np, NNP_NT), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)h->nnp_lds));
     int slot = 0;
     for (auto &rh : h->runs) {
         rh.info.slot_base = slot;
         rh.info.local_base = 0;
-        rh.kl = NNP_NT;
-        rh.lanes = NNP_NT;
+        rh.kl = h->nnp_nt;
+        rh.lanes = h->nnp_nt;
         rh.tile = -1;
         slot += rh.d.n_temps;
     }
@@ -1060,8 +1080,8 @@ int prepare_nnp(ptmc_engine *h)
     L.fn = (SweepFn)fs;
     L.init = (SweepFn)fi;
     L.ntiles = slot;
-    L.wgs = NNP_NT;
-    L.kl = NNP_NT;
+    L.wgs = h->nnp_nt;
+    L.kl = h->nnp_nt;
     L.lds = h->nnp_lds;
     h->launches.push_back(L);
     h->n_coord = (int64_t)slot * 3 * h->nnp_np;
@@ -2578,7 +2598,10 @@ int ptmc_surrogate_enable(ptmc_handle h, int32_t on)
         L.lds = pair_slot_lds_bytes(h->sur.da);
         return PTMC_OK;
     }
-    L.fn = h->sur.da ? nnp_sweep_da_fn() : nnp_sweep_fn(h->nnp_np);
+    // delayed acceptance runs on NNP_NT threads
+    L.wgs = h->sur.da ? NNP_NT : h->nnp_nt;
+    L.init = nnp_init_fn(h->nnp_np, L.wgs);
+    L.fn = h->sur.da ? nnp_sweep_da_fn() : nnp_sweep_fn(h->nnp_np, h->nnp_nt);
     L.lds = h->nnp_lds + (h->sur.da ? sur_lds_floats() * sizeof(float) : 0);
     return PTMC_OK;
 }

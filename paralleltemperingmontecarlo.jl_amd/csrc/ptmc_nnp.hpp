@@ -223,10 +223,11 @@ __device__ __forceinline__ uint64_t nnp_drop(uint64_t m, int n)
 // for ten and one lane per slot writes.  Every old value is read before the
 // first is written: the reads are in flight together.  All lanes call.
 static_assert(NNP_KSLOT == 5, "slots (k, k + 1) of each lambda in three registers");
-template <int NP>
+template <int NP, int SETS>
 __device__ __forceinline__ void nnp_store(const NnpGroup &G, const int32_t *gd, int lp, bool writer, int j, int i,
-                                          int lane, float *Dp, const float *aj, const float *ai)
+                                          int lane, float *Dp, float *col, const float *aj, const float *ai)
 {
+    const float p1 = lp >= 1 ? 1.0f : 0.0f, p2 = lp >= 2 ? 1.0f : 0.0f, p3 = lp >= 3 ? 1.0f : 0.0f;
     // the slot whose sum this lane writes
     const int kq = 2 * (lane & 3) + ((lane >> 4) & 1), qi = NNP_KSLOT * (lane >> 5) + kq;
     const bool iw = (lane & 15) < 3 && kq < NNP_KSLOT;
@@ -236,18 +237,16 @@ __device__ __forceinline__ void nnp_store(const NnpGroup &G, const int32_t *gd, 
     float old[NNP_GMAX];
 #pragma unroll
     for (int q = 0; q < NNP_GMAX; ++q) old[q] = Dp[(G.row0 + (G.rk[q] < 0 ? 0 : G.rk[q])) * NP + j];
-    float *di = Dp + (G.row0 + (irk < 0 ? 0 : irk)) * NP + i;
-    const float oldi = *di;
+    const int irow = G.row0 + (irk < 0 ? 0 : irk);
+    float *di = Dp + irow * NP + i;
+    const float oldi = SETS == 1 ? *di : 0.0f;
 #pragma unroll
     for (int q = 0; q < NNP_GMAX; ++q) {
         if (G.rk[q] >= 0) {
             float v = aj[q];
-            const float t1 = dpp_f<0xB1>(v);
-            v = lp >= 1 ? v + t1 : v;
-            const float t2 = dpp_f<0x4E>(v);
-            v = lp >= 2 ? v + t2 : v;
-            const float t3 = dpp_f<0x141>(v);
-            v = lp >= 3 ? v + t3 : v;
+            v = __builtin_fmaf(dpp_f<0xB1>(v), p1, v);
+            v = __builtin_fmaf(dpp_f<0x4E>(v), p2, v);
+            v = __builtin_fmaf(dpp_f<0x141>(v), p3, v);
             if (writer) Dp[(G.row0 + G.rk[q]) * NP + j] = __builtin_fmaf(v, G.tpz[q], old[q]);
         }
     }
@@ -258,19 +257,22 @@ __device__ __forceinline__ void nnp_store(const NnpGroup &G, const int32_t *gd, 
     const float s1 = row_sum16(row_merge<16>(h[2], h[3]));
     const float s2 = row_sum16(row_pair_sum<16>(h[4]));
     const float s = (lane & 3) == 0 ? s0 : ((lane & 3) == 1 ? s1 : s2);
-    if (iw && irk >= 0) *di = __builtin_fmaf(s, itpz, oldi);
+    if (iw && irk >= 0) {
+        if (SETS == 1) *di = __builtin_fmaf(s, itpz, oldi);
+        else col[irow] = s * itpz;  // the other half adds its own
+    }
 }
 
 // Full feature matrix from positions into Gout (total_symm_calc,
 // SymmFunc.jl:494-510; radial :259-278, angular :280-312).  All threads call.
-template <int NP>
+template <int NP, int NT>
 __device__ void nnp_full_build(const NnpTables &T, const NnpLds &L, float *Gout, int N)
 {
     const int tid = threadIdx.x;
-    for (int e = tid; e < T.nf * NP; e += NNP_NT) Gout[e] = 0.0f;
+    for (int e = tid; e < T.nf * NP; e += NT) Gout[e] = 0.0f;
     __syncthreads();
     // radial: one (function, atom) per item
-    for (int e = tid; e < T.n_rad_active * N; e += NNP_NT) {
+    for (int e = tid; e < T.n_rad_active * N; e += NT) {
         const int q = e / N, a = e % N;
         const float eta = L.rad[4 * q], norm = L.rad[4 * q + 1];
         const int row = (int)L.rad[4 * q + 2];
@@ -286,7 +288,7 @@ __device__ void nnp_full_build(const NnpTables &T, const NnpLds &L, float *Gout,
     }
     // angular: one triangle a < b < c per item, all functions
     const int ntri = N * (N - 1) * (N - 2) / 6;
-    for (int e = tid; e < ntri; e += NNP_NT) {
+    for (int e = tid; e < ntri; e += NT) {
         // decode e -> (a, b, c)
         int a = 0, rem = e;
         while (rem >= (N - 1 - a) * (N - 2 - a) / 2) {
@@ -330,7 +332,7 @@ __device__ void nnp_full_build(const NnpTables &T, const NnpLds &L, float *Gout,
         }
     }
     __syncthreads();
-    for (int e = tid; e < T.nf * N; e += NNP_NT) {
+    for (int e = tid; e < T.nf * N; e += NT) {
         const int q = e / N, a = e % N;
         Gout[q * NP + a] += T.row_off[q];
     }
@@ -364,16 +366,21 @@ __device__ __forceinline__ nnp_f32x4 nnp_tile(int n, X x, W w)
     const int lk = (threadIdx.x & 63) >> 4;
     nnp_f32x4 z[4] = {};
     int k0 = 0;
-    for (; k0 + 16 <= n; k0 += 16) {
-        float a[4], b[4];
+    auto block = [&](auto steps) {  // the operands of all steps in flight together
+        constexpr int S = decltype(steps)::value;
+        float a[S], b[S];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < S; ++u) {
             a[u] = x(k0 + 4 * u + lk);
             b[u] = w(k0 + 4 * u + lk);
         }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) z[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u], b[u], z[u], 0, 0, 0);
-    }
+        for (int u = 0; u < S; ++u) z[u & 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u], b[u], z[u & 3], 0, 0, 0);
+        k0 += 4 * S;
+    };
+    while (k0 + 32 <= n) block(std::integral_constant<int, 8>{});
+    if (k0 + 16 <= n) block(std::integral_constant<int, 4>{});
+    if (k0 + 8 <= n) block(std::integral_constant<int, 2>{});
     for (; k0 < n; k0 += 4) {
         const int k = k0 + lk, kc = k < n ? k : n - 1;
         const float m = k < n ? 1.0f : 0.0f;
@@ -389,7 +396,7 @@ __device__ __forceinline__ nnp_f32x4 nnp_tile(int n, X x, W w)
 // tiles left the other six waiting for 44 steps of 64 cycles).  The
 // output layer's dot product is a row sum per tile; the FP64 total is a sum
 // over each wave of 64 atoms (DPP and row swaps), then the waves' sums in order.  All threads call.
-template <int NP>
+template <int NP, int NT>
 __device__ void nnp_forward(const NnpTables &T, const NnpLds &L, const float *Gin, int N, float *out,
                             double *total = nullptr)
 {
@@ -399,7 +406,7 @@ __device__ void nnp_forward(const NnpTables &T, const NnpLds &L, const float *Gi
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lr = l & 15, lk = l >> 4;
     const int nf = T.nf, h1 = T.h1, h2 = T.h2;
-    for (int t = w; t < 2 * (NP / 16); t += NNP_NT / 64) {
+    for (int t = w; t < 2 * (NP / 16); t += NT / 64) {
         const int r0 = 16 * (t % (NP / 16)), c0 = 16 * (t / (NP / 16));
         if (r0 >= N || c0 >= h1) continue;
         const int c = c0 + lr, cc = c < h1 ? c : h1 - 1;
@@ -412,7 +419,7 @@ __device__ void nnp_forward(const NnpTables &T, const NnpLds &L, const float *Gi
         }
     }
     __syncthreads();
-    for (int t = w; t < 2 * (NP / 16); t += NNP_NT / 64) {
+    for (int t = w; t < 2 * (NP / 16); t += NT / 64) {
         const int r0 = 16 * (t % (NP / 16)), c0 = 16 * (t / (NP / 16));
         if (r0 >= N || c0 >= h2) continue;
         const int c = c0 + lr, cc = c < h2 ? c : h2 - 1;
@@ -462,19 +469,19 @@ __device__ void nnp_forward(const NnpTables &T, const NnpLds &L, const float *Gi
     __syncthreads();
 }
 
-template <int NP>
+template <int NP, int NT>
 __device__ __forceinline__ void nnp_load(const SweepArgs &a, const NnpLds &L, int slot)
 {
     const NnpTables &T = a.nnp;
     const float *gX = reinterpret_cast<const float *>(a.coords) + (size_t)slot * 3 * NP;
     const int tid = threadIdx.x;
-    for (int e = tid; e < 3 * NP; e += NNP_NT) L.X[e] = gX[e];
-    for (int e = tid; e < T.nf * T.h1; e += NNP_NT) L.W1[e] = T.w1[e];
-    for (int e = tid; e < 4 * T.n_rad_active; e += NNP_NT) L.rad[e] = T.rad[e];
-    for (int e = tid; e < NNP_GD * T.n_groups; e += NNP_NT) L.gd[e] = T.gdesc[e];
-    for (int e = tid; e < (NNP_NT / 64) * (NNP_WG + 1); e += NNP_NT) L.wg[e] = T.wgroups[e];
-    for (int e = tid; e < T.h1 * T.h2; e += NNP_NT) L.W2[e] = T.w2[e];
-    for (int e = tid; e < NNP_MAXH; e += NNP_NT) {
+    for (int e = tid; e < 3 * NP; e += NT) L.X[e] = gX[e];
+    for (int e = tid; e < T.nf * T.h1; e += NT) L.W1[e] = T.w1[e];
+    for (int e = tid; e < 4 * T.n_rad_active; e += NT) L.rad[e] = T.rad[e];
+    for (int e = tid; e < NNP_GD * T.n_groups; e += NT) L.gd[e] = T.gdesc[e];
+    for (int e = tid; e < (NNP_NT / 64) * (NNP_WG + 1); e += NT) L.wg[e] = T.wgroups[e];
+    for (int e = tid; e < T.h1 * T.h2; e += NT) L.W2[e] = T.w2[e];
+    for (int e = tid; e < NNP_MAXH; e += NT) {
         L.B[e] = e < T.h1 ? T.b1[e] : 0.0f;
         L.B[NNP_MAXH + e] = e < T.h2 ? T.b2[e] : 0.0f;
         L.B[2 * NNP_MAXH + e] = e < T.h2 ? T.w3[e] : 0.0f;
@@ -490,8 +497,8 @@ __device__ __forceinline__ void nnp_load(const SweepArgs &a, const NnpLds &L, in
 
 // set_variables + initialise_energy (src/EnergyEvaluation.jl:1812-1822,
 // :1735-1747): features, per-atom energies and the FP64 total of each slot.
-template <int NP>
-__global__ void __launch_bounds__(NNP_NT) nnp_init_kernel(SweepArgs a)
+template <int NP, int NT>
+__global__ void __launch_bounds__(NT) nnp_init_kernel(SweepArgs a)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     const NnpTables &T = a.nnp;
@@ -501,14 +508,14 @@ __global__ void __launch_bounds__(NNP_NT) nnp_init_kernel(SweepArgs a)
     NnpLds L = nnp_lds<NP>(reinterpret_cast<float *>(lds_raw), T.nf, T.h1);
     NNP_BIND_TABLES(L);
     const int N = a.runs[a.slot_run[slot]].n_atoms;
-    nnp_load<NP>(a, L, slot);
+    nnp_load<NP, NT>(a, L, slot);
     __syncthreads();
-    nnp_full_build<NP>(T, L, L.G, N);
+    nnp_full_build<NP, NT>(T, L, L.G, N);
     __shared__ double s_tot;
-    nnp_forward<NP>(T, L, L.G, N, L.eat, &s_tot);
+    nnp_forward<NP, NT>(T, L, L.G, N, L.eat, &s_tot);
     float *gG = a.feat + (size_t)slot * T.nf * NP;
-    for (int e = threadIdx.x; e < T.nf * NP; e += NNP_NT) gG[e] = L.G[e];
-    for (int e = threadIdx.x; e < NP; e += NNP_NT) a.eatom[(size_t)slot * NP + e] = e < N ? L.eat[e] : 0.0f;
+    for (int e = threadIdx.x; e < T.nf * NP; e += NT) gG[e] = L.G[e];
+    for (int e = threadIdx.x; e < NP; e += NT) a.eatom[(size_t)slot * NP + e] = e < N ? L.eat[e] : 0.0f;
     if (threadIdx.x == 0) a.slot_en[slot] = s_tot;
 }
 
@@ -516,26 +523,33 @@ __global__ void __launch_bounds__(NNP_NT) nnp_init_kernel(SweepArgs a)
 // (mc_step!, src/MCRun.jl:169-182, with energy_update!(RuNNerPotential)).
 // DA: delayed acceptance with the learned surrogate (one workgroup per CU by
 // LDS, so the register budget is relaxed for that variant).  NP: atoms of a
-// slot, 64 (two workgroups per CU) or 128 (one; the near atoms of a move are
-// then up to 127, their partner masks two words, and the angular targets are
-// taken in chunks of 64 lanes).
+// slot, 64 or 128 (the near atoms of a move are then up to 127, their partner
+// masks two words).  NT: 512 threads, or 1024 where a workgroup has a CU to
+// itself (always with NP = 128): the second half's waves own the same groups as
+// the first's and take every other target, their sums at the moved atom are
+// added after the visits.
 //
 // Bound by instruction issue in the angular visits (a 55-atom move visits about
-// 1000 triangles from two of their atoms, once per wave): 28,000 of a move's
-// 51,000 cycles with one workgroup on a CU.  A visit's instructions went from
-// about 330 to 190: the lane's share of the partners is cut from the mask once
-// per target (not popped past on every visit), cosines from unit vectors in
-// place of IEEE divides and roots, one squaring chain for both groups of a
-// wave, no select per slot.  Store: sums merged across rows before they are
-// summed, 20 wave sums as 6 row sums.  Cycle of 40 temperatures x 55 atoms
-// (8 + 80 functions) 2.07 ms -> 1.21, of 1280 configurations 6.9 -> 4.0, of 20 x
-// 78 atoms 3.0 -> 1.97.
-template <bool DA, int NP>
-__global__ void __launch_bounds__(NNP_NT) __attribute__((amdgpu_waves_per_eu((DA || NP > NNP_NP) ? 2 : 4)))
+// 1000 triangles from two of their atoms, once per group pair): 28,000 of a
+// move's 51,000 cycles with one workgroup of 512 threads on a CU.  A visit's
+// instructions went from about 330 to 190: the lane's share of the partners is
+// cut from the mask once per target (not popped past on every visit), cosines
+// from unit vectors in place of IEEE divides and roots, one squaring chain for
+// both groups of a wave, no select per slot.  Store: sums merged across rows
+// before they are summed, 20 wave sums as 6 row sums, and the lanes of a target
+// added by one fma each.  us per cycle of 40 temperatures x 55 atoms (8 + 80
+// functions) 2070 before, 1210 so, 1117 on 1024 threads; of 1280 configurations
+// 6900, 3950, 3740 with the visits split by their terms; of 20 x 78 atoms 3000,
+// 1970, 1665 on 1024 threads.
+template <bool DA, int NP, int NT>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(DA ? 2 : 4)))
 nnp_sweep_kernel(SweepArgs a)
 {
-    static_assert(NP == NNP_NP || (NP == NNP_NP_WIDE && !DA), "slots of 64 atoms, or 128 without the surrogate");
+    static_assert(NT == NNP_NT || (NT == 2 * NNP_NT && !DA), "one or two workgroup halves");
+    static_assert(NP == NNP_NP || (NP == NNP_NP_WIDE && NT == 2 * NNP_NT), "the targets of a half fit a wave");
+    constexpr int SETS = NT / NNP_NT;  // halves of the workgroup, each with every other near atom as its targets
     constexpr int NW = NP / 64;  // 64-bit words of an atom mask
+    constexpr bool SPLIT = NW == 1;  // visits with and without the terms at i apart
     extern __shared__ __align__(16) unsigned char lds_raw[];
     __shared__ int s_flag, s_err, s_nnear;
     __shared__ uint64_t s_wmask[NW];
@@ -559,10 +573,10 @@ nnp_sweep_kernel(SweepArgs a)
     const float delta_r = (float)a.t_displ[2 * Tg];
     const float radius2 = (float)ri.radius2;
 
-    nnp_load<NP>(a, L, slot);
+    nnp_load<NP, NT>(a, L, slot);
     const float *gG = a.feat + (size_t)slot * T.nf * NP;
-    for (int e = tid; e < T.nf * NP; e += NNP_NT) L.G[e] = gG[e];
-    for (int e = tid; e < NP; e += NNP_NT) L.eat[e] = a.eatom[(size_t)slot * NP + e];
+    for (int e = tid; e < T.nf * NP; e += NT) L.G[e] = gG[e];
+    for (int e = tid; e < NP; e += NT) L.eat[e] = a.eatom[(size_t)slot * NP + e];
     double E = a.slot_en[slot];
     if (tid == 0) s_err = 0;
     // delayed acceptance: surrogate descriptors and atom energies in LDS
@@ -588,9 +602,9 @@ nnp_sweep_kernel(SweepArgs a)
         net.b2 = net.b1 + SUR_H;
         net.w3 = net.b2 + SUR_H;
         sgeo = net.w3 + SUR_H;  // per atom: r_new, r_old, f_c(r_new), f_c(r_old)
-        sur_load_net(net, a.sur_w, NNP_NT);
-        sur_descriptors(sg, L.X, N, Sd, SUR_SS, NNP_NT);
-        for (int e = tid; e < NP * SUR_SS; e += NNP_NT) Sn[e] = 0.0f;
+        sur_load_net(net, a.sur_w, NT);
+        sur_descriptors(sg, L.X, N, Sd, SUR_SS, NT);
+        for (int e = tid; e < NP * SUR_SS; e += NT) Sn[e] = 0.0f;
         __syncthreads();
         sur_atom_energies(net, Sd, N, L.H1, sat, &s_ehat);
         Ehat = s_ehat;
@@ -600,6 +614,12 @@ nnp_sweep_kernel(SweepArgs a)
     // current features and the scratch that becomes the trial features; an
     // accepted move swaps the two (swap_vars!(NNPVariables), src/swap_config.jl:213-221)
     float *Gp = L.G, *Dp = L.D;
+    // scratch in H1 until the network pass: partner masks [near atom][NW words],
+    // lane tables of the waves, and with two halves their sums at the moved atom
+    uint64_t *s_mask = reinterpret_cast<uint64_t *>(L.H1);
+    uint16_t *s_lt = reinterpret_cast<uint16_t *>(L.H1 + 2 * NW * NP) + 64 * (tid >> 6);
+    float *s_col = L.H1 + 2 * NW * NP + 32 * (NT / 64);
+    static_assert(2 * NW * NP + 32 * (NT / 64) + (SETS > 1 ? SETS * NNP_MAXF : 0) <= NP * NNP_HS, "H1 holds the scratch");
     // 16-byte aligned by its offset, so that the compiler still sees an LDS
     // address (a pointer through an integer is read with flat loads)
     float *nb_base = reinterpret_cast<float *>(lds_raw) + (((int)(L.H2 - reinterpret_cast<float *>(lds_raw)) + 3) & ~3);
@@ -717,8 +737,9 @@ nnp_sweep_kernel(SweepArgs a)
         }
         // trial features start as the current ones; every changed entry is
         // written once, as current plus change
-        for (int e = tid; e < T.nf * NP / 4; e += NNP_NT)
+        for (int e = tid; e < T.nf * NP / 4; e += NT)
             reinterpret_cast<float4 *>(Dp)[e] = reinterpret_cast<const float4 *>(Gp)[e];
+        if (SETS > 1 && tid < SETS * NNP_MAXF) s_col[tid] = 0.0f;
         if (da && tid < SUR_K) s_acci[tid] = 0.0f;
         __syncthreads();
         // delayed acceptance, stage 1: Metropolis on the surrogate energy change
@@ -735,9 +756,9 @@ nnp_sweep_kernel(SweepArgs a)
             }
             __syncthreads();
             float accq = 0.0f;
-            const int kq = tid & (SUR_K - 1);  // NNP_NT is a multiple of SUR_K: fixed k per thread
+            const int kq = tid & (SUR_K - 1);  // NT is a multiple of SUR_K: fixed k per thread
             const float mu = sur_mu(sg, kq);
-            for (int j = tid / SUR_K; j < N; j += NNP_NT / SUR_K) {
+            for (int j = tid / SUR_K; j < N; j += NT / SUR_K) {
                 if (j == i) continue;
                 const float fcn = sgeo[2 * NP + j], fco = sgeo[3 * NP + j];
                 const float pn = sur_phi_mu(sg, sgeo[j], fcn, mu);
@@ -766,7 +787,7 @@ nnp_sweep_kernel(SweepArgs a)
             }
             // radial changes, DeltaMatrix.jl:794-822: one wave per function,
             // one lane per atom (NW atoms per lane in the wide layout)
-            for (int q = tid >> 6; q < T.n_rad_active; q += NNP_NT / 64) {
+            for (int q = tid >> 6; q < T.n_rad_active; q += NT / 64) {
                 const float eta = L.rad[4 * q], norm = L.rad[4 * q + 1];
                 const int row = (int)L.rad[4 * q + 2];
                 float dsum = 0.0f;
@@ -792,10 +813,8 @@ nnp_sweep_kernel(SweepArgs a)
             // feature entry is written by one lane with a plain store: no LDS
             // atomics (float LDS adds run far below the store rate).
             const int n_near = s_nnear;
-            // partner masks [near atom][NW words] (scratch until the network pass)
-            uint64_t *s_mask = reinterpret_cast<uint64_t *>(L.H1);
             const float rc2 = T.r_cut * T.r_cut * 1.0001f;  // loose: the cut-off function decides below
-            for (int a = tid >> 6; a < n_near; a += NNP_NT / 64) {
+            for (int a = tid >> 6; a < n_near; a += NT / 64) {
                 const float4 pa = nb_a[a];
                 const float foa = nb_b[a].z;
 #pragma unroll
@@ -814,32 +833,27 @@ nnp_sweep_kernel(SweepArgs a)
                 }
             }
             __syncthreads();
-            // Targets in chunks of 64 near atoms; per chunk, lanes per target:
-            // target a gets P_a = 1, 2, 4 or 8 lanes, the fewest that bring its
-            // share of visits down to the load T, T the smallest load for which
-            // the shares fit 64 lanes (bisection, the lane count summed by
-            // ballots).  Blocks of P lanes are laid out by P (8, 4, 2, 1), so
-            // each is aligned for the quad and half-row exchanges that combine
-            // them.  Every wave builds the same tables in its own LDS slice (no
-            // barrier needed within a wave).
-            uint16_t *s_lt = reinterpret_cast<uint16_t *>(L.H1 + 2 * NW * NP) + NP * (tid >> 6);
-            const int nch = (n_near + 63) >> 6;
-            int used_c[NW];
-#pragma unroll
-            for (int c = 0; c < NW; ++c) {
-                used_c[c] = 0;
-                if (c >= nch) continue;
-                const int nc = n_near - 64 * c < 64 ? n_near - 64 * c : 64;
+            // Lanes per target: target a gets P_a = 1, 2, 4 or 8 lanes, the fewest
+            // that bring its share of visits down to the load T, T the smallest
+            // load for which the shares fit 64 lanes (bisection, the lane count
+            // summed by ballots).  Blocks of P lanes are laid out by P (8, 4, 2,
+            // 1), so each is aligned for the quad and half-row exchanges that
+            // combine them.  Every wave builds the same tables (of its half's
+            // targets) in its own LDS slice: no barrier needed within a wave.
+            // uniform over the wave, and said so: the loops over groups and
+            // powers then branch on scalars
+            const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+            const int set = w / (NNP_NT / 64), wl = w % (NNP_NT / 64);
+            const int nc = (n_near - set + SETS - 1) / SETS;  // entry e: near atom SETS e + set
+            int used = 0;
+            {
                 int La = 0;
                 if (lane < nc) {
 #pragma unroll
-                    for (int v = 0; v < NW; ++v) La += __popcll(s_mask[(64 * c + lane) * NW + v]);
+                    for (int v = 0; v < NW; ++v) La += __popcll(s_mask[(SETS * lane + set) * NW + v]);
                 }
                 // lanes of a target at load T: 1 up to T visits, 2 up to 2 T,
                 // 4 up to 4 T, else 8; their sum over the targets
-                auto lanes_for = [&](int load) {
-                    return lane >= nc ? 0 : (La <= load ? 1 : (La <= 2 * load ? 2 : (La <= 4 * load ? 4 : 8)));
-                };
                 auto lanes_used = [&](int load) {
                     return nc + __popcll(__ballot(La > load)) + 2 * __popcll(__ballot(La > 2 * load)) +
                            4 * __popcll(__ballot(La > 4 * load));
@@ -850,99 +864,109 @@ nnp_sweep_kernel(SweepArgs a)
                     if (lanes_used(mid) <= 64) hi = mid;
                     else lo = mid + 1;
                 }
-                const int Pa = lanes_for(lo);
-                int used = 0;
+                const int Pa = lane >= nc ? 0 : (La <= lo ? 1 : (La <= 2 * lo ? 2 : (La <= 4 * lo ? 4 : 8)));
 #pragma unroll
                 for (int cc = 3; cc >= 0; --cc) {
                     const bool in = Pa == (1 << cc);
                     const uint64_t b = __ballot(in);
                     if (in)
                         for (int q = 0; q < Pa; ++q)
-                            s_lt[64 * c + used + (mbcnt64(b) << cc) + q] = (uint16_t)(lane | (q << 6) | (cc << 9));
+                            s_lt[used + (mbcnt64(b) << cc) + q] = (uint16_t)(lane | (q << 6) | (cc << 9));
                     used += __popcll(b) << cc;
                 }
-                used_c[c] = used;
             }
-            // this lane's target in chunk c: lanes, part, atom, the partners of
-            // its part (and those of larger list index, the visits that also carry the
-            // terms centred on i), packed data
+            // this lane's target: lanes, part, atom, the partners of its part with
+            // which the visit also carries the terms centred on i (o) and the
+            // others (m), packed data.  Of the n near atoms in a circle, a target
+            // carries those terms for the (n - 1) / 2 after it (and of an opposite
+            // pair the first does): every target for about half of its partners,
+            // so the lanes of a wave do such visits together, and then the
+            // others.  Slots of 128 atoms go through all partners at once and
+            // test each (o holds the circle): with two mask words and 26 functions
+            // the cut costs more than it saves (20 x 78 atoms 1.83 ms split, 1.66
+            // so; 1280 x 55 atoms, 88 functions, 3.95 unsplit, 3.72 split).
             struct Target {
                 int lp, part, j;
                 bool tact;
-                uint64_t m0, m1, after0, after1;
+                uint64_t m0, m1, o0, o1;
                 float4 ja, jb, ju, jv;
             };
-            auto target = [&](int c) {
+            auto target = [&]() {
                 Target g;
-                const int ent = lane < used_c[c] ? (int)s_lt[64 * c + lane] : 0;
+                const int ent = lane < used ? (int)s_lt[lane] : 0;
                 g.lp = ent >> 9;
-                const int ta = 64 * c + (ent & 63);
+                const int ta = SETS * (ent & 63) + set;
                 g.part = (ent >> 6) & 7;
-                g.tact = lane < used_c[c];
+                g.tact = lane < used;
                 g.j = g.tact ? (int)s_near[ta] : 0;
-                g.m0 = g.tact ? s_mask[ta * NW] : 0ull;
-                g.m1 = 0ull;
-                g.after0 = ta < 63 ? ~((2ull << ta) - 1ull) : 0ull;
-                g.after1 = 0ull;
-                if constexpr (NW > 1) {
-                    g.m1 = g.tact ? s_mask[ta * NW + 1] : 0ull;
-                    const int sh = ta - 64;
-                    g.after1 = sh < 0 ? ~0ull : (sh < 63 ? ~((2ull << sh) - 1ull) : 0ull);
-                }
-                // the part's share: equal counts, by rank among the partners
-                const int n0 = __popcll(g.m0), n = n0 + (NW > 1 ? __popcll(g.m1) : 0);
-                const int r0 = (g.part * n) >> g.lp, r1 = ((g.part + 1) * n) >> g.lp;
-                auto cut_word = [](uint64_t m, int c, int a, int b) {  // bits of rank a .. b - 1 of c
-                    a = a < 0 ? 0 : (a < c ? a : c);
-                    b = b < 0 ? 0 : (b < c ? b : c);
-                    return nnp_drop(m, a) & ~nnp_drop(m, b);
+                uint64_t m0 = g.tact ? s_mask[ta * NW] : 0ull, m1 = 0ull;
+                if constexpr (NW > 1) m1 = g.tact ? s_mask[ta * NW + 1] : 0ull;
+                // list indices ta + 1 .. ta + h round the circle of n_near
+                const int h = (n_near - 1) / 2 + (((n_near & 1) == 0 && 2 * ta < n_near) ? 1 : 0);
+                const int end = ta + 1 + h;  // past n_near: the rest from 0
+                auto below = [](int b, int word) {  // bits of a word whose index is below b
+                    const int k = b - 64 * word;
+                    return k <= 0 ? 0ull : (k >= 64 ? ~0ull : (1ull << k) - 1ull);
                 };
-                if constexpr (NW > 1) g.m1 = cut_word(g.m1, n - n0, r0 - n0, r1 - n0);
-                g.m0 = cut_word(g.m0, n0, r0, r1);
+                auto circle = [&](int word) {
+                    const uint64_t up = below(end, word) & ~below(ta + 1, word);
+                    return end > n_near ? up | below(end - n_near, word) : up;
+                };
+                const uint64_t c0 = circle(0), c1 = NW > 1 ? circle(1) : 0ull;
+                g.o0 = SPLIT ? m0 & c0 : c0;
+                g.o1 = SPLIT ? m1 & c1 : c1;
+                g.m0 = SPLIT ? m0 & ~c0 : m0;
+                g.m1 = SPLIT ? m1 & ~c1 : m1;
+                // the part's share: equal counts, by rank among the partners
+                auto share = [&](uint64_t &a0, uint64_t &a1, int part) {
+                    const int n0 = __popcll(a0), n = n0 + (NW > 1 ? __popcll(a1) : 0);
+                    const int r0 = (part * n) >> g.lp, r1 = ((part + 1) * n) >> g.lp;
+                    auto cut_word = [](uint64_t m, int c, int a, int b) {  // bits of rank a .. b - 1 of c
+                        a = a < 0 ? 0 : (a < c ? a : c);
+                        b = b < 0 ? 0 : (b < c ? b : c);
+                        return nnp_drop(m, a) & ~nnp_drop(m, b);
+                    };
+                    if constexpr (NW > 1) a1 = cut_word(a1, n - n0, r0 - n0, r1 - n0);
+                    a0 = cut_word(a0, n0, r0, r1);
+                };
+                if constexpr (SPLIT) share(g.o0, g.o1, g.part);
+                share(g.m0, g.m1, g.part);
                 g.ja = nb_a[ta];
                 g.jb = nb_b[ta];
                 g.ju = nb_u[ta];
                 g.jv = nb_v[ta];
                 return g;
             };
-            Target t1{};
-            if constexpr (NW == 1) t1 = target(0);  // one chunk: read once for all group passes
-            // uniform over the wave, and said so: the functions' masks then
-            // branch instead of selecting every accumulator
-            const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-            const int ngw = __builtin_amdgcn_readfirstlane(L.wg[w * (NNP_WG + 1)]);
+            const Target tg = target();  // read once for all group passes
+            const int ngw = __builtin_amdgcn_readfirstlane(L.wg[wl * (NNP_WG + 1)]);
             for (int gi = 0; gi < ngw; gi += 2) {
                 // up to two groups per pass over the visits
-                const int ga = __builtin_amdgcn_readfirstlane(L.wg[w * (NNP_WG + 1) + 1 + gi]);
-                const int gb = gi + 1 < ngw ? __builtin_amdgcn_readfirstlane(L.wg[w * (NNP_WG + 1) + 2 + gi]) : -1;
+                const int ga = __builtin_amdgcn_readfirstlane(L.wg[wl * (NNP_WG + 1) + 1 + gi]);
+                const int gb = gi + 1 < ngw ? __builtin_amdgcn_readfirstlane(L.wg[wl * (NNP_WG + 1) + 2 + gi]) : -1;
                 NnpGroup G0, G1;
                 nnp_group(L.gd, ga, G0);
                 if (gb >= 0) nnp_group(L.gd, gb, G1);
                 else G1.none();
                 const int top_p = G0.top[0] > G1.top[0] ? G0.top[0] : G1.top[0];
                 const int top_m = G0.top[1] > G1.top[1] ? G0.top[1] : G1.top[1];
-#pragma unroll
-                for (int c = 0; c < NW; ++c) {
-                    if (c >= nch) continue;
-                    const Target tg = NW == 1 ? t1 : target(c);
+                {
                     const float4 ja = tg.ja, jb = tg.jb, ju = tg.ju, jv = tg.jv;
                     float aj0[NNP_GMAX], ai0[NNP_GMAX], aj1[NNP_GMAX], ai1[NNP_GMAX];
 #pragma unroll
                     for (int q = 0; q < NNP_GMAX; ++q) aj0[q] = ai0[q] = aj1[q] = ai1[q] = 0.0f;
-                    auto visits = [&](auto two) {
+                    auto visits = [&](auto two, auto own, uint64_t m0, uint64_t m1) {
                         constexpr bool TWO = decltype(two)::value;
-                        uint64_t m0 = tg.m0, m1 = tg.m1;
                         while (NW == 1 ? m0 != 0ull : (m0 | m1) != 0ull) {
                             int bk;
-                            bool own;
+                            bool at_i = decltype(own)::value;
                             if (NW == 1 || m0 != 0ull) {
                                 bk = __builtin_ctzll(m0);
                                 m0 &= m0 - 1ull;
-                                own = ((tg.after0 >> bk) & 1ull) != 0ull;
+                                if (!SPLIT) at_i = ((tg.o0 >> bk) & 1ull) != 0ull;
                             } else {
                                 bk = __builtin_ctzll(m1);
                                 m1 &= m1 - 1ull;
-                                own = ((tg.after1 >> bk) & 1ull) != 0ull;
+                                if (!SPLIT) at_i = ((tg.o1 >> bk) & 1ull) != 0ull;
                                 bk += 64;
                             }
                             const float4 ka = nb_a[bk], kb = nb_b[bk];
@@ -964,7 +988,7 @@ nnp_sweep_kernel(SweepArgs a)
                                 eo1 = -(__builtin_amdgcn_exp2f(-G1.eta2 * rso) * fpo);
                             }
                             nnp_terms<TWO>(top_p, top_m, cjn, cjo, en0, eo0, en1, eo1, aj0, aj1);
-                            if (own) {
+                            if (at_i) {
                                 // and at i
                                 const float4 ku = nb_u[bk], kv = nb_v[bk];
                                 const float cin = __builtin_fmaf(ju.z, ku.z, __builtin_fmaf(ju.y, ku.y, ju.x * ku.x));
@@ -975,16 +999,28 @@ nnp_sweep_kernel(SweepArgs a)
                     };
                     const bool writer = tg.tact && tg.part == 0;
                     if (gb >= 0) {
-                        visits(std::true_type{});
-                        nnp_store<NP>(G1, L.gd + NNP_GD * gb, tg.lp, writer, tg.j, i, lane, Dp, aj1, ai1);
+                        if constexpr (SPLIT) visits(std::true_type{}, std::true_type{}, tg.o0, tg.o1);
+                        visits(std::true_type{}, std::false_type{}, tg.m0, tg.m1);
+                        nnp_store<NP, SETS>(G1, L.gd + NNP_GD * gb, tg.lp, writer, tg.j, i, lane, Dp, s_col + set * NNP_MAXF, aj1, ai1);
                     } else {
-                        visits(std::false_type{});
+                        if constexpr (SPLIT) visits(std::false_type{}, std::true_type{}, tg.o0, tg.o1);
+                        visits(std::false_type{}, std::false_type{}, tg.m0, tg.m1);
                     }
-                    nnp_store<NP>(G0, L.gd + NNP_GD * ga, tg.lp, writer, tg.j, i, lane, Dp, aj0, ai0);
+                    nnp_store<NP, SETS>(G0, L.gd + NNP_GD * ga, tg.lp, writer, tg.j, i, lane, Dp, s_col + set * NNP_MAXF, aj0, ai0);
                 }
             }
             __syncthreads();
-            nnp_forward<NP>(T, L, Dp, N, L.eatn, &s_en);
+            if constexpr (SETS > 1) {
+                // the halves' sums at the moved atom, one after the other
+                if (tid < T.nf) {
+                    float d = Dp[tid * NP + i];
+#pragma unroll
+                    for (int v = 0; v < SETS; ++v) d += s_col[v * NNP_MAXF + tid];
+                    Dp[tid * NP + i] = d;
+                }
+                __syncthreads();
+            }
+            nnp_forward<NP, NT>(T, L, Dp, N, L.eatn, &s_en);
             new_en = s_en;
         }
         // Metropolis, src/MCRun.jl:122-132 and src/Exchange.jl:53-57; with
@@ -1013,7 +1049,7 @@ nnp_sweep_kernel(SweepArgs a)
             float *tmp = Gp;
             Gp = Dp;
             Dp = tmp;
-            for (int e = tid; e < N; e += NNP_NT) L.eat[e] = L.eatn[e];
+            for (int e = tid; e < N; e += NT) L.eat[e] = L.eatn[e];
             if (da) {
                 float *t1 = Sd;
                 Sd = Sn;
@@ -1036,8 +1072,8 @@ nnp_sweep_kernel(SweepArgs a)
 
     // periodic full rebuild bounds the drift of the incremental features
     if (a.recompute_every > 0 && ((long long)sweep + 1) % a.recompute_every == 0) {
-        nnp_full_build<NP>(T, L, Gp, N);
-        nnp_forward<NP>(T, L, Gp, N, L.eat, &s_en);
+        nnp_full_build<NP, NT>(T, L, Gp, N);
+        nnp_forward<NP, NT>(T, L, Gp, N, L.eat, &s_en);
         const double dr = __builtin_fabs(E - s_en);
         if (tid == 0 && dr > a.slot_drift[slot]) a.slot_drift[slot] = dr;
         E = s_en;
@@ -1045,9 +1081,9 @@ nnp_sweep_kernel(SweepArgs a)
 
     float *gX = reinterpret_cast<float *>(a.coords) + (size_t)slot * 3 * NP;
     float *gGw = a.feat + (size_t)slot * T.nf * NP;
-    for (int e = tid; e < 3 * NP; e += NNP_NT) gX[e] = L.X[e];
-    for (int e = tid; e < T.nf * NP; e += NNP_NT) gGw[e] = Gp[e];
-    for (int e = tid; e < NP; e += NNP_NT) a.eatom[(size_t)slot * NP + e] = L.eat[e];
+    for (int e = tid; e < 3 * NP; e += NT) gX[e] = L.X[e];
+    for (int e = tid; e < T.nf * NP; e += NT) gGw[e] = Gp[e];
+    for (int e = tid; e < NP; e += NT) a.eatom[(size_t)slot * NP + e] = L.eat[e];
     if (tid == 0) {
         a.slot_en[slot] = E;
         a.t_count_atom[2 * Tg] += nacc;

@@ -22,10 +22,13 @@ import paralleltemperingmontecarlo as pt  # noqa: E402
 from paralleltemperingmontecarlo.api import NeuralNetworkPotential, PTEngine, RuNNerPotential  # noqa: E402
 from paralleltemperingmontecarlo.nnp_setup import synthetic_cu55_potential  # noqa: E402
 
-# atoms, radial and angular functions kept, hidden widths, how far apart the atoms are
-SHAPES = [(2, 1, 1, 1, 1, 4.5), (3, 8, 80, 20, 20, 4.5), (15, 2, 5, 16, 17, 4.8), (16, 8, 26, 17, 16, 4.8),
+# atoms, radial and angular functions kept, hidden widths, how far apart the atoms are, temperatures (above 256
+# the slots of 33 to 64 atoms take 512 threads)
+SHAPES = [s + (2,) for s in (
+          (2, 1, 1, 1, 1, 4.5), (3, 8, 80, 20, 20, 4.5), (15, 2, 5, 16, 17, 4.8), (16, 8, 26, 17, 16, 4.8),
           (17, 5, 33, 32, 32, 4.8), (33, 3, 60, 20, 5, 9.0), (49, 8, 80, 20, 20, 5.4), (63, 1, 80, 31, 20, 4.8),
-          (64, 8, 79, 20, 20, 4.8), (65, 4, 22, 20, 20, 4.8), (97, 8, 26, 16, 32, 5.4), (128, 2, 9, 20, 17, 4.8)]
+          (64, 8, 79, 20, 20, 4.8), (65, 4, 22, 20, 20, 4.8), (97, 8, 26, 16, 32, 5.4), (128, 2, 9, 20, 17, 4.8))]
+SHAPES.append((34, 2, 9, 20, 17, 4.8, 258))
 
 
 def _cluster(n, spacing, seed):
@@ -36,8 +39,8 @@ def _cluster(n, spacing, seed):
     return np.ascontiguousarray((x - x.mean(0)).astype(np.float32).astype(np.float64))
 
 
-@pytest.mark.parametrize("n,n_rad,n_ang,h1,h2,spacing", SHAPES)
-def test_moves_at_tile_edges(oracle, n, n_rad, n_ang, h1, h2, spacing):
+@pytest.mark.parametrize("n,n_rad,n_ang,h1,h2,spacing,R", SHAPES)
+def test_moves_at_tile_edges(oracle, n, n_rad, n_ang, h1, h2, spacing, R):
     full = synthetic_cu55_potential(GOLDEN / "nnp" / "scaling.data")
     nf = n_rad + n_ang
     n_par = nf * h1 + h1 + h1 * h2 + h2 + h2 + 1
@@ -45,7 +48,7 @@ def test_moves_at_tile_edges(oracle, n, n_rad, n_ang, h1, h2, spacing):
     pot = RuNNerPotential(NeuralNetworkPotential([nf, h1, h2, 1], [1, 2, 2, 1], w), full.radsymfunctions[:n_rad],
                           full.angsymfunctions[:n_ang])
     scale = n * (abs(w[-1]) + np.abs(w[-1 - h2:-1]).sum())
-    R, ncyc = 2, 2 if n < 40 else 1
+    ncyc = 2 if n < 34 else 1
     x0, radius = _cluster(n, spacing, 100 + n), 45.0
     temp = pt.TempGrid(300.0, 30000.0, R)
     eng = PTEngine(pot, pt.NVT(n), pt.SphericalBC(radius), pt.MCParams(10, R, n, n_adjust=5),
