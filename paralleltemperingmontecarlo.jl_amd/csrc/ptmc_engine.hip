@@ -32,7 +32,7 @@ SweepFn nnp2_sweep_fn(bool pow);
 SweepFn nnp2_init_fn(bool pow);
 SweepFn nnp2_sweep_fn_f32(bool pow);
 SweepFn nnp2_init_fn_f32(bool pow);
-void (*nnp_cycle_fn())(SweepArgs, int);
+SweepFn nnp_cycle_fn();
 hipError_t sur_launch_desc(const float *x, const int32_t *n_atoms, float *bd, float r_cut, int n, hipStream_t st);
 hipError_t sur_launch_collect(const SweepArgs &a, int n_slots, float *bd, double *be, int32_t *bn, long long base,
                               int cap, hipStream_t st);
@@ -1896,8 +1896,8 @@ int ptmc_cycles(ptmc_handle h, int64_t n_cycles)
                 a.trace_cycle = (int32_t)c;
             }
             if ((rc = launch_one(h, 0, a, h->stream, false))) return rc;
-            void *args[] = {&a, &n_runs};
-            HIPCHK(h, hipLaunchKernel((const void *)nnp_cycle_fn(), dim3((n_runs + 63) / 64), dim3(64), args, 0,
+            void *args[] = {&a};
+            HIPCHK(h, hipLaunchKernel((const void *)nnp_cycle_fn(), dim3(n_runs), dim3(64), args, 0,
                                       h->stream));
             if (h->sur.init && h->sur.collect_every > 0 && (h->sweep_counter + 1) % h->sur.collect_every == 0) {
                 HIPCHK(h, sur_launch_collect(a, h->n_slots, h->d_sur_D.p, h->d_sur_E.p, h->d_sur_N.p, h->sur.n_samples,

@@ -18,6 +18,6 @@ SweepFn nnp_init_fn(int np, int nt)
     if (np > NNP_NP) return &nnp_init_kernel<NNP_NP_WIDE, 2 * NNP_NT>;
     return nt > NNP_NT ? &nnp_init_kernel<NNP_NP, 2 * NNP_NT> : &nnp_init_kernel<NNP_NP, NNP_NT>;
 }
-void (*nnp_cycle_fn())(SweepArgs, int) { return &nnp_cycle_kernel; }
+SweepFn nnp_cycle_fn() { return &nnp_cycle_kernel; }
 
 }  // namespace ptmc

@@ -1099,12 +1099,14 @@ nnp_sweep_kernel(SweepArgs a)
 
 // Between cycles: replica exchange (src/Exchange.jl:103-155, src/MCRun.jl:203-205),
 // step adaptation (src/Exchange.jl:198-263) and sampling (src/Sampling.jl:330-371),
-// one thread per run.
-__global__ void nnp_cycle_kernel(SweepArgs a, int n_runs)
+// one wave per run: the pairs of an even/odd exchange are disjoint and go to
+// lanes, and so do the temperatures.  Bound by the latency of the dependent
+// reads of a pair (labels, slots, energies): one thread per run took 45 us for
+// 40 temperatures, 4 so.
+__global__ void __launch_bounds__(64) nnp_cycle_kernel(SweepArgs a)
 {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= n_runs) return;
-    const RunInfo &ri = a.runs[r];
+    const RunInfo &ri = a.runs[blockIdx.x];
+    const int lane = threadIdx.x;
     const int R = ri.n_temps, tb = ri.temp_base, N = ri.n_atoms;
     const uint32_t sweep = (uint32_t)a.sweep0;
     const long long pidx = a.cycle0 + 1;
@@ -1129,14 +1131,15 @@ __global__ void nnp_cycle_kernel(SweepArgs a, int n_runs)
     };
     if (R > 1 && (sweep + 1u) % (uint32_t)a.exchange_every == 0u) {
         if (a.exchange_mode == EXC_EVEN_ODD) {
-            for (int n = (int)(sweep & 1u); n + 1 < R; n += 2) try_pair(n);
-        } else {
+            for (int n = (int)(sweep & 1u) + 2 * lane; n + 1 < R; n += 128) try_pair(n);
+        } else if (lane == 0) {
             u32x4 X0 = draw(a.seed, ri.run_key, RNG_EXCH, 0u, 0u, sweep, 0u);
             const double u = u53(X0.x, X0.y);
             if (a.exchange_mode == EXC_EVERY || u < 0.1) try_pair((int)below(X0.z, (uint32_t)(R - 1)));
         }
     }
-    for (int t = 0; t < R; ++t) {
+    __syncthreads();  // the exchanged labels, before they are read by temperature
+    for (int t = lane; t < R; t += 64) {
         const int T = tb + t;
         if (pidx % a.n_adjust == 0) {
             const double ar = (double)a.t_count_atom[2 * T + 1] / (double)((long long)a.n_adjust * N);
