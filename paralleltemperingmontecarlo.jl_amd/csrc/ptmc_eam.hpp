@@ -28,6 +28,92 @@ __device__ __forceinline__ void eam_terms(Real r2, Real n, Real m, Real &phi, Re
     }
 }
 
+// FP64 terms of K distances together, bit for bit eam_terms' (the operations of
+// det_log and det_exp in their order) without their tests: squared distances are
+// normal and finite, and the exponents within +-700, or everything is done by
+// eam_terms.  The quotient has no scaling to undo (1.7 < 2 + f < 2.5, |f| < 0.5 and
+// zero or above 2^-53), so the Newton steps of a correctly rounded division do
+// alone, and 2^k is a normal number, so the product by it is one ldexp.
+//
+// Bound by FP64 issue.  det_exp's and det_log's range tests are 22 branches for
+// two distances, with every polynomial constant moved to a register in each: 800
+// instructions a partner; the 2 K chains side by side share the constants.  One
+// ladder of 32 x 55 atoms on 8 lanes 500 us a cycle before, 292 so.
+template <int K>
+__device__ __forceinline__ void eam_terms_n(const double (&r2)[K], double n, double m, double (&phi)[K], double (&rho)[K])
+{
+    bool ok = true;
+    double hl[K];
+#pragma unroll
+    for (int i = 0; i < K; ++i) ok = ok && r2[i] >= 0x1.0p-1022 && r2[i] < __longlong_as_double(0x7ff0000000000000ll);
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        const uint64_t b = (uint64_t)__double_as_longlong(r2[i]);
+        double x = __longlong_as_double((long long)((b & 0x000fffffffffffffull) | 0x3ff0000000000000ull));
+        const bool up = x > 1.4142135623730951;
+        const int e = (int)((b >> 52) & 0x7ff) - 1023 + (up ? 1 : 0);
+        x = up ? x * 0.5 : x;
+        const double f = x - 1.0, d = 2.0 + f;
+        double y = __builtin_amdgcn_rcp(d);
+        y = fma(fma(-d, y, 1.0), y, y);
+        y = fma(fma(-d, y, 1.0), y, y);
+        double s = f * y;
+        s = fma(fma(-d, s, f), y, s);
+        const double z = s * s;
+        double q = 1.0 / 21.0;
+        q = fma(q, z, 1.0 / 19.0);
+        q = fma(q, z, 1.0 / 17.0);
+        q = fma(q, z, 1.0 / 15.0);
+        q = fma(q, z, 1.0 / 13.0);
+        q = fma(q, z, 1.0 / 11.0);
+        q = fma(q, z, 1.0 / 9.0);
+        q = fma(q, z, 1.0 / 7.0);
+        q = fma(q, z, 1.0 / 5.0);
+        q = fma(q, z, 1.0 / 3.0);
+        const double two_s = 2.0 * s, lm = fma(two_s * z, q, two_s), ed = (double)e;
+        hl[i] = -0.5 * fma(ed, 6.93147180369123816490e-01, fma(ed, 1.90821492927058770002e-10, lm));
+    }
+    double r[2 * K], p[2 * K], kd[2 * K];
+#pragma unroll
+    for (int i = 0; i < 2 * K; ++i) {
+        const double x = (i < K ? n : m) * hl[i % K];
+        ok = ok && __builtin_fabs(x) <= 700.0;
+        kd[i] = rint(x * 1.4426950408889634);
+        r[i] = fma(-kd[i], 6.93147180369123816490e-01, x);
+        r[i] = fma(-kd[i], 1.90821492927058770002e-10, r[i]);
+        p[i] = 2.08767569878680989792e-09;
+    }
+    const double c[12] = {2.50521083854417187751e-08, 2.75573192239858906526e-07, 2.75573192239858906526e-06,
+                          2.48015873015873015873e-05, 1.98412698412698412698e-04, 1.38888888888888888889e-03,
+                          8.33333333333333333333e-03, 4.16666666666666666667e-02, 1.66666666666666666667e-01,
+                          0.5, 1.0, 1.0};
+#pragma unroll
+    for (int u = 0; u < 12; ++u)
+#pragma unroll
+        for (int i = 0; i < 2 * K; ++i) p[i] = fma(p[i], r[i], c[u]);
+    if (ok) {
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+            phi[i] = __builtin_amdgcn_ldexp(p[i], (int)kd[i]);
+            rho[i] = __builtin_amdgcn_ldexp(p[K + i], (int)kd[K + i]);
+        }
+    } else {
+#pragma unroll 1
+        for (int i = 0; i < K; ++i) {
+            double a, b;
+            double x = r2[0];
+#pragma unroll
+            for (int k = 1; k < K; ++k) x = i == k ? r2[k] : x;
+            eam_terms<double>(x, n, m, a, b);
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                phi[k] = i == k ? a : phi[k];
+                rho[k] = i == k ? b : rho[k];
+            }
+        }
+    }
+}
+
 // component slab: (buffer b, slab s, component c in {phi, rho}, lane)
 template <int LANES>
 __device__ __forceinline__ int coff(int A, int b, int s, int c, int lane)
@@ -59,10 +145,10 @@ __device__ double eam_build(const Real *X, Real *Cp, int A, int cur, int gb, int
             const int sl = l / KL, ll = gb + (l % KL);
             const double r2 = dist2_64(xj, yj, zj, (double)X[xoff<LANES>(sl, 0, ll)], (double)X[xoff<LANES>(sl, 1, ll)],
                                        (double)X[xoff<LANES>(sl, 2, ll)], BC, box, invL, false);
-            double pf, pg;
-            eam_terms<double>(r2, n, m, pf, pg);
-            f += pf;
-            g += pg;
+            double pf[1], pg[1];
+            eam_terms_n<1>({r2}, n, m, pf, pg);
+            f += pf[0];
+            g += pg[0];
         }
         Cp[coff<LANES>(A, cur, s, 0, gb + q)] = (Real)f;
         Cp[coff<LANES>(A, cur, s, 1, gb + q)] = (Real)g;
@@ -178,8 +264,18 @@ __global__ void __launch_bounds__(LANES) eam_kernel(SweepArgs a)
                     const Real r2n = dist2<Real, BC, false>(tx, ty, tz, xj, yj, zj, Lr, invLr);
                     const Real r2o = dist2<Real, BC, false>(xi, yi, zi, xj, yj, zj, Lr, invLr);
                     Real fn, gn, fo, go;
-                    eam_terms<Real>(r2n, nr, mr, fn, gn);
-                    eam_terms<Real>(r2o, nr, mr, fo, go);
+                    if constexpr (F32) {
+                        eam_terms<Real>(r2n, nr, mr, fn, gn);
+                        eam_terms<Real>(r2o, nr, mr, fo, go);
+                    } else {
+                        // the moved atom's own entry (distance 0) is not used: 1
+                        double f2[2], g2[2];
+                        eam_terms_n<2>({valid ? r2n : 1.0, valid ? r2o : 1.0}, nr, mr, f2, g2);
+                        fn = f2[0];
+                        fo = f2[1];
+                        gn = g2[0];
+                        go = g2[1];
+                    }
                     const Real t1 = valid ? fn - fo : Real(0);
                     const Real t2 = valid ? gn - go : Real(0);
                     const Real pj = Cp[coff<LANES>(A, cur, s, 0, tid)];
