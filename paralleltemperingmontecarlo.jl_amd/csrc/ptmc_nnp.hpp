@@ -4,10 +4,10 @@
 //
 // One workgroup owns one configuration for a whole cycle.  Its positions,
 // feature matrix G (nf x atoms) and per-atom energies live in LDS.  A move
-// builds the change D of G caused by moving atom i (radial terms by pair,
-// angular terms by partner pair (j, k) with the exponentials shared by all
-// functions of one eta), evaluates the network on G + D for every atom, and
-// on acceptance folds D into G.  Exchange, step adaptation and sampling run
+// builds the trial features D from G and the changes caused by moving atom i
+// (radial terms by pair, angular terms by partner pair (j, k) with the
+// exponentials shared by all functions of one eta), evaluates the network on D
+// for every atom, and on acceptance swaps D and G.  Exchange, step adaptation and sampling run
 // between cycles in nnp_cycle_kernel, so one launch of the sweep kernel is
 // one cycle of every configuration.
 #pragma once
