@@ -319,7 +319,8 @@ int default_lanes(int n_atoms, int precision)
 // a CU over the whole batch.  us per cycle at default_lanes / so: 32
 // temperatures x 13 atoms 40 / 14, x 20 45 / 23, x 38 90 / 60, 8 x 55 107 / 81;
 // 32 atoms in a cubic box at constant pressure, 32 temperatures 488 / 216; 1024
-// ladders of 32 x 13 39 / 28.  Past it waves share a SIMD and the exchange of
+// ladders of 32 x 13 39 / 28; EAM, 32 x 13 68 / 30, 32 x 30 183 / 102, 8 x 55
+// 282 / 192, 256 ladders of 32 x 30 176 / 104.  Past it waves share a SIMD and the exchange of
 // partial sums is paid for nothing (1024 x 32 x 13: 2 and 4 lanes 28, 8 37, 16 56;
 // one ladder of 32 x 13 on 16 lanes 15, on 8 14).  Binary32 keeps its widths:
 // the order of its sums decides between trajectories; so does the reference
@@ -649,7 +650,7 @@ int plan(ptmc_engine *h)
         const int N = rh.d.n_atoms, R = rh.d.n_temps;
         const int req = rh.d.lanes_per_replica > 0 ? rh.d.lanes_per_replica
                         : h->cfg.lanes_per_replica > 0 ? h->cfg.lanes_per_replica
-                        : prec == 0 && !eam && h->cfg.pair_form == 0 ? fp64_lanes(N, R, all_slots, cus)
+                        : prec == 0 && h->cfg.pair_form == 0 ? fp64_lanes(N, R, all_slots, cus)
                                                        : default_lanes(N, prec);
         if (req > 16)
             return fail(h, PTMC_E_UNSUPPORTED, "run %d: %d lanes per configuration need the spread layout "
