@@ -23,12 +23,12 @@
 
 #include "../../include/ptmc.h"
 #include "ptmc_device.hpp"
+#include "ptmc_multihist_cut.hpp"
+
+using namespace ptmc;
 
 namespace {
 
-constexpr int MH_THREADS = 256;
-constexpr int MH_BINS = 128;                   // bins of a block, whose sums are formed together
-constexpr size_t MH_SLICE_LDS = 96 * 1024;     // largest slice of a run's bins kept in LDS
 constexpr double MH_REBASE = 16.0;
 constexpr unsigned MH_SPIN = 1u << 26;         // polls of a grid barrier before it gives up (seconds)
 
@@ -133,14 +133,6 @@ __device__ bool mh_barrier(const MHArgs &a, int run, unsigned epoch, int *s_ok)
     __syncthreads();
     return *s_ok != 0;
 }
-
-// LDS of mh_iterate_kernel in doubles: the temperatures' terms, and with KEEP
-// a slice of `bins` bins (matrix, histogram sums, offsets, ratios)
-__host__ __device__ inline size_t mh_lds(int R, bool keep, bool totals)
-{
-    return (size_t)3 * R + (keep || R <= MH_THREADS ? MH_THREADS : 0) + (totals ? R : 0);
-}
-__host__ __device__ inline size_t mh_slice(int R, size_t bins) { return bins * ((size_t)R + 3); }
 
 // The fixed point of every run.  KEEP: a workgroup keeps its bins' slice of K
 // and their terms in LDS; an iteration reads K twice, lanes over bins both
@@ -471,29 +463,14 @@ int mh_run(const MHCall &q, int device, size_t max_lds)
     const size_t nR = (size_t)q.n_runs * R, nX = (size_t)q.n_runs * q.n_res;
     int cus = 0;
     MHCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
-    // Workgroups of a run.  Up to 512 bins (NVT histograms) one, if its slice
-    // fits LDS: an iteration (4.5 us) is not worth a barrier between workgroups
-    // (about 3 us).  Else the bins are cut so that every slice fits LDS, and
-    // over more workgroups while the runs leave compute units idle (48 x 10^4
-    // NPT bins: 79 workgroups of one block each).
     MHArgs a{};
-    a.n_blk = (int)((B + MH_BINS - 1) / MH_BINS);
-    auto cut = [&](int n) {
-        a.wg_blk = (a.n_blk + n - 1) / n;
-        a.n_wg = (a.n_blk + a.wg_blk - 1) / a.wg_blk;
-    };
-    auto slice = [&]() { return 8 * mh_slice(q.n_temps, std::min(B, (size_t)a.wg_blk * MH_BINS)); };
-    cut(1);
-    const size_t base = 8 * mh_lds(q.n_temps, true, false);
-    const size_t room = std::min(MH_SLICE_LDS, max_lds > base ? max_lds - base : 0);
-    if (B > 512 || slice() > room) {
-        cut(std::max(1, std::min(a.n_blk, cus / q.n_runs)));
-        while (slice() > room && a.wg_blk > 1 && a.n_wg < cus) cut(std::min(cus, 2 * a.n_wg));
-    }
-    const bool keep = slice() <= room;
-    const size_t lds = keep ? base + slice() : 8 * mh_lds(q.n_temps, false, false);
-    const void *fn = keep ? reinterpret_cast<const void *>(&mh_iterate_kernel<true>)
-                          : reinterpret_cast<const void *>(&mh_iterate_kernel<false>);
+    const MhCut cut = mh_cut(q.n_temps, B, q.n_runs, cus, max_lds);
+    a.n_blk = cut.n_blk;
+    a.wg_blk = cut.wg_blk;
+    a.n_wg = cut.n_wg;
+    const size_t lds = cut.lds;
+    const void *fn = cut.keep ? reinterpret_cast<const void *>(&mh_iterate_kernel<true>)
+                              : reinterpret_cast<const void *>(&mh_iterate_kernel<false>);
     MHCHK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     // runs of one launch: all, or as many as are resident together when a run has several workgroups
     const int batch = a.n_wg == 1 ? q.n_runs : std::max(1, std::min(q.n_runs, cus / a.n_wg));

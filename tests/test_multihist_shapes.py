@@ -61,7 +61,7 @@ def test_nvt(n_runs, R, nb, iters):
 
 
 @pytest.mark.parametrize("n_runs,R,nb,iters", [(1, 3, 11, 20), (2, 3, 22, 20), (2, 3, 23, 20), (260, 2, 23, 5),
-                                               (1, 90, 23, 1)])
+                                               (1, 90, 23, 1), (1, 48, 182, 1)])
 def test_npt(n_runs, R, nb, iters):
     rng = np.random.default_rng(100 * R + nb)
     t = 10.0 * 2.0 ** (np.arange(R) / (R - 1))
