@@ -111,9 +111,15 @@ __global__ void __launch_bounds__(MH_THREADS) mh_total_kernel(MHArgs a)
 
 // All workgroups of a run have arrived `epoch` times.  The launch is
 // cooperative (every workgroup is resident), and a wait that lasts for
-// seconds gives up with the error flag, so every wave ends.
+// seconds gives up with the error flag, so every wave ends.  Each wave waits
+// for its own block sums before the workgroup's barrier: that barrier waits for
+// LDS only, and the arrival's release for the stores of its own wave.  The sums
+// are agent-scope stores, written past the L2, so the wait is all they need (a
+// release fence in every wave would write the L2 back four times, 2.3 us an
+// iteration on 79 workgroups).
 __device__ bool mh_barrier(const MHArgs &a, int run, unsigned epoch, int *s_ok)
 {
+    __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     if (threadIdx.x == 0) {
         __hip_atomic_fetch_add(&a.count[run], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
