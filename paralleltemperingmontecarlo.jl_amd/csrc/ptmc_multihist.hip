@@ -48,6 +48,7 @@ struct MHArgs {
     int *iterations;         // runs, or null
     double *ncyc;            // runs x R histogram totals, or null: each workgroup forms its run's
     double *off, *ratio;     // runs x n_bins: offsets and H_m / D_m of the last free energies
+    double *hsum;            // runs x n_bins histogram sums H_m (slices that are not kept)
     double *part;            // runs x 2 x n_blk x R block sums (n_wg > 1)
     unsigned *count;         // runs arrivals at the barrier, zeroed (n_wg > 1)
     int *error;              // set when a barrier gave up, zeroed (n_wg > 1)
@@ -178,7 +179,7 @@ __global__ void __launch_bounds__(MH_THREADS) mh_iterate_kernel(MHArgs a)
     double *end = fe + mh_lds(R, KEEP, false);
     double *ncyc = a.ncyc ? a.ncyc + (size_t)run * R : end;  // end: the entry point without workspace, never KEEP
     const size_t g0 = (size_t)run * a.n_bins + b0;
-    double *hs = end;                              // KEEP: nc histogram sums
+    double *hs = KEEP ? end : a.hsum + g0;         // nc histogram sums
     double *off = KEEP ? hs + nc : a.off + g0;
     double *ratio = KEEP ? off + nc : a.ratio + g0;  // H_m / D_m
     double *K = ratio + nc;                        // KEEP: R x nc
@@ -200,8 +201,7 @@ __global__ void __launch_bounds__(MH_THREADS) mh_iterate_kernel(MHArgs a)
         for (int i = 0; i < R; ++i) s = s + h[(size_t)i * bins.stride()];
         return s;
     };
-    if constexpr (KEEP)
-        for (int m = tid; m < nc; m += MH_THREADS) hs[m] = hist_sum(m);
+    for (int m = tid; m < nc; m += MH_THREADS) hs[m] = hist_sum(m);  // read by the same thread
     if (tid == 0) s_rebase = 1;
     __syncthreads();
 
@@ -255,7 +255,7 @@ __global__ void __launch_bounds__(MH_THREADS) mh_iterate_kernel(MHArgs a)
 #pragma unroll
                     for (int k = 0; k < 4; ++k)
                         if (i + k < R) d[k] = __builtin_fma(wgt[i + k], term(i + k, h, o), d[k]);
-                ratio[m] = hist_sum(m) / ((d[0] + d[2]) + (d[1] + d[3]));
+                ratio[m] = hs[m] / ((d[0] + d[2]) + (d[1] + d[3]));
             }
         }
         __syncthreads();
@@ -270,18 +270,28 @@ __global__ void __launch_bounds__(MH_THREADS) mh_iterate_kernel(MHArgs a)
         // block sums, a row of 16 lanes per temperature (all steps of the row
         // sum are lane permutations of the VALU); without a cut they go
         // straight into the sequences, each temperature's by one row in order
-        for (int i0 = 0; i0 < R; i0 += MH_THREADS / 16) {
-            const int i = i0 + tid / 16, row = tid & 15;
-            for (int g = 0; g < nblk; ++g) {
+        const int row = tid & 15;
+        for (int g = 0; g < nblk; ++g) {
+            constexpr int U = MH_BINS / 16;
+            double rb[U], hb[U], ob[U];  // the lane's bins, for all its temperatures
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int m = min(g * MH_BINS + 16 * u + row, nc - 1);
+                rb[u] = ratio[m];
+                hb[u] = KEEP ? 0.0 : bins.h(b0 + m);
+                ob[u] = KEEP ? 0.0 : off[m];
+            }
+            for (int i0 = 0; i0 < R; i0 += MH_THREADS / 16) {
+                const int i = i0 + tid / 16;
                 double s = 0.0;
 #pragma unroll
-                for (int u = 0; u < MH_BINS; u += 16) {
-                    const int m = g * MH_BINS + u + row;
+                for (int u = 0; u < U; ++u) {
+                    const int m = g * MH_BINS + 16 * u + row;
                     if (i < R && m < nc) {
                         double k;
                         if constexpr (KEEP) k = K[(size_t)i * nc + m];
-                        else k = term(i, bins.h(b0 + m), off[m]);
-                        s = __builtin_fma(ratio[m], k, s);
+                        else k = term(i, hb[u], ob[u]);
+                        s = __builtin_fma(rb[u], k, s);
                     }
                 }
                 s = mh_row_sum(s);
@@ -295,9 +305,9 @@ __global__ void __launch_bounds__(MH_THREADS) mh_iterate_kernel(MHArgs a)
                     }
                 }
             }
-            if (a.n_wg == 1 && row == 0 && i < R)
-                for (int k = nblk; k < q; ++k) dpart[k * R + i] = 0.0;
         }
+        if (a.n_wg == 1)
+            for (int e = nblk * R + tid; e < q * R; e += MH_THREADS) dpart[e] = 0.0;
         if (a.n_wg > 1) {
             if (!mh_barrier(a, run, (unsigned)it, &s_ok)) break;
             for (int e = tid; e < q * R; e += MH_THREADS) {
@@ -413,9 +423,8 @@ __global__ void __launch_bounds__(T) mh_result_kernel(MHArgs a)
 }
 
 // Device-resident scratch of the allocation-free entry point: the per-bin
-// terms of every run of one call (3 n_bin^2 doubles per run are asked for, the
-// offsets and ratios use two thirds), one copy per GPU for the life of the
-// process.  Every element a call reads it has written first, so nothing needs
+// terms of every run of one call (3 n_bin^2 doubles per run: histogram sums,
+// offsets and ratios), one copy per GPU for the life of the process.  Every element a call reads it has written first, so nothing needs
 // clearing between calls; calls that overlap on one GPU share
 // it and race.
 static __device__ __align__(256) double npt_scratch[PTMC_NOALLOC_NPT_SCRATCH_DOUBLES];
@@ -487,6 +496,7 @@ int mh_run(const MHCall &q, int device, size_t max_lds)
     const size_t o_out = m.take(((q.moments ? 4 : 1) * nX + nR) * 8 + (size_t)q.n_runs * sizeof(int));
     const size_t o_ncyc = m.take(nR * 8), o_off = m.take((size_t)q.n_runs * B * 8);
     const size_t o_ratio = m.take((size_t)q.n_runs * B * 8);
+    const size_t o_hsum = m.take(cut.keep ? 8 : (size_t)q.n_runs * B * 8);
     const size_t o_part = m.take(a.n_wg > 1 ? 2 * nR * a.n_blk * 8 : 8);
     const size_t o_count = m.take(((size_t)q.n_runs + 1) * sizeof(unsigned));
     MHCHK(hipMalloc((void **)&m.p, m.used));
@@ -531,6 +541,7 @@ int mh_run(const MHCall &q, int device, size_t max_lds)
     a.ncyc = reinterpret_cast<double *>(m.p + o_ncyc);
     a.off = reinterpret_cast<double *>(m.p + o_off);
     a.ratio = reinterpret_cast<double *>(m.p + o_ratio);
+    a.hsum = reinterpret_cast<double *>(m.p + o_hsum);
     a.part = reinterpret_cast<double *>(m.p + o_part);
     a.count = reinterpret_cast<unsigned *>(m.p + o_count);
     a.error = reinterpret_cast<int *>(a.count + q.n_runs);
@@ -552,6 +563,7 @@ int mh_run(const MHCall &q, int device, size_t max_lds)
         b.ncyc += (size_t)r0 * R;
         b.off += (size_t)r0 * B;
         b.ratio += (size_t)r0 * B;
+        if (!cut.keep) b.hsum += (size_t)r0 * B;
         b.part += 2 * (size_t)r0 * a.n_blk * R;
         b.count += r0;
         void *args[] = {&b};
@@ -693,6 +705,7 @@ extern "C" int ptmc_multihistogram_npt_noalloc(int32_t n_runs, int32_t n_temps, 
     a.iterations = iterations;
     a.off = scr;
     a.ratio = scr + (size_t)n_runs * a.n_bins;
+    a.hsum = scr + 2 * (size_t)n_runs * a.n_bins;
     const hipStream_t s = static_cast<hipStream_t>(stream);
     hipLaunchKernelGGL(mh_iterate_kernel<false>, dim3(n_runs), dim3(MH_THREADS), lds, s, a);
     if (hipGetLastError() != hipSuccess) return PTMC_E_DEVICE;
