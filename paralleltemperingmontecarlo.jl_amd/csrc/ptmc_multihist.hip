@@ -479,7 +479,9 @@ int mh_run(const MHCall &q, int device, size_t max_lds)
     int cus = 0;
     MHCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
     MHArgs a{};
-    const MhCut cut = mh_cut(q.n_temps, B, q.n_runs, cus, max_lds);
+    hipFuncAttributes fa{};  // LDS beside what is asked for
+    MHCHK(hipFuncGetAttributes(&fa, reinterpret_cast<const void *>(&mh_iterate_kernel<true>)));
+    const MhCut cut = mh_cut(q.n_temps, B, q.n_runs, cus, max_lds - std::min(max_lds, fa.sharedSizeBytes));
     a.n_blk = cut.n_blk;
     a.wg_blk = cut.wg_blk;
     a.n_wg = cut.n_wg;

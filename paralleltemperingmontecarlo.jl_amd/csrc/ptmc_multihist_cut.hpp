@@ -9,7 +9,6 @@ namespace ptmc {
 
 constexpr int MH_THREADS = 256;
 constexpr int MH_BINS = 128;                   // bins of a block, whose sums are formed together
-constexpr size_t MH_SLICE_LDS = 96 * 1024;     // largest slice of a run's bins kept in LDS
 
 // LDS of mh_iterate_kernel in doubles: the temperatures' terms, and with KEEP
 // a slice of `bins` bins (matrix, histogram sums, offsets, ratios)
@@ -26,7 +25,7 @@ struct MhCut {
 };
 
 // Workgroups of a run of `bins` bins and R temperatures, one of `runs` runs, on
-// a device of `cus` compute units with max_lds bytes of LDS a workgroup.  Up to
+// a device of `cus` compute units with max_lds bytes of LDS that a workgroup can ask for.  Up to
 // 512 bins (NVT histograms) one, if its slice fits LDS: an iteration (4.5 us)
 // is not worth a barrier between workgroups (about 3 us).  Else the bins are cut
 // so that every slice fits LDS, and over more workgroups while the runs leave
@@ -44,7 +43,7 @@ inline MhCut mh_cut(int R, size_t bins, int runs, int cus, size_t max_lds)
     auto slice = [&]() { return 8 * mh_slice(R, std::min(bins, (size_t)c.wg_blk * MH_BINS)); };
     cut(1);
     const size_t base = 8 * mh_lds(R, true, false);
-    const size_t room = std::min(MH_SLICE_LDS, max_lds > base ? max_lds - base : 0);
+    const size_t room = max_lds > base ? max_lds - base : 0;
     if (bins > 512 || slice() > room) {
         const size_t fit = room / (8 * mh_slice(R, MH_BINS));  // blocks of a slice
         const int need = fit > 0 ? (int)((c.n_blk + fit - 1) / fit) : c.n_blk;

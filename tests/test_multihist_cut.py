@@ -32,8 +32,7 @@ int main(int argc, char **argv)
         // every slice fits once there are as many workgroups as compute units, or it is not kept
         const size_t most = (size_t)((c.n_blk + cus - 1) / cus) * MH_BINS, least = bins < most ? bins : most;
         const size_t base = 8 * mh_lds(R, true, false);
-        const bool could = base < max_lds && 8 * mh_slice(R, least) <= max_lds - base &&
-                           8 * mh_slice(R, least) <= MH_SLICE_LDS;
+        const bool could = base < max_lds && 8 * mh_slice(R, least) <= max_lds - base;
         if (!covers || !fits || (c.n_wg > 1 && c.n_wg > cus) || could != c.keep) {
             if (bad++ < 5) std::printf("R %d bins %zu runs %d: n_wg %d wg_blk %d keep %d\\n", R, bins, n, c.n_wg, c.wg_blk, (int)c.keep);
         }

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from conftest import gpu_available
-from oracle.multihist import KB, multihistogram_npt, multihistogram_nvt
+from oracle.multihist import KB, K_MULTIHIST, multihistogram_npt, multihistogram_nvt
 
 pytestmark = pytest.mark.gpu
 
@@ -61,7 +61,7 @@ def test_nvt(n_runs, R, nb, iters):
 
 
 @pytest.mark.parametrize("n_runs,R,nb,iters", [(1, 3, 11, 20), (2, 3, 22, 20), (2, 3, 23, 20), (260, 2, 23, 5),
-                                               (1, 90, 23, 1), (1, 48, 182, 1)])
+                                               (1, 90, 23, 1), (1, 160, 23, 1), (1, 48, 182, 1)])
 def test_npt(n_runs, R, nb, iters):
     rng = np.random.default_rng(100 * R + nb)
     t = 10.0 * 2.0 ** (np.arange(R) / (R - 1))
@@ -82,3 +82,34 @@ def test_npt(n_runs, R, nb, iters):
         np.testing.assert_allclose(fe[r], rfe, rtol=1e-11, atol=1e-11)
     for r in range(len(hs), n_runs):
         assert np.array_equal(cp[r], cp[r % len(hs)])
+
+
+# 8 ((R + 3) (nb + 3) + 247) bytes of LDS for the slice and the temperatures'
+# terms are 24 short of the 160 KiB of a workgroup: with those the kernel declares
+# itself they do not fit, and the slice is not kept
+@pytest.mark.parametrize("R,nb", [(2887, 4), (167, 116)])
+def test_nvt_slice_at_the_lds_limit(R, nb):
+    rng = np.random.default_rng(R)
+    t = 5.0 * 2.0 ** (np.arange(R) / (R - 1))
+    h, e0, e1 = _hists(rng, t, nb, False)
+    beta = 1.0 / (KB * t)
+    cv, t_res, fe, it = pt.multihistogram_nvt_batch([t], beta[None], h[None], [e0], [e1], nb, 0.0, max_iter=3)
+    e = e0 + (np.arange(nb) + 0.5) * (e1 - e0) / nb
+    f, n, hs = np.zeros(R), h[:, 1:-1].sum(1), h[:, 1:-1].sum(0)
+
+    def terms():
+        x = -beta[:, None] * e - f[:, None]
+        off = x.max(0) + np.log(1000.0)
+        return off, hs / (n[:, None] * np.exp(x - off)).sum(0)
+
+    for _ in range(3):
+        off, ratio = terms()
+        f = np.log((ratio * np.exp(-beta[:, None] * e - off)).sum(1))
+    off, ratio = terms()
+    tr = t[0] * (t[-1] / t[0]) ** (np.arange(10 * R) / (10 * R - 1))
+    q = ratio * np.exp(-e / (KB * tr)[:, None] - off)
+    q /= q.sum(1, keepdims=True)
+    d = e - (q * e).sum(1, keepdims=True)
+    assert it[0] == 3
+    np.testing.assert_allclose(fe[0], f, rtol=1e-11, atol=1e-11)
+    np.testing.assert_allclose(cv[0], (q * d * d).sum(1) / (K_MULTIHIST * tr**2), **TOL)
