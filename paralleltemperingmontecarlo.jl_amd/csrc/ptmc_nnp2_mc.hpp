@@ -47,6 +47,7 @@ namespace ptmc {
 namespace {
 
 constexpr int N2_NW = NNP2_NT / 64;
+constexpr bool N2_F32 = sizeof(N2R) == 4;
 
 // one move's draws: the atom move, and the species picks of a swap
 struct N2Draw {
@@ -165,6 +166,14 @@ __device__ __forceinline__ N2R n2_d2(const N2R *a, const N2R *b)
 __device__ __forceinline__ N2R n2_rad(N2R r2, N2R f, N2R eta)
 {
     return (f != N2R(0.0) && f != N2R(1.0)) ? f * exp(-eta * r2) : N2R(0.0);
+}
+
+// A feature's scale and offset are applied in FP64 and the feature rounded once:
+// a narrow range makes both large and of opposite sign.
+__device__ __forceinline__ N2R n2_scaled(N2R sum, double scale, double offset) { return (N2R)((double)sum * scale + offset); }
+__device__ __forceinline__ N2R n2_changed(N2R feature, N2R change, double scale)
+{
+    return (N2R)((double)feature + (double)change * scale);
 }
 
 // b^zeta: integer zeta by squaring, else pow (rounding can leave b = 1 +
@@ -349,13 +358,15 @@ __device__ __forceinline__ N2R n2_sum8(const N2R (&v)[8], int lane)
 
 // Visits of a wave: moved atom a (the m-th), partners k = part, part + 2, ...
 // of each species block, a lane per target j.  Changes of the rows of the
-// wave's group at the unmoved atoms: part 0 into D, part 1 into B (added to D
-// after a barrier); sums at the moved atom into S (both orders of an
-// equal-species pair are visited).  b: the other moved atom of a swap, a
+// wave's group at the unmoved atoms: FP64 part 0 into D, part 1 into B (added to
+// D after a barrier); binary32 unscaled, part 0 kept by the wave and part 1 into B,
+// for n2_add to round a row's change into D once.  Sums at the moved atom into S
+// (both orders of an equal-species pair are visited).  b: the other moved atom of a swap, a
 // partner at its trial position, or -1; the triangles with both moved atoms
 // count at j once (m = 0).
 template <bool POW, bool SWAP>
-__device__ __forceinline__ void n2_visits(const N2R *Pg, int N, int gl, int m, int a, int b, int part, int lane)
+__device__ __forceinline__ void n2_visits(const N2R *Pg, int N, int gl, int m, int a, int b, int part, int lane,
+                                          N2R (&kept)[2][NNP2_GMAX])
 {
     N2Tab &T = n2_fresh();
     const N2Lds L = n2_lds(T, N);
@@ -416,17 +427,26 @@ __device__ __forceinline__ void n2_visits(const N2R *Pg, int N, int gl, int m, i
                 own[l] = fma_<N2R>(ea, t[2], own[l]);
             });
         }
-        // the scales first, so that their loads are in flight together
-        N2R sf[NNP2_GMAX];
+        if constexpr (N2_F32) {
 #pragma unroll
-        for (int l = 0; l < NNP2_GMAX; ++l) sf[l] = (N2R)T.ang[G.q[l] * 15 + 3 + 3 * sc + sa + blk];
+            for (int l = 0; l < NNP2_GMAX; ++l) {
+                if (blk) kept[1][l] = accJ[l];
+                else kept[0][l] = accJ[l];
+                if (l < G.cnt && still && part == 1) L.B[((gl * NNP2_GMAX + l) * 2 + blk) * N + lane] = accJ[l];
+            }
+        } else {
+            // the scales first, so that their loads are in flight together
+            N2R sf[NNP2_GMAX];
 #pragma unroll
-        for (int l = 0; l < NNP2_GMAX; ++l) {
-            if (l < G.cnt) {
-                const int q = G.q[l];
-                if (still) {
-                    if (part == 0) L.D[(2 * T.n_rad + 3 * q + sa + blk) * N + lane] += accJ[l] * sf[l];
-                    else L.B[((gl * NNP2_GMAX + l) * 2 + blk) * N + lane] = accJ[l] * sf[l];
+            for (int l = 0; l < NNP2_GMAX; ++l) sf[l] = (N2R)T.ang[G.q[l] * 15 + 3 + 3 * sc + sa + blk];
+#pragma unroll
+            for (int l = 0; l < NNP2_GMAX; ++l) {
+                if (l < G.cnt) {
+                    const int q = G.q[l];
+                    if (still) {
+                        if (part == 0) L.D[(2 * T.n_rad + 3 * q + sa + blk) * N + lane] += accJ[l] * sf[l];
+                        else L.B[((gl * NNP2_GMAX + l) * 2 + blk) * N + lane] = accJ[l] * sf[l];
+                    }
                 }
             }
         }
@@ -580,7 +600,7 @@ __device__ __forceinline__ double n2_rebuild(N2R *P, int N, double *s_tot)
                 const N2R v = lane < N && lane != c ? n2_rad(r2, n2_cut(sqrt(r2), (N2R)T.r_cut), (N2R)R[0]) : N2R(0.0);
                 for (int r = 0; r < 2; ++r) {
                     const N2R s = n2_wave_sum((lane < n1) == (r == 0) ? v : N2R(0.0));
-                    if (lane == 0) L.D[(size_t)(2 * q + r) * N + c] = s * (N2R)R[1 + 2 * sc + r] + (N2R)R[5 + 2 * sc + r];
+                    if (lane == 0) L.D[(size_t)(2 * q + r) * N + c] = n2_scaled(s, R[1 + 2 * sc + r], R[5 + 2 * sc + r]);
                 }
                 continue;
             }
@@ -605,7 +625,7 @@ __device__ __forceinline__ double n2_rebuild(N2R *P, int N, double *s_tot)
                         const int q = G.q[l];
                         auto store = [&](int row, N2R v) {
                             const double *A = T.ang + (size_t)q * 15 + 3 * sc + row;
-                            if (lane == 0) L.D[(size_t)(2 * T.n_rad + 3 * q + row) * N + c] = v * (N2R)A[3] + (N2R)A[9];
+                            if (lane == 0) L.D[(size_t)(2 * T.n_rad + 3 * q + row) * N + c] = n2_scaled(v, A[3], A[9]);
                         };
                         // both orders of an equal-species pair were visited
                         const N2R v = n2_species_sum(own[l], n1, lane, false);
@@ -726,11 +746,31 @@ __device__ __forceinline__ void n2_radial(int q, const N2Move &mv, int mm, int N
     const N2R vn = lane < N ? n2_rad(L.r2n[mm * 64 + lc], L.fn[mm * 64 + lc], eta) : N2R(0.0);
     if (lane < N && lane != mv.a && lane != mv.b) {
         const N2R vo = n2_rad(L.r2o[mm * 64 + lc], L.fo[mm * 64 + lc], eta);
-        L.D[(2 * q + sa) * N + lane] += (vn - vo) * (N2R)R[1 + 2 * sc + sa];
+        N2R &d = L.D[(2 * q + sa) * N + lane];
+        d = n2_changed(d, vn - vo, R[1 + 2 * sc + sa]);
     }
     for (int r = 0; r < 2; ++r) {
         const N2R v = n2_species_sum(vn, n1, lane, r == 1);
-        if (lane == 0) L.D[(2 * q + r) * N + aa] = v * (N2R)R[1 + 2 * sa + r] + (N2R)R[5 + 2 * sa + r];
+        if (lane == 0) L.D[(2 * q + r) * N + aa] = n2_scaled(v, R[1 + 2 * sa + r], R[5 + 2 * sa + r]);
+    }
+}
+
+// Binary32: both parts' changes of the wave's group at an unmoved atom into D.
+__device__ __forceinline__ void n2_add(const N2Lds &L, N2Tab &T, const N2R (&kept)[2][NNP2_GMAX], int N, int gl, int sa,
+                                       int lane)
+{
+    const int sc = lane < T.n1 ? 0 : 1, cnt = __builtin_amdgcn_readfirstlane(L.G[gl].cnt);
+#pragma unroll
+    for (int l = 0; l < NNP2_GMAX; ++l) {
+        if (l < cnt) {
+            const int q = __builtin_amdgcn_readfirstlane(L.G[gl].q[l]);
+#pragma unroll
+            for (int blk = 0; blk < 2; ++blk) {
+                N2R &d = L.D[(2 * T.n_rad + 3 * q + sa + blk) * N + lane];
+                d = n2_changed(d, kept[blk][l] + L.B[((gl * NNP2_GMAX + l) * 2 + blk) * N + lane],
+                               T.ang[q * 15 + 3 + 3 * sc + sa + blk]);
+            }
+        }
     }
 }
 
@@ -762,10 +802,11 @@ __device__ __forceinline__ void n2_features(const N2Move &mv, N2R *P, int N, int
         __syncthreads();
         for (int mm = 0; mm < nm; ++mm) {
             const int aa = mv.atom(mm);
+            N2R kept[2][NNP2_GMAX];
             if (gl < ngp) {
                 const N2R *Pg = P + (size_t)(g0 + gl) * N * 64;
-                if (mv.swap) n2_visits<POW, true>(Pg, N, gl, mm, aa, mv.other(mm), part, lane);
-                else n2_visits<POW, false>(Pg, N, gl, mm, aa, -1, part, lane);
+                if (mv.swap) n2_visits<POW, true>(Pg, N, gl, mm, aa, mv.other(mm), part, lane, kept);
+                else n2_visits<POW, false>(Pg, N, gl, mm, aa, -1, part, lane, kept);
             }
             // radial functions, by the waves without a group if there are any
             const int idle = N2_NW - 2 * ngp;
@@ -776,10 +817,14 @@ __device__ __forceinline__ void n2_features(const N2Move &mv, N2R *P, int N, int
             N2Tab &T = n2_fresh();
             const N2Lds L = n2_lds(T, N);
             const int sa = aa < T.n1 ? 0 : 1;
-            for (int u = w; u < ngp * 2 * NNP2_GMAX; u += N2_NW) {
-                const int g = u / (2 * NNP2_GMAX), l = u % (2 * NNP2_GMAX) / 2, blk = u & 1;
-                if (l < L.G[g].cnt && lane < N && lane != mv.a && lane != mv.b)
-                    L.D[(2 * T.n_rad + 3 * L.G[g].q[l] + sa + blk) * N + lane] += L.B[u * N + lane];
+            if constexpr (N2_F32) {
+                if (gl < ngp && part == 0 && lane < N && lane != mv.a && lane != mv.b) n2_add(L, T, kept, N, gl, sa, lane);
+            } else {
+                for (int u = w; u < ngp * 2 * NNP2_GMAX; u += N2_NW) {
+                    const int g = u / (2 * NNP2_GMAX), l = u % (2 * NNP2_GMAX) / 2, blk = u & 1;
+                    if (l < L.G[g].cnt && lane < N && lane != mv.a && lane != mv.b)
+                        L.D[(2 * T.n_rad + 3 * L.G[g].q[l] + sa + blk) * N + lane] += L.B[u * N + lane];
+                }
             }
             if (mm + 1 < nm) __syncthreads();
         }
@@ -790,7 +835,7 @@ __device__ __forceinline__ void n2_features(const N2Move &mv, N2R *P, int N, int
     for (int u = threadIdx.x; u < nm * T.n_ang * 3; u += NNP2_NT) {
         const int mm = u >= T.n_ang * 3, v = mm ? u - T.n_ang * 3 : u, q = v / 3, row = v % 3, aa = mv.atom(mm);
         const double *A = T.ang + (size_t)q * 15 + 3 * (aa < T.n1 ? 0 : 1) + row;
-        L.D[(2 * T.n_rad + 3 * q + row) * N + aa] = (L.S[2 * u] + L.S[2 * u + 1]) * (N2R)A[3] + (N2R)A[9];
+        L.D[(2 * T.n_rad + 3 * q + row) * N + aa] = n2_scaled(L.S[2 * u] + L.S[2 * u + 1], A[3], A[9]);
     }
     __syncthreads();
 }

@@ -225,3 +225,22 @@ def test_nnvt_binary32_replay(base_pot, oracle):
     c = eng.counters(0)
     np.testing.assert_array_equal(c["count_vol"], run.count_vol)
     eng.close()
+
+
+def test_nnvt_binary32_energies(base_pot):
+    """Binary32 features are scaled and offset in FP64 and rounded once: over 64
+    configurations of Cu50Zn5 the root mean square error of the total is below
+    2^-23 |E| (the spacing of binary32 at the total).  Scale and offset rounded
+    to binary32 are the same for every configuration and atom: they gave a mean
+    error of 2^-22 |E|."""
+    pot = replace(base_pot, n1=50, n2=5)
+    x = np.stack([cluster(55, 100 + t) for t in range(64)]).astype(np.float32).astype(np.float64)
+    beta = 1.0 / (KB * np.linspace(300.0, 900.0, len(x)))
+    eng = pt.PTEngine(pot, pt.NNVT.of([50, 5], natomswaps=1), pt.SphericalBC(40.0), pt.MCParams(10, len(x), 55),
+                      pt.EngineOptions(precision="fp32", seed=1))
+    eng.add_run(55, beta, x, pt.SphericalBC(40.0))
+    eng.prepare()
+    ref = pt.nnp2_energies(pot, x)[0]
+    err = eng.energies(0) - ref
+    eng.close()
+    assert np.sqrt((err**2).mean()) <= 2.0**-23 * np.abs(ref).mean(), (np.sqrt((err**2).mean()), err.mean())
