@@ -41,6 +41,7 @@
 // (no include guard: included once per element type)
 #include "ptmc_nnp_layout.hpp"
 #include "ptmc_sweep.hpp"
+#include "ptmc_tanh.hpp"
 
 namespace ptmc {
 
@@ -128,32 +129,7 @@ __device__ __forceinline__ N2R n2_cut(N2R r, N2R rc)
     return r < rc ? c * c : N2R(0.0);
 }
 
-// tanh x = t / (t + 2), t = e^(2x) - 1 = 2^k q + (2^k - 1) with q = e^r - 1 by
-// its Taylor series, 2x = k ln 2 + r (Cody-Waite): within 2 ulp, small x
-// included; a fifth of the library's instructions.
-__device__ __forceinline__ double n2_tanh(double x)
-{
-    const double y = fmin(fabs(x), 20.0) * 2.0;
-    const double kd = rint(y * 1.4426950408889634);
-    const double r = fma(-kd, 1.90821492927058770002e-10, fma(-kd, 6.93147180369123816490e-01, y));
-    double q = 1.0 / 6227020800.0;
-    q = fma(q, r, 1.0 / 479001600.0);
-    q = fma(q, r, 1.0 / 39916800.0);
-    q = fma(q, r, 1.0 / 3628800.0);
-    q = fma(q, r, 1.0 / 362880.0);
-    q = fma(q, r, 1.0 / 40320.0);
-    q = fma(q, r, 1.0 / 5040.0);
-    q = fma(q, r, 1.0 / 720.0);
-    q = fma(q, r, 1.0 / 120.0);
-    q = fma(q, r, 1.0 / 24.0);
-    q = fma(q, r, 1.0 / 6.0);
-    q = fma(q, r, 0.5);
-    q = fma(q * r, r, r);
-    const double p = __longlong_as_double((long long)(1023 + (int)kd) << 52);
-    const double t = fma(p, q, p - 1.0);
-    const double v = t / (t + 2.0);
-    return x != x ? x : copysign(v, x);
-}
+__device__ __forceinline__ double n2_tanh(double x) { return net_tanh(x); }
 __device__ __forceinline__ float n2_tanh(float x) { return tanhf(x); }
 
 __device__ __forceinline__ N2R n2_d2(const N2R *a, const N2R *b)
