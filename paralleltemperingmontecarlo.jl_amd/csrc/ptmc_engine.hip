@@ -940,6 +940,14 @@ int prepare_nnp2(ptmc_engine *h)
     HIPCHK(h, hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
     const int N = n.n1 + n.n2;
     const bool f32 = h->cfg.precision == 1;
+    const bool pw = std::find(n.gprog.begin(), n.gprog.end(), NNP2_POW) != n.gprog.end();
+    const void *fs = (const void *)(f32 ? nnp2_sweep_fn_f32(pw) : nnp2_sweep_fn(pw));
+    const void *fi = (const void *)(f32 ? nnp2_init_fn_f32(pw) : nnp2_init_fn(pw));
+    // what a launch can ask for: the kernels' own LDS comes off
+    hipFuncAttributes as{}, ai{};
+    HIPCHK(h, hipFuncGetAttributes(&as, fs));
+    HIPCHK(h, hipFuncGetAttributes(&ai, fi));
+    max_lds -= (int)std::max(as.sharedSizeBytes, ai.sharedSizeBytes);
     // groups of a pass: as many as the workgroup has pairs of waves, fewer
     // where LDS would not hold their rows
     int pass = std::max(1, std::min(NNP2_GP, n.n_groups));
@@ -957,9 +965,6 @@ int prepare_nnp2(ptmc_engine *h)
     if ((long long)h->nnp2_lds > max_lds)
         return fail(h, PTMC_E_UNSUPPORTED, "%d atoms with %d feature rows need %zu B of LDS (%d available)", N, n.ng,
                     h->nnp2_lds, max_lds);
-    const bool pw = std::find(n.gprog.begin(), n.gprog.end(), NNP2_POW) != n.gprog.end();
-    const void *fs = (const void *)(f32 ? nnp2_sweep_fn_f32(pw) : nnp2_sweep_fn(pw));
-    const void *fi = (const void *)(f32 ? nnp2_init_fn_f32(pw) : nnp2_init_fn(pw));
     HIPCHK(h, hipFuncSetAttribute(fs, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->nnp2_lds));
     HIPCHK(h, hipFuncSetAttribute(fi, hipFuncAttributeMaxDynamicSharedMemorySize, (int)h->nnp2_lds));
     int slot = 0;

@@ -2,7 +2,8 @@
 kernel's work changes: groups of angular functions in one pass and in several
 (more than eight eta), groups split at six functions, powers by squaring, by
 pow and of non-integer zeta, layers of one and of several 16 x 16 tiles, no
-radial or no angular functions, two atoms, a full slot of 64; FP64 against the
+radial or no angular functions, two atoms, a full slot of 64, weights that would
+fill LDS to its last byte (the kernels declare some themselves); FP64 against the
 oracle move by move, binary32 against the oracle's replay of its decisions."""
 import numpy as np
 import pytest
@@ -52,6 +53,7 @@ GENERAL = ((1.0, 3.0), (-1.0, 2.5), (0.5, 4.0), (-1.0, 5.0))
     (1, 1, (0.02,), POW2[:1], 2, (4, 4), (2, 2)),
     (7, 2, (), (), 4, (8, 8), (2, 2)),
     (50, 14, (0.008, 0.03), POW2, 2, (20, 20), (2, 2)),
+    (14, 14, tuple(np.geomspace(0.002, 0.08, 8)), POW2, 2, (59, 8), (2, 2)),
 ])
 def test_moves_match_oracle(oracle, n1, n2, etas, zetas, n_rad, hidden, act):
     rng = np.random.default_rng(100 * n1 + n2)
