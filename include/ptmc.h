@@ -58,8 +58,12 @@ typedef struct {
     int32_t n_bin;             /* MCParams.n_bin (default 100) */
     double min_acc, max_acc;   /* MCParams.min_acc/max_acc (0.4, 0.6) */
     int32_t recompute_every;   /* full FP64 energy recompute every this many cycles (0 = never) */
-    int32_t lanes_per_replica; /* 0: chosen (FP64: by the room on the device too); else 1, 2, 4, 8 or 16 (32 or 64 in the
-                                  spread layout, workgroup_lanes > 0) */
+    int32_t lanes_per_replica; /* 0: chosen from the atom count (FP64 outside pair_form 1: also from the number of
+                                  configurations in the handle and the device's compute units); else 1, 2, 4, 8 or 16
+                                  (32 or 64 in the spread layout, workgroup_lanes > 0).  The lanes set the order of a
+                                  move's sums: an FP64 run keeps its bits in another batch, resumed in one, sharded or
+                                  on another device where they are given (ptmc_run_lanes tells those in use), and may
+                                  differ in the rounding of its energies where they are chosen */
     int32_t cycles_per_launch; /* cycles per kernel launch (0 = 256) */
     int32_t device;            /* HIP device ordinal */
     uint64_t seed;             /* Philox key */
@@ -98,7 +102,7 @@ typedef struct {
     int32_t n_configs;         /* start configuration of temperature i is i mod n_configs */
     double max_displ_atom;     /* initial atom step (reference default 0.1, src/MCStates.jl:104) */
     double max_displ_vol;      /* initial volume step (reference default 0.1) */
-    int32_t lanes_per_replica; /* 0: engine default */
+    int32_t lanes_per_replica; /* 0: that of the configuration */
     uint32_t run_key;          /* Philox counter word for this run; 0xffffffff = run index */
     double box_height;         /* RectangularBC, RhombicBC height (bohr) */
 } ptmc_run_desc;

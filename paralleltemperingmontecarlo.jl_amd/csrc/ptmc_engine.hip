@@ -322,9 +322,13 @@ int default_lanes(int n_atoms, int precision)
 // ladders of 32 x 13 39 / 28; EAM, 32 x 13 68 / 30, 32 x 30 183 / 102, 8 x 55
 // 282 / 192, 256 ladders of 32 x 30 176 / 104.  Past it waves share a SIMD and the exchange of
 // partial sums is paid for nothing (1024 x 32 x 13: 2 and 4 lanes 28, 8 37, 16 56;
-// one ladder of 32 x 13 on 16 lanes 15, on 8 14).  Binary32 keeps its widths:
-// the order of its sums decides between trajectories; so does the reference
-// pair form, whose sums are the reference's only in sequence.
+// one ladder of 32 x 13 on 16 lanes 15, on 8 14).  A run's FP64 sums are thus
+// taken in another order in another batch or on another device, which moves its
+// energies by their rounding (given lanes pin the order); a rule on the run alone
+// would have to stay at the widths that a full chip wants (4096 ladders of 32 x
+// 13: 1 and 2 lanes 85, 4 106, 8 135).  Binary32 pair sums keep their widths: there
+// the order soon decides between trajectories; so does the reference pair form,
+// whose sums are the reference's only in sequence.
 int fp64_lanes(int n_atoms, int n_temps, int64_t all_slots, int cus)
 {
     int kl = default_lanes(n_atoms, 0);

@@ -553,7 +553,12 @@ class EngineOptions:
     cuts the runs into that many groups launched on their own streams.
     exchange_every: replica exchange is attempted (as `exchange` says) only
     after the cycles with (cycle + 1) % exchange_every == 0; 1 (default)
-    attempts it after every cycle as src/MCRun.jl:203 does.  pair_slots: pair
+    attempts it after every cycle as src/MCRun.jl:203 does.
+    lanes_per_replica: lanes of a configuration, 0 = chosen; FP64 ladders then
+    take more while the handle's configurations leave the device idle, so that a
+    run in another batch, resumed in one or on another device may round its
+    energies differently; a given number keeps its bits (`lanes_of` tells the
+    one in use).  pair_slots: pair
     potentials one workgroup per configuration (binary32, spherical container,
     NVT, up to 64 atoms), the layout in which the learned surrogate filters
     their moves (delayed acceptance)."""
