@@ -225,6 +225,8 @@ struct ptmc_engine {
     // plugin functions: FP64 network tables (uploaded on first use) and a
     // grow-only arena for each call's inputs, outputs and workspace
     DevBuf<double> d_plug_rad, d_plug_ang, d_plug_w, d_plug;
+    DevBuf<int32_t> d_plug_lead;
+    int plug_n_lead = 0;
     bool plug_nnp_up = false;
     NnpTables nnp_dev{};
     size_t nnp_lds = 0;
@@ -1286,6 +1288,7 @@ int ptmc_destroy(ptmc_handle h)
     h->d_lut32.free_();
     h->d_plug_rad.free_();
     h->d_plug_ang.free_();
+    h->d_plug_lead.free_();
     h->d_plug_w.free_();
     h->d_plug.free_();
     h->d_maxboxh.free_();
@@ -2877,6 +2880,15 @@ int plugin_job(ptmc_engine *h, int32_t n_conf, int32_t n_atoms, const double *x,
             int rc = upload(h, h->d_plug_rad, n.rad64.empty() ? std::vector<double>(4, 0.0) : n.rad64);
             if (!rc) rc = upload(h, h->d_plug_ang, n.ang64.empty() ? std::vector<double>(6, 0.0) : n.ang64);
             if (!rc) rc = upload(h, h->d_plug_w, n.w64);
+            std::vector<int32_t> lead;
+            for (int q = 0; q < n.n_ang; ++q) {
+                const double *a = n.ang64.data();
+                bool first = a[6 * q + 5] != 0.0;
+                for (int p = 0; p < q; ++p) first = first && !(a[6 * p + 5] != 0.0 && a[6 * p] == a[6 * q]);
+                if (first) lead.push_back(q);
+            }
+            h->plug_n_lead = (int)lead.size();
+            if (!rc) rc = upload(h, h->d_plug_lead, lead);
             if (rc) return rc;
             h->plug_nnp_up = true;
         }
@@ -2889,6 +2901,8 @@ int plugin_job(ptmc_engine *h, int32_t n_conf, int32_t n_atoms, const double *x,
         j.hardcore2 = n.hardcore2;
         j.rad = h->d_plug_rad.p;
         j.ang = h->d_plug_ang.p;
+        j.lead = h->d_plug_lead.p;
+        j.n_lead = h->plug_n_lead;
         j.w = h->d_plug_w.p;
         break;
     }

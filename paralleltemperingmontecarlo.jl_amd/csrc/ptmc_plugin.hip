@@ -468,13 +468,14 @@ __global__ void __launch_bounds__(PT) plugin_nnp_feature_kernel(PluginJob j)
 // hard-core test failed.  A thread per (atom, output of a layer), four atoms a
 // workgroup: every dot product in order, as one thread per atom would take it,
 // but the outputs of a layer at once (one thread per atom waited for 88 x 20
-// loads in a row: 0.29 ms for 40 x 55 atoms, 0.02 so).
+// loads in a row: 0.29 ms for 40 x 55 atoms, 0.02 so).  b0: first workgroup of the
+// launch.
 constexpr int NET_ATOMS = PT / PLUGIN_MAXH;
-__global__ void __launch_bounds__(PT) plugin_nnp_network_kernel(PluginJob j)
+__global__ void __launch_bounds__(PT) plugin_nnp_network_kernel(PluginJob j, size_t b0)
 {
     __shared__ double a1[NET_ATOMS][PLUGIN_MAXH], a2[NET_ATOMS][PLUGIN_MAXH];
     const int nf = plugin_nf(j), la = threadIdx.x / PLUGIN_MAXH, o = threadIdx.x % PLUGIN_MAXH;
-    const size_t t = (size_t)blockIdx.x * NET_ATOMS + la;
+    const size_t t = (b0 + blockIdx.x) * NET_ATOMS + la;
     const bool in = t < (size_t)j.n_conf * j.N && ws_of(j).flag[t / j.N] == 0.0;
     const double *W1 = j.w, *B1 = W1 + (size_t)nf * j.h1, *W2 = B1 + j.h1, *B2 = W2 + (size_t)j.h1 * j.h2;
     const double *W3 = B2 + j.h2, *B3 = W3 + j.h2;
@@ -556,17 +557,23 @@ __device__ __forceinline__ double square_up(double p, int sq)
     return h + l;
 }
 
-// sum over the workgroup, on every thread, in a fixed order
-__device__ __forceinline__ double block_sum(double v, double *red)
+// sums over the wave and over the workgroup, on every thread, in a fixed order
+__device__ __forceinline__ double wave_sum(double v)
 {
     v = group_sum<16>(v);
     v += row_xor<16>(v);
-    v += row_xor<32>(v);
+    return v + row_xor<32>(v);
+}
+template <int NT>
+__device__ __forceinline__ double block_sum(double v, double *red)
+{
+    v = wave_sum(v);
+    if (NT == 64) return v;
     __syncthreads();
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
     double s = red[0];
-    for (int k = 1; k < PT / 64; ++k) s += red[k];
+    for (int k = 1; k < NT / 64; ++k) s += red[k];
     return s;
 }
 
@@ -575,67 +582,78 @@ __device__ __forceinline__ double block_sum(double v, double *red)
 // partner couples (k, l) that hold the atom (all of them for the moved atom).
 // Where the hard-core test failed the features are copied.
 //
-// One workgroup per (configuration, function).  The angular functions of one eta
-// are done by the first of them (the other workgroups end at once), DU at a time,
-// so a couple's two exponentials and four cosines are taken once for all; S lanes
+// Per configuration one workgroup for the radial functions, a wave each, and one
+// per eta for its angular functions (lead: the first of them), DU at a time, so a
+// couple's two exponentials and four cosines are taken once for all; S lanes
 // share the partners of a target atom, and the couple's term centred on i is
 // added where the target is the smaller of the two.  The sums at an atom are
 // taken by lane and then over the lanes, those at i over the workgroup, both in
 // a fixed order.  Before, a thread took one (function, atom) with a pow per
 // term: the moved atom's thread went through 1431 couples in a row, 4.9 ms for
 // 40 x 55 atoms x 88 functions whatever else ran; 0.14 ms so.  Bound by the FP64
-// instructions of a couple (about 700 for eight functions).
+// instructions of a couple (about 700 for eight functions); for a few atoms by
+// the workgroups themselves (one per function, most of them ending at once, took
+// three times as long for 20,000 x 3 atoms).  b0: first workgroup of the launch.
 constexpr int DU = 8;
-__global__ void __launch_bounds__(PT) plugin_nnp_delta_kernel(PluginJob j)
+template <int NT, int G>
+__global__ void __launch_bounds__(NT) plugin_nnp_delta_kernel(PluginJob j, size_t b0)
 {
     __shared__ uint64_t s_same[2];
     __shared__ int s_idx[DU];
-    __shared__ double s_par[DU][2], red[PT / 64];
+    __shared__ double s_par[DU][2], red[NT / 64];
     __shared__ int s_sq[DU];
-    const int N = j.N, nf = plugin_nf(j), tid = threadIdx.x;
-    const int c = (int)(blockIdx.x / (unsigned)nf), q = (int)(blockIdx.x % (unsigned)nf);
+    static_assert(G == NT || (G == 16 && NT == 64), "a workgroup, or a row of a wave");
+    const int N = j.N, nf = plugin_nf(j), tid = threadIdx.x, lt = tid % G;
+    const size_t wg = b0 + blockIdx.x, tasks = 1 + (size_t)j.n_lead;
+    const int task = (int)(wg % tasks), cu = (int)(wg / tasks) * (NT / G) + tid / G, c = min(cu, j.n_conf - 1);
     const WS w = ws_of(j);
     const size_t base = (size_t)c * N * nf;
     const double *in = j.vars_in + base;
     double *out = j.vars_out + base;
-    const bool rad = q < j.n_rad;
-    const double *A = rad ? j.rad + 4 * q : j.ang + 6 * (q - j.n_rad);
-    if (w.flag[c] != 0.0 || A[rad ? 3 : 5] == 0.0) {
-        for (int a = tid; a < N; a += PT) out[(size_t)a * nf + q] = in[(size_t)a * nf + q];
-        return;
-    }
+    const bool failed = w.flag[c] != 0.0, live = cu < j.n_conf && !failed;
+    if (G == NT && failed && task > 0) return;
     const int i = j.index[c];
     const double *R = w.rows + (size_t)c * PLUGIN_ROWS * N;
     const double *rn = R, *ro = R + N, *fn = R + 2 * N, *fo = R + 3 * N, *dn = R + 4 * N, *dold = R + 5 * N;
-    if (rad) {
-        const double eta = A[0], norm = A[1];
-        double sum = 0.0;
-        for (int a = tid; a < N; a += PT) {
-            if (a == i) continue;
-            const double tn = exp(-eta * rn[a]) * (fn[a] * norm), to = exp(-eta * ro[a]) * (-fo[a] * norm);
-            const double v = in[(size_t)a * nf + q] + tn;
-            out[(size_t)a * nf + q] = v + to;
-            sum += tn;
-            sum += to;
+    if (task == 0) {
+        // functions that no wave and no other workgroup writes
+        for (int e = lt; e < N * nf; e += G) {
+            const int q = e % nf;
+            const double active = q < j.n_rad ? j.rad[4 * q + 3] : j.ang[6 * (q - j.n_rad) + 5];
+            if (cu < j.n_conf && (failed || active == 0.0)) out[e] = in[e];
         }
-        sum = block_sum(sum, red);
-        if (tid == 0) out[(size_t)i * nf + q] = in[(size_t)i * nf + q] + sum;
+        constexpr int RL = G < 64 ? G : 64;  // lanes of a function
+        const int lane = lt % RL;
+        for (int q = lt / RL; q < j.n_rad; q += G / RL) {
+            const double eta = j.rad[4 * q], norm = j.rad[4 * q + 1];
+            if (j.rad[4 * q + 3] == 0.0) continue;
+            double sum = 0.0;
+            for (int a = lane; a < N; a += RL) {
+                if (a == i || !live) continue;
+                const double tn = exp(-eta * rn[a]) * (fn[a] * norm), to = exp(-eta * ro[a]) * (-fo[a] * norm);
+                const double v = in[(size_t)a * nf + q] + tn;
+                out[(size_t)a * nf + q] = v + to;
+                sum += tn;
+                sum += to;
+            }
+            sum = G < 64 ? group_sum<16>(sum) : wave_sum(sum);
+            if (lane == 0 && live) out[(size_t)i * nf + q] = in[(size_t)i * nf + q] + sum;
+        }
         return;
     }
-    // the active functions of this eta (at most 128 functions in all); the first does them
-    const int qa = q - j.n_rad;
-    const double eta = A[0];
-    if (tid < 128) {
-        const bool same = tid < j.n_ang && j.ang[6 * tid + 5] != 0.0 && (j.ang[6 * tid] == eta || tid == qa);
+    // the active functions of this eta (at most 128 functions in all)
+    const int qa = j.lead[task - 1];
+    const double eta = j.ang[6 * qa];
+    for (int u = tid; u < 128; u += NT) {
+        const bool same = u < j.n_ang && j.ang[6 * u + 5] != 0.0 && (j.ang[6 * u] == eta || u == qa);
         const uint64_t b = __ballot(same);
-        if ((tid & 63) == 0) s_same[tid >> 6] = b;
+        if ((u & 63) == 0) s_same[u >> 6] = b;
     }
     __syncthreads();
     uint64_t same[2] = {s_same[0], s_same[1]};
-    if ((qa < 64 ? same[0] & ((1ull << qa) - 1) : same[0] | (same[1] & ((1ull << (qa - 64)) - 1))) != 0) return;
-    int S = 1;  // lanes of a target: as many as the workgroup has for N targets, up to a row
-    while (S < 16 && 2 * S * N <= PT) S *= 2;
-    const int part = tid & (S - 1);
+    int S = 1;  // lanes of a target: as many as the configuration has for N targets, up to a row
+    while (S < 16 && 2 * S * N <= G) S *= 2;
+    const int part = lt & (S - 1);
     const double *r2 = w.d2 + (size_t)c * N * N, *f = w.m1 + (size_t)c * N * N;
     const double *X = j.x + (size_t)c * N * 3, *T = j.trial + 3 * (size_t)c, *Xi = X + 3 * i;
     while ((same[0] | same[1]) != 0) {
@@ -655,12 +673,12 @@ __global__ void __launch_bounds__(PT) plugin_nnp_delta_kernel(PluginJob j)
         double vi[DU];
 #pragma unroll
         for (int u = 0; u < DU; ++u) vi[u] = 0.0;
-        for (int a0 = 0; a0 < N; a0 += PT / S) {
-            const int a = a0 + tid / S;
+        for (int a0 = 0; a0 < N; a0 += G / S) {
+            const int a = a0 + lt / S;
             double va[DU];
 #pragma unroll
             for (int u = 0; u < DU; ++u) va[u] = 0.0;
-            if (a < N && a != i) {
+            if (a < N && a != i && live) {
                 const double *Xa = X + 3 * a;
                 for (int b = part; b < N; b += S) {
                     if (b == i || b == a) continue;
@@ -705,7 +723,7 @@ __global__ void __launch_bounds__(PT) plugin_nnp_delta_kernel(PluginJob j)
                 if (S >= 4) v += dpp_perm<0x4E>(v);
                 if (S >= 8) v += dpp_perm<0x141>(v);
                 if (S >= 16) v += dpp_perm<0x140>(v);
-                if (part == 0 && a < N && a != i) {
+                if (part == 0 && a < N && a != i && live) {
                     const size_t o = (size_t)a * nf + s_idx[u];
                     out[o] = in[o] + v;
                 }
@@ -714,8 +732,8 @@ __global__ void __launch_bounds__(PT) plugin_nnp_delta_kernel(PluginJob j)
 #pragma unroll
         for (int u = 0; u < DU; ++u) {
             if (u >= cnt) break;
-            const double v = block_sum(vi[u], red);
-            if (tid == 0) {
+            const double v = G < 64 ? group_sum<16>(vi[u]) : block_sum<NT>(vi[u], red);
+            if (lt == 0 && live) {
                 const size_t o = (size_t)i * nf + s_idx[u];
                 out[o] = in[o] + v;
             }
@@ -725,7 +743,20 @@ __global__ void __launch_bounds__(PT) plugin_nnp_delta_kernel(PluginJob j)
 static_assert(NNP_MAXF <= 128, "the functions of one eta in two masks");
 
 inline unsigned blocks(size_t n) { return (unsigned)((n + PT - 1) / PT); }
-inline unsigned net_blocks(size_t n) { return (unsigned)((n + NET_ATOMS - 1) / NET_ATOMS); }
+
+// n workgroups in launches of what one takes (2^32 - 1 work items)
+template <typename Launch>
+void in_launches(size_t n, Launch launch)
+{
+    constexpr size_t most = 0xffffffffu / PT;
+    for (size_t b = 0; b < n; b += most) launch(b, dim3((unsigned)(n - b < most ? n - b : most)));
+}
+void launch_network(const PluginJob &j, hipStream_t s)
+{
+    in_launches(((size_t)j.n_conf * j.N + NET_ATOMS - 1) / NET_ATOMS, [&](size_t b0, dim3 wgs) {
+        hipLaunchKernelGGL(plugin_nnp_network_kernel, wgs, dim3(PT), 0, s, j, b0);
+    });
+}
 
 }  // namespace
 
@@ -744,7 +775,7 @@ hipError_t plugin_initialise(const PluginJob &j, hipStream_t s)
         hipLaunchKernelGGL(plugin_eam_energy_kernel, dim3(blocks(C)), dim3(PT), 0, s, j);
     } else if (j.kind == POT_NNP) {
         hipLaunchKernelGGL(plugin_nnp_feature_kernel, dim3(blocks(C * plugin_nf(j) * N)), dim3(PT), 0, s, j);
-        hipLaunchKernelGGL(plugin_nnp_network_kernel, dim3(net_blocks(C * N)), dim3(PT), 0, s, j);
+        launch_network(j, s);
         hipLaunchKernelGGL(plugin_nnp_sum_kernel, dim3(blocks(C)), dim3(PT), 0, s, j);
     } else {
         hipLaunchKernelGGL(plugin_pair_kernel, dim3(blocks(C * N * N)), dim3(PT), 0, s, j);
@@ -762,8 +793,15 @@ hipError_t plugin_update(const PluginJob &j, hipStream_t s)
     } else if (j.kind == POT_NNP) {
         hipLaunchKernelGGL(plugin_geom_kernel, dim3(blocks(C * N * N)), dim3(PT), 0, s, j);
         hipLaunchKernelGGL(plugin_nnp_row_kernel, dim3(blocks(C * N)), dim3(PT), 0, s, j);
-        hipLaunchKernelGGL(plugin_nnp_delta_kernel, dim3((unsigned)(C * plugin_nf(j))), dim3(PT), 0, s, j);
-        hipLaunchKernelGGL(plugin_nnp_network_kernel, dim3(net_blocks(C * N)), dim3(PT), 0, s, j);
+        // up to 8 atoms by a wave, up to 4 by a row of one, whose lanes hold the targets'
+        // parts (20,000 x 3 atoms on 256 threads 5420 us, a wave 1570, a row 418; x 5 5550,
+        // 1550); the atoms alone choose, as the lanes of a target set the order of its sum
+        in_launches((N <= 4 ? (C + 3) / 4 : C) * (1 + (size_t)j.n_lead), [&](size_t b0, dim3 wgs) {
+            if (N <= 4) hipLaunchKernelGGL((plugin_nnp_delta_kernel<64, 16>), wgs, dim3(64), 0, s, j, b0);
+            else if (N <= 8) hipLaunchKernelGGL((plugin_nnp_delta_kernel<64, 64>), wgs, dim3(64), 0, s, j, b0);
+            else hipLaunchKernelGGL((plugin_nnp_delta_kernel<PT, PT>), wgs, dim3(PT), 0, s, j, b0);
+        });
+        launch_network(j, s);
         hipLaunchKernelGGL(plugin_nnp_sum_kernel, dim3(blocks(C)), dim3(PT), 0, s, j);
     } else {
         hipLaunchKernelGGL(plugin_pair_row_kernel, dim3(blocks(C * N)), dim3(PT), 0, s, j);

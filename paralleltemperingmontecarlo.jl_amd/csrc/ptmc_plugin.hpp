@@ -35,6 +35,8 @@ struct PluginJob {
     double r_cut = 0.0, hardcore2 = 0.0;
     const double *rad = nullptr;  // n_rad x 4: eta, norm, offset, active
     const double *ang = nullptr;  // n_ang x 6: eta, lambda, zeta, tpz, offset, active
+    const int32_t *lead = nullptr;  // n_lead: the first active angular function of every eta
+    int n_lead = 0;
     const double *w = nullptr;    // RuNNer parameter order, [nf, h1, h2, 1]
     // inputs (device)
     const double *x = nullptr;        // n_conf x N x 3 (null: distances from d2_in)
