@@ -40,7 +40,7 @@ CFLAGS = [
 # constants of every phase's polynomials hoisted out of it spill to scratch
 # (two species: 16 VGPRs and 141 SGPRs spilled with hoisting, none and 104
 # without; one species: 22 VGPRs with hoisting, none without).
-NO_MACHINE_LICM = ("ptmc_nnp", "ptmc_nnp2_mc", "ptmc_nnp2_mc_f32")
+NO_MACHINE_LICM = ("ptmc_nnp", "ptmc_nnp2_mc", "ptmc_nnp2_mc_f32", "ptmc_nnp2_mc_half", "ptmc_nnp2_mc_f32_half")
 
 
 def _compile(src: pathlib.Path) -> tuple[pathlib.Path, str]:

@@ -32,6 +32,10 @@ SweepFn nnp2_sweep_fn(bool pow);
 SweepFn nnp2_init_fn(bool pow);
 SweepFn nnp2_sweep_fn_f32(bool pow);
 SweepFn nnp2_init_fn_f32(bool pow);
+SweepFn nnp2_sweep_fn_half(bool pow);
+SweepFn nnp2_init_fn_half(bool pow);
+SweepFn nnp2_sweep_fn_f32_half(bool pow);
+SweepFn nnp2_init_fn_f32_half(bool pow);
 SweepFn nnp_cycle_fn();
 hipError_t sur_launch_desc(const float *x, const int32_t *n_atoms, float *bd, float r_cut, int n, hipStream_t st);
 hipError_t sur_launch_collect(const SweepArgs &a, int n_slots, float *bd, double *be, int32_t *bn, long long base,
@@ -947,8 +951,19 @@ int prepare_nnp2(ptmc_engine *h)
     const int N = n.n1 + n.n2;
     const bool f32 = h->cfg.precision == 1;
     const bool pw = std::find(n.gprog.begin(), n.gprog.end(), NNP2_POW) != n.gprog.end();
-    const void *fs = (const void *)(f32 ? nnp2_sweep_fn_f32(pw) : nnp2_sweep_fn(pw));
-    const void *fi = (const void *)(f32 ? nnp2_init_fn_f32(pw) : nnp2_init_fn(pw));
+    // Up to four groups are one pass of 512 threads, which have more registers each
+    // (FP64), or two workgroups a CU (binary32): us a cycle on 1024 / 512 threads, FP64
+    // 9 atoms without angular functions x 1000 421 / 356, 50 atoms, 1 group x 10 900 /
+    // 842, 50 atoms, 2 groups x 500 7226 / 6859; binary32 2 atoms x 4000 607 / 344, 10
+    // atoms, 1 group x 4000 2022 / 1134, 50 atoms, 1 group x 1000 2833 / 1628.  With
+    // more groups the second pass costs more (7 groups, 20 atoms x 10 FP64 564 / 759).
+    // The results have the same bits: no sum follows the number of waves.
+    const bool half = n.n_groups <= NNP2_GP / 2;
+    const int nt = half ? NNP2_NT / 2 : NNP2_NT;
+    const void *fs = (const void *)(f32 ? (half ? nnp2_sweep_fn_f32_half(pw) : nnp2_sweep_fn_f32(pw))
+                                        : (half ? nnp2_sweep_fn_half(pw) : nnp2_sweep_fn(pw)));
+    const void *fi = (const void *)(f32 ? (half ? nnp2_init_fn_f32_half(pw) : nnp2_init_fn_f32(pw))
+                                        : (half ? nnp2_init_fn_half(pw) : nnp2_init_fn(pw)));
     // what a launch can ask for: the kernels' own LDS comes off
     hipFuncAttributes as{}, ai{};
     HIPCHK(h, hipFuncGetAttributes(&as, fs));
@@ -956,15 +971,16 @@ int prepare_nnp2(ptmc_engine *h)
     max_lds -= (int)std::max(as.sharedSizeBytes, ai.sharedSizeBytes);
     // groups of a pass: as many as the workgroup has pairs of waves, fewer
     // where LDS would not hold their rows
-    int pass = std::max(1, std::min(NNP2_GP, n.n_groups));
+    int pass = std::max(1, std::min(nt / 128, n.n_groups));
     auto lds = [&]() { return nnp2_lds_bytes(N, n.ng, n.n_ang, pass, n.h1, n.h2, f32 ? 4 : 8); };
     while (pass > 1 && (long long)lds() > max_lds) --pass;
     h->nnp2_lds = lds();
-    // weights into what LDS is left
+    // weights into what LDS is left, a CU's half where two workgroups share it
+    const int room = half && f32 && h->nnp2_lds <= (size_t)max_lds / 2 ? max_lds / 2 : max_lds;
     const size_t esz = f32 ? 4 : 8, w23 = 2 * esz * ((size_t)n.h1 * n.h2 + 2 * n.h2 + 1), w1 = esz * ((size_t)n.ng + 1) * n.h1;
     int stage = 0;
     for (size_t add : {w23, w1, w1}) {
-        if (h->nnp2_lds + add > (size_t)max_lds) break;
+        if (h->nnp2_lds + add > (size_t)room) break;
         h->nnp2_lds += add;
         ++stage;
     }
@@ -979,8 +995,8 @@ int prepare_nnp2(ptmc_engine *h)
             return fail(h, PTMC_E_ARG, "every run holds the potential's %d + %d atoms (got %d)", n.n1, n.n2, rh.d.n_atoms);
         rh.info.slot_base = slot;
         rh.info.local_base = 0;
-        rh.kl = NNP2_NT;
-        rh.lanes = NNP2_NT;
+        rh.kl = nt;
+        rh.lanes = nt;
         rh.tile = -1;
         slot += rh.d.n_temps;
     }
@@ -991,8 +1007,8 @@ int prepare_nnp2(ptmc_engine *h)
     L.fn = (SweepFn)fs;
     L.init = (SweepFn)fi;
     L.ntiles = slot;
-    L.wgs = NNP2_NT;
-    L.kl = NNP2_NT;
+    L.wgs = nt;
+    L.kl = nt;
     L.lds = h->nnp2_lds;
     h->launches.push_back(L);
     h->n_coord = (int64_t)slot * 3 * NNP_NP;

@@ -47,7 +47,8 @@ namespace ptmc {
 
 namespace {
 
-constexpr int N2_NW = NNP2_NT / 64;
+constexpr int N2_NT = N2_THREADS;  // threads of a workgroup
+constexpr int N2_NW = N2_NT / 64;
 constexpr bool N2_F32 = sizeof(N2R) == 4;
 
 // one move's draws: the atom move, and the species picks of a swap
@@ -203,7 +204,7 @@ static_assert(sizeof(N2Group) <= NNP2_GROUP_BYTES, "group record");
 // records of groups g0, g0 + 1, ... of a pass into LDS
 __device__ __forceinline__ void n2_stage_groups(N2Tab &T, N2Group *to, int g0)
 {
-    for (int u = threadIdx.x; u < T.pass * NNP2_GMAX; u += NNP2_NT) {
+    for (int u = threadIdx.x; u < T.pass * NNP2_GMAX; u += N2_NT) {
         const int gl = u / NNP2_GMAX, l = u % NNP2_GMAX;
         if (g0 + gl >= T.n_groups) continue;
         const int first = T.grp[2 * (g0 + gl)], cnt = T.grp[2 * (g0 + gl) + 1], f = first + (l < cnt ? l : 0), q = T.gfn[f];
@@ -265,7 +266,7 @@ __device__ __forceinline__ void n2_tables(N2R *P, int N)
 {
     N2Tab &T = n2_fresh();
     const N2Lds L = n2_lds(T, N);
-    for (int e = threadIdx.x; e < N * 64; e += NNP2_NT) {
+    for (int e = threadIdx.x; e < N * 64; e += N2_NT) {
         const int k = e >> 6, j = e & 63;
         N2R r2 = N2R(0.0), f = N2R(0.0);
         if (j < N) {
@@ -504,7 +505,7 @@ __device__ __forceinline__ void n2_layer(const N2R *in, N2R *out, int N, int n, 
         }
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < h * N; e += NNP2_NT) out[e] = n2_act(act, out[e]);
+    for (int e = threadIdx.x; e < h * N; e += N2_NT) out[e] = n2_act(act, out[e]);
     __syncthreads();
 }
 
@@ -622,7 +623,7 @@ __device__ __forceinline__ double n2_rebuild(N2R *P, int N, double *s_tot)
 __device__ __forceinline__ void n2_load_x(N2Args &a, const N2Lds &L, int slot, int N)
 {
     const N2R *gX = reinterpret_cast<const N2R *>(a.coords) + (size_t)slot * 3 * NNP_NP;
-    for (int e = threadIdx.x; e < 3 * N; e += NNP2_NT) L.X[(e / N) * 64 + e % N] = gX[(e / N) * NNP_NP + e % N];
+    for (int e = threadIdx.x; e < 3 * N; e += N2_NT) L.X[(e / N) * 64 + e % N] = gX[(e / N) * NNP_NP + e % N];
 }
 
 // the weights T.stage says, once per launch
@@ -630,9 +631,9 @@ __device__ __forceinline__ void n2_stage_weights(N2Tab &T, N2R *W)
 {
     const int o2 = T.ng * T.h1 + T.h1, n23 = T.h1 * T.h2 + T.h2 + T.h2 + 1;
     if (T.stage > 0)
-        for (int e = threadIdx.x; e < 2 * n23; e += NNP2_NT) W[e] = (N2R)(e < n23 ? T.p1[o2 + e] : T.p2[o2 + e - n23]);
+        for (int e = threadIdx.x; e < 2 * n23; e += N2_NT) W[e] = (N2R)(e < n23 ? T.p1[o2 + e] : T.p2[o2 + e - n23]);
     for (int s = 0; s + 2 <= T.stage; ++s)
-        for (int e = threadIdx.x; e < o2; e += NNP2_NT) W[2 * n23 + s * o2 + e] = (N2R)(s ? T.p2 : T.p1)[e];
+        for (int e = threadIdx.x; e < o2; e += N2_NT) W[2 * n23 + s * o2 + e] = (N2R)(s ? T.p2 : T.p1)[e];
 }
 
 __device__ __forceinline__ N2R *n2_pairs(N2Tab &T, int slot, int N)
@@ -642,7 +643,7 @@ __device__ __forceinline__ N2R *n2_pairs(N2Tab &T, int slot, int N)
 
 // set_variables + initialise_energy (src/EnergyEvaluation.jl:1824-1856, :1748-1768)
 template <bool POW>
-__global__ void __launch_bounds__(NNP2_NT) nnp2_init_kernel(SweepArgs)
+__global__ void __launch_bounds__(N2_NT) nnp2_init_kernel(SweepArgs)
 {
     N2Args &a = n2_args();
     __shared__ double s_tot;
@@ -655,8 +656,8 @@ __global__ void __launch_bounds__(NNP2_NT) nnp2_init_kernel(SweepArgs)
     n2_stage_weights(T, L.W);
     const double E = n2_rebuild<POW>( n2_pairs(T, slot, N), N, &s_tot);
     N2R *gG = reinterpret_cast<N2R *>(T.feat) + (size_t)slot * NNP_NP * T.ng;
-    for (int e = threadIdx.x; e < N * T.ng; e += NNP2_NT) gG[e] = L.D[e];
-    for (int e = threadIdx.x; e < NNP_NP; e += NNP2_NT)
+    for (int e = threadIdx.x; e < N * T.ng; e += N2_NT) gG[e] = L.D[e];
+    for (int e = threadIdx.x; e < NNP_NP; e += N2_NT)
         reinterpret_cast<N2R *>(T.eatom)[(size_t)slot * NNP_NP + e] = e < N ? L.eatn[e] : N2R(0.0);
     if (threadIdx.x == 0) a.slot_en[slot] = E;
 }
@@ -808,7 +809,7 @@ __device__ __forceinline__ void n2_features(const N2Move &mv, N2R *P, int N, int
     __syncthreads();
     N2Tab &T = n2_fresh();
     const N2Lds L = n2_lds(T, N);
-    for (int u = threadIdx.x; u < nm * T.n_ang * 3; u += NNP2_NT) {
+    for (int u = threadIdx.x; u < nm * T.n_ang * 3; u += N2_NT) {
         const int mm = u >= T.n_ang * 3, v = mm ? u - T.n_ang * 3 : u, q = v / 3, row = v % 3, aa = mv.atom(mm);
         const double *A = T.ang + (size_t)q * 15 + 3 * (aa < T.n1 ? 0 : 1) + row;
         L.D[(2 * T.n_rad + 3 * q + row) * N + aa] = n2_scaled(L.S[2 * u] + L.S[2 * u + 1], A[3], A[9]);
@@ -838,7 +839,7 @@ __device__ __forceinline__ void n2_commit(const N2Move &mv, N2R *P, N2R *gG, int
             P[((size_t)g * N + lane) * 64 + aa] = v;
         }
     }
-    for (int e = tid; e < N * T.ng; e += NNP2_NT) gG[e] = L.D[e];
+    for (int e = tid; e < N * T.ng; e += N2_NT) gG[e] = L.D[e];
     if (tid < 3 * nm) {
         const int mm = tid >= 3, k = mm ? tid - 3 : tid, aa = mv.atom(mm);
         L.X[k * 64 + aa] = L.rec[(mm * 64 + aa) * 8 + k];
@@ -849,7 +850,7 @@ __device__ __forceinline__ void n2_commit(const N2Move &mv, N2R *P, N2R *gG, int
 // One cycle (N + n_swaps moves) of one configuration per workgroup
 // (mc_step! / mc_move!, src/MCRun.jl:142-182, with get_energy!(NNVT) :87-112).
 template <bool POW>
-__global__ void __launch_bounds__(NNP2_NT) nnp2_sweep_kernel(SweepArgs)
+__global__ void __launch_bounds__(N2_NT) nnp2_sweep_kernel(SweepArgs)
 {
     __shared__ int s_err, s_acc;
     __shared__ double s_en;
@@ -945,12 +946,12 @@ __global__ void __launch_bounds__(NNP2_NT) nnp2_sweep_kernel(SweepArgs)
             const int nd = N * T.ng;
             N2R g[8];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) g[u] = gG[min(tid + u * NNP2_NT, nd - 1)];
+            for (int u = 0; u < 8; ++u) g[u] = gG[min(tid + u * N2_NT, nd - 1)];
             n2_rows(L, mv, N, w, lane, (N2R)T.r_cut);
 #pragma unroll
             for (int u = 0; u < 8; ++u)
-                if (tid + u * NNP2_NT < nd) L.D[tid + u * NNP2_NT] = g[u];
-            for (int e = tid + 8 * NNP2_NT; e < nd; e += NNP2_NT) L.D[e] = gG[e];
+                if (tid + u * N2_NT < nd) L.D[tid + u * N2_NT] = g[u];
+            for (int e = tid + 8 * N2_NT; e < nd; e += N2_NT) L.D[e] = gG[e];
         }
         __syncthreads();
         n2_features<POW>(mv, P, N, w, lane);
@@ -991,14 +992,14 @@ __global__ void __launch_bounds__(NNP2_NT) nnp2_sweep_kernel(SweepArgs)
         const double Er = n2_rebuild<POW>(P, N, &s_tot);
         const double dr = __builtin_fabs(E - Er);
         if (tid == 0 && dr > z.slot_drift[slot]) z.slot_drift[slot] = dr;
-        for (int e = tid; e < N * z.nnp2.ng; e += NNP2_NT) gG[e] = L.D[e];
+        for (int e = tid; e < N * z.nnp2.ng; e += N2_NT) gG[e] = L.D[e];
         if (tid < N) L.eat[tid] = L.eatn[tid];
         E = Er;
         __syncthreads();
     }
 
     N2R *gX = reinterpret_cast<N2R *>(z.coords) + (size_t)slot * 3 * NNP_NP;
-    for (int e = tid; e < 3 * N; e += NNP2_NT) gX[(e / N) * NNP_NP + e % N] = L.X[(e / N) * 64 + e % N];
+    for (int e = tid; e < 3 * N; e += N2_NT) gX[(e / N) * NNP_NP + e % N] = L.X[(e / N) * 64 + e % N];
     if (tid < N) reinterpret_cast<N2R *>(z.nnp2.eatom)[(size_t)slot * NNP_NP + tid] = L.eat[tid];
     if (tid == 0) {
         z.slot_en[slot] = E;

@@ -84,9 +84,9 @@ __host__ __device__ inline size_t sur_lds_floats()
            3 * SUR_H + 4 * NNP_NP;
 }
 
-// Two-species NNVT kernels: threads per workgroup, angular functions per eta
-// group (larger groups are split), groups of one pass of a move (two waves
-// each), moves drawn together and the bytes of a draw record.
+// Two-species NNVT kernels: threads per workgroup (half of them up to NNP2_GP / 2
+// groups), angular functions per eta group (larger groups are split), groups of
+// one pass of a move (two waves each), moves drawn together and the bytes of a draw record.
 constexpr int NNP2_NT = 1024;
 constexpr int NNP2_GMAX = 6;
 constexpr int NNP2_GP = NNP2_NT / 128;
