@@ -185,25 +185,6 @@ __device__ __forceinline__ uint32_t row_xor_u32(uint32_t v)
 template <int ROW>
 __device__ __forceinline__ float row_xor(float v) { return __uint_as_float(row_xor_u32<ROW>(__float_as_uint(v))); }
 
-// v + (v of the lane across the row boundary), from one row swap of v with
-// a copy of itself: after v_permlane16_swap(a = v, b = v) (or the 32-lane
-// swap) a lane of an even row holds its own value in a and its partner's in
-// b, a lane of an odd row the reverse, so a + b is the pair sum on every lane
-// (the same bits as v + partner: the two operands are the same, in either
-// order).
-template <int ROW>
-__device__ __forceinline__ float row_pair_sum(float v)
-{
-    const uint32_t u = __float_as_uint(v);
-    if constexpr (ROW == 16) {
-        const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-    } else {
-        static_assert(ROW == 32, "row swap of 16 or 32 lanes");
-        const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-    }
-}
 // Two values merged across the row boundary: lanes of the even rows (the
 // lower half) get a + (a across the boundary), lanes of the odd rows (the
 // upper half) the same of b.
@@ -220,6 +201,11 @@ __device__ __forceinline__ float row_merge(float a, float b)
         return __uint_as_float(r[0]) + __uint_as_float(r[1]);
     }
 }
+// v + (v of the lane across the row boundary) on every lane: the swap of v with a
+// copy of itself leaves a lane's own value and its partner's in the two
+// registers, in either order.
+template <int ROW>
+__device__ __forceinline__ float row_pair_sum(float v) { return row_merge<ROW>(v, v); }
 template <int ROW>
 __device__ __forceinline__ double row_xor(double v)
 {

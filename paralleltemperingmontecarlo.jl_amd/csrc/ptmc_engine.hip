@@ -1050,19 +1050,21 @@ int prepare_nnp2(ptmc_engine *h)
     return PTMC_OK;
 }
 
-// Slots of a neural-network engine: one workgroup per slot, slots of a run
-// consecutive, temperature t of run r starting in slot slot_base + t.
 // Threads of a slot.  Slots of 128 atoms have a CU to themselves (LDS) and take
 // 1024 threads, and so do slots of 64 while there are no more of them than CUs
 // (us per cycle on 512 / 1024 threads: 40 x 55 atoms 1224 / 1121, 40 x 33 618 /
 // 602, 256 x 55 1248 / 1150).  Past that two slots of 512 share a CU and hide
 // each other's barriers (264 x 55 1624 / 2129, 1280 x 55 3950 / 5348), and small
-// clusters do not fill 16 waves (40 x 13 201 / 221).
+// clusters do not fill 16 waves (40 x 13 201 / 221).  The widths round their sums
+// differently; these runs do not repeat bit for bit on one width either, as the
+// start features are summed by LDS atomics.
 int nnp_threads(int np, int n_max, int64_t slots, int cus)
 {
     return np > NNP_NP || (slots <= cus && n_max > NNP_NP / 2) ? 2 * NNP_NT : NNP_NT;
 }
 
+// Slots of a neural-network engine: one workgroup per slot, slots of a run
+// consecutive, temperature t of run r starting in slot slot_base + t.
 int prepare_nnp(ptmc_engine *h)
 {
     if (h->cfg.precision != 1) return fail(h, PTMC_E_UNSUPPORTED, "the network potential runs in binary32 (precision 1)");

@@ -157,12 +157,12 @@ __device__ __forceinline__ void nnp_group(const int32_t *gd, int g, NnpGroup &G)
     }
     G.eta2 = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(dw[0]));
     G.row0 = __builtin_amdgcn_readfirstlane(dw[1]);
-    G.top[0] = G.top[1] = 0;
+    G.top[0] = __builtin_amdgcn_readfirstlane(dw[2]) + 1;
+    G.top[1] = __builtin_amdgcn_readfirstlane(dw[3]) + 1;
 #pragma unroll
     for (int q = 0; q < NNP_GMAX; ++q) {
         G.tpz[q] = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(dw[4 + q]));
         G.rk[q] = __builtin_amdgcn_readfirstlane(dw[4 + NNP_GMAX + q]);
-        if (G.rk[q] >= 0) G.top[q / NNP_KSLOT] = q % NNP_KSLOT + 1;
     }
 }
 
