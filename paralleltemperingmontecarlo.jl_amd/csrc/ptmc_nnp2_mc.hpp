@@ -130,7 +130,14 @@ __device__ __forceinline__ N2R n2_cut(N2R r, N2R rc)
     return r < rc ? c * c : N2R(0.0);
 }
 
-__device__ __forceinline__ double n2_tanh(double x) { return net_tanh(x); }
+__device__ __forceinline__ double n2_tanh(double x)
+{
+    return net_tanh(x, [](double d) {
+        double y = __builtin_amdgcn_rcp(d);
+        y = fma(fma(-d, y, 1.0), y, y);
+        return fma(fma(-d, y, 1.0), y, y);
+    });
+}
 __device__ __forceinline__ float n2_tanh(float x) { return tanhf(x); }
 
 __device__ __forceinline__ N2R n2_d2(const N2R *a, const N2R *b)

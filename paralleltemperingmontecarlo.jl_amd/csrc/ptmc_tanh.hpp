@@ -10,7 +10,10 @@ namespace ptmc {
 // Taylor series, 2x = k ln 2 + r (Cody-Waite).  r, q, t and t + 2 carry the
 // rounding of their last operation (2^k q takes up to half of 2^k - 1 away at k
 // = 1: 2.5 ulp without), so that the value is within 0.7 ulp, small x included.
-__host__ __device__ inline double net_tanh(double x)
+// rcp(d): 1 / d for d in [2, 2^59) to a few ulp; the quotient's remainder is put
+// back.
+template <typename Rcp>
+__host__ __device__ inline double net_tanh(double x, Rcp rcp)
 {
     const double y = fmin(fabs(x), 20.0) * 2.0;
     const double kd = rint(y * 1.4426950408889634);
@@ -34,7 +37,7 @@ __host__ __device__ inline double net_tanh(double x)
     const double p = ldexp(1.0, (int)kd), a = p - 1.0, b = p * q;
     const double t = a + b, tl = fma(p, ql, b - (t - a));  // |b| < a, or a = 0
     const double d = t + 2.0, dl = t >= 2.0 ? 2.0 - (d - t) : t - (d - 2.0);
-    const double i = 1.0 / d, v = t * i;
+    const double i = rcp(d), v = t * i;
     const double w = fma(fma(-v, d, t) + fma(-v, dl + tl, tl), i, v);
     return x != x ? x : copysign(w, x);
 }
