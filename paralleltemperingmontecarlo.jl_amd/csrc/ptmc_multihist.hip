@@ -154,9 +154,10 @@ __device__ bool mh_barrier(const MHArgs &a, int run, unsigned epoch, int *s_ok)
 // added in one order, so that results do not depend on the cut.
 //
 // Bound by the latency of an iteration's chain (two reductions, one exp and
-// log per temperature, the barrier), not by arithmetic: 4.5 us an iteration
-// for 16 runs of 32 x 100 bins (917 -> 184 us a call's kernel against one
-// exponential per temperature and bin twice an iteration), 8 us for one run
+// log per temperature, the barrier), not by arithmetic (VALU issued in 17 % of
+// the cycles): 4 us an iteration for 16 runs of 32 x 100 bins, which have no
+// barrier (917 -> 162 us a call's kernel against one exponential per temperature
+// and bin twice an iteration), 8 us for one run
 // of 48 x 10^4 bins on 79 workgroups (98 -> 1.02 ms; 17 us an iteration with
 // shuffles instead of row permutations and the exchange's loads one by one).
 template <bool KEEP>

@@ -26,7 +26,7 @@ struct MhCut {
 
 // Workgroups of a run of `bins` bins and R temperatures, one of `runs` runs, on
 // a device of `cus` compute units with max_lds bytes of LDS that a workgroup can ask for.  Up to
-// 512 bins (NVT histograms) one, if its slice fits LDS: an iteration (4.5 us)
+// 512 bins (NVT histograms) one, if its slice fits LDS: an iteration (4 us)
 // is not worth a barrier between workgroups (about 3 us).  Else the bins are cut
 // so that every slice fits LDS, and over more workgroups while the runs leave
 // compute units idle (48 x 10^4 NPT bins: 79 workgroups of one block each).

@@ -33,11 +33,12 @@
 //
 // Bound by the instructions of the triangle visits (about 45 and 10 per
 // function each, only partners inside the cut-off, half of a move's time) and
-// the latency of the move's phases (rows, pair factors, three layers, commit).
+// the latency of the move's phases (rows, pair factors, three layers, commit):
+// VALU issues in 46 % of the SIMDs' cycles, and a wave waits for 57 % of its own.
 // Cu50Zn5 (5 + 26 functions, 7 groups, one workgroup of 16 waves per CU), a
 // launch of 57 moves: 11.1 ms with an exponential, a division and two square
-// roots per triangle and group, 1.9 ms so; 25 ladders of 10 1.35 -> 6.5e6
-// moves/s, 50 ladders in binary32 2.85 -> 8.5e6.
+// roots per triangle and group, 1.85 ms so; 25 ladders of 10 1.35 -> 7.0e6
+// moves/s, 50 ladders in binary32 2.85e6 -> 1.02e7.
 // (no include guard: included once per element type)
 #include "ptmc_nnp_layout.hpp"
 #include "ptmc_sweep.hpp"

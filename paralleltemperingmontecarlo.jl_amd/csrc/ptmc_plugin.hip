@@ -590,7 +590,7 @@ __device__ __forceinline__ double block_sum(double v, double *red)
 // taken by lane and then over the lanes, those at i over the workgroup, both in
 // a fixed order.  Before, a thread took one (function, atom) with a pow per
 // term: the moved atom's thread went through 1431 couples in a row, 4.9 ms for
-// 40 x 55 atoms x 88 functions whatever else ran; 0.14 ms so.  Bound by the FP64
+// 40 x 55 atoms x 88 functions whatever else ran; 0.07 ms so.  Bound by the FP64
 // instructions of a couple (about 700 for eight functions); for a few atoms by
 // the workgroups themselves (one per function, most of them ending at once, took
 // three times as long for 20,000 x 3 atoms).  b0: first workgroup of the launch.
