@@ -9,6 +9,7 @@ namespace ptmc {
 
 constexpr int MH_THREADS = 256;
 constexpr int MH_BINS = 128;                   // bins of a block, whose sums are formed together
+constexpr size_t MH_LARGE = 96 * 1024;         // bytes of a slice above which few runs are cut
 
 // LDS of mh_iterate_kernel in doubles: the temperatures' terms, and with KEEP
 // a slice of `bins` bins (matrix, histogram sums, offsets, ratios)
@@ -25,13 +26,15 @@ struct MhCut {
 };
 
 // Workgroups of a run of `bins` bins and R temperatures, one of `runs` runs, on
-// a device of `cus` compute units with max_lds bytes of LDS that a workgroup can ask for.  Up to
-// 512 bins (NVT histograms) one, if its slice fits LDS: an iteration (4 us)
-// is not worth a barrier between workgroups (about 3 us).  Else the bins are cut
-// so that every slice fits LDS, and over more workgroups while the runs leave
-// compute units idle (48 x 10^4 NPT bins: 79 workgroups of one block each).
-// Where even one workgroup per compute unit would hold too much (48 x 40,000
-// bins: 313 blocks of 52 kB) the slices are not kept.
+// a device of `cus` compute units with max_lds bytes of LDS that a workgroup can
+// ask for.  Up to 512 bins (NVT histograms) one, if its slice fits LDS: an
+// iteration (4 us) is not worth a barrier between workgroups (about 3 us), unless
+// the slice is large and the runs few (20 iterations of one run of 32 x 500 bins
+// on one workgroup 259 us, on four 233; of 16 runs 363, 404; 300 runs of 40 x 400
+// 2197, 2416).  Else the bins are cut so that every slice fits LDS, and over more
+// workgroups while the runs leave compute units idle (48 x 10^4 NPT bins: 79
+// workgroups of one block each).  Where even one workgroup per compute unit would
+// hold too much (20 x 400^2 bins fit, 48 x 400^2 do not) the slices are not kept.
 inline MhCut mh_cut(int R, size_t bins, int runs, int cus, size_t max_lds)
 {
     MhCut c{};
@@ -44,7 +47,7 @@ inline MhCut mh_cut(int R, size_t bins, int runs, int cus, size_t max_lds)
     cut(1);
     const size_t base = 8 * mh_lds(R, true, false);
     const size_t room = max_lds > base ? max_lds - base : 0;
-    if (bins > 512 || slice() > room) {
+    if (bins > 512 || slice() > room || (slice() > MH_LARGE && runs < 16)) {
         const size_t fit = room / (8 * mh_slice(R, MH_BINS));  // blocks of a slice
         const int need = fit > 0 ? (int)((c.n_blk + fit - 1) / fit) : c.n_blk;
         cut(std::max({1, std::min(c.n_blk, cus / runs), need <= cus ? need : 0}));
